@@ -850,6 +850,7 @@ int sdot_amd_linear_solves_2d( void *stream, long long n, const long long *row, 
         mo.fp32 = options && options[ 5 ] == 1;          // ( the multigrid's cycle in FP32, the flexible CG in FP64 )
         if ( options && options[ 8 ] >= 0 ) mo.kcycle = int( options[ 8 ] );
         if ( options && options[ 9 ] > 0 ) mo.nu = int( options[ 9 ] );
+        mo.smoothed = options && options[ 4 ] == 1;      // ( asked for: rows in an order of the caller's have no compact aggregates )
         for ( long long j = 0; j < k; ++j ) {
             CgStats cs;
             int levels = 0;

@@ -6,6 +6,7 @@
 
 #include "../../include/sdot_amd.h"
 #include "memory.h"
+#include "smoothed.h"
 #include "solver.h"
 #include "tree.h"
 #include "cells3.h"
@@ -45,28 +46,27 @@ void solve_parts( I64 n, int dim, int density_kind, const double *o, int precisi
     // Newton's vectors ( targets, weights and trial weights, direction, right-hand side, staging ), the moments' diagram
     parts[ 5 ] = 7 * 8 * m;
     parts[ 6 ] = ( d3 ? 24 : 16 ) * m + 16 * m;
-    // the linear solver: the multigrid's levels ( coarse rows of 96 entries, their vectors, the K-cycle's ), its outer
-    // vectors; Jacobi-PCG's when asked for
+    // the linear solver: the multigrid's levels, their vectors, the outer iteration's; Jacobi-PCG's when asked for
     if ( o && int( o[ O_LIN ] ) == 1 ) {
-        const int pack = o[ O_MG_SHIFT ] > 0 ? 1 << int( o[ O_MG_SHIFT ] ) : 8;
-        const int kc = o[ O_MG_KCYCLE ] >= 0 ? int( o[ O_MG_KCYCLE ] ) : 2;
-        // the coarse levels in `s`-byte values; the FP64 flexible CG's four vectors and the finest level's work vector; with the
-        // FP32 preconditioner ( `mg_float` ) its own levels, work vector, FP32 copies of the rows, diagonal, `r` and `z`, beside
-        // the FP64 solve it falls back to
+        // the FP32 preconditioner's copies of the rows and their diagonal ( `mg_float` ), then the smoothed hierarchy in the cycle's
+        // float; or, where the options set the K-cycle's own, its coarse levels in `s`-byte values and vectors. ( A system redone with
+        // the FP64 cycle, or one the smoothed hierarchy has no room for, takes that cycle's buffers beside these. )
         const bool f32 = o[ O_MG_FLOAT ] != 0;
-        auto coarse = [&]( double s ) {
-            double b = 0;
+        const double s = f32 ? 4 : 8;
+        double lin = f32 ? 4 * cap + 4 * m : 0;
+        if ( smoothed_asked( o ) && n > SA_MIN_ROWS )
+            lin += smoothed_bytes( n, d3, s );
+        else {
+            const int pack = o[ O_MG_SHIFT ] > 0 ? 1 << int( o[ O_MG_SHIFT ] ) : 8;
+            const int kc = o[ O_MG_KCYCLE ] >= 0 ? int( o[ O_MG_KCYCLE ] ) : 2;
             double nl = m;
+            lin += 4 * 8 * m + s * m + ( f32 ? 8 * m : 0 ) + 24 * 5 * 512 * 8 + 64 * 64 * 8 + 4 * 512 * 8;
             for ( int l = 1; nl > 64 && l < 24; ++l ) {
                 nl = std::ceil( nl / pack );
-                b += nl * ( 4 + MG_STRIDE_B * ( 4 + s ) + s ) + 3 * s * nl + ( l <= kc ? 5 * s * nl : 0 );
+                lin += nl * ( 4 + MG_STRIDE_B * ( 4 + s ) + s ) + 3 * s * nl + ( l <= kc ? 5 * s * nl : 0 );
             }
-            return b;
-        };
-        double lin = 4 * 8 * m + 8 * m + coarse( 8 );
-        if ( f32 ) lin += 4 * 8 * m + 4 * m + coarse( 4 ) + 4 * cap + 4 * m + 8 * m;
-        // each precision's partial sums, K-cycle partials and dense inverse of the coarsest level
-        parts[ 7 ] = lin + ( f32 ? 2 : 1 ) * ( 24 * 5 * 512 * 8 + 64 * 64 * 8 + 4 * 512 * 8 );
+        }
+        parts[ 7 ] = lin;
     } else
         parts[ 7 ] = 3 * 8 * m;
     // the density's copies: an image's blurred copies ( the width continuation ) and its pyramid of minima ( the limits )

@@ -21,10 +21,18 @@ struct MgOptions {
     /// coarse solves ) in FP32 from an FP32 copy of the rows ( the reference card's float levels, `gpu/Linear2D.cuh:993-1000` );
     /// the FP64 cycle when that solve does not converge
     bool   fp32 = false;
+    /// the smoothed-aggregation V-cycle ( smoothed.hip ) before the K-cycle over plain aggregates, which then takes the systems it has
+    /// no room for ( a coarse row past its entries ) and the callers that set `pack`, `nu`, `kcycle` or `bottom` themselves
+    bool   smoothed = true;
 };
 
-/// `L d = b` ( `b` of zero sum ) by flexible CG preconditioned with one multigrid cycle whose aggregates are `pack`
-/// consecutive tree ranks ( the cycle in FP32 when `o.fp32` ); the solution shifted so that `d[ gauge ] = 0`.
+/// whether a solve's options leave the cycle to the smoothed hierarchy ( settings of the K-cycle ask for the K-cycle )
+inline bool smoothed_asked( const double *o ) {
+    return ! ( o[ O_MG_SHIFT ] > 0 || o[ O_MG_NU ] > 0 || o[ O_MG_KCYCLE ] >= 0 || o[ O_MG_STOP ] != 0 );
+}
+
+/// `L d = b` ( `b` of zero sum ) by flexible CG preconditioned with one multigrid cycle whose aggregates are consecutive
+/// tree ranks ( the cycle in FP32 when `o.fp32` ); the solution shifted so that `d[ gauge ] = 0`.
 /// Returns the iteration count, or -1 when it did not reach `tol` ( relative residual ) in `maxit`, or
 /// -2 when the hierarchy could not be built ( a coarse row with too many neighbours ).
 int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, int maxit, const MgOptions &o, hipStream_t st, CgStats &cs,

@@ -23,9 +23,8 @@
 // Deterministic: fixed-shape reductions, each coarse row merged in a fixed order.
 
 #include "multigrid.h"
-
-#include <algorithm>
-#include <cstdint>
+#include "graph_cache.h"
+#include "smoothed.h"
 
 namespace sdot_amd {
 
@@ -767,55 +766,8 @@ void cycle( Hierarchy<R> &H, int l, const R *r, R *x, const MgOptions &o, const 
     }
 }
 
-/// THE ITERATIONS AS A GRAPH: a batch of flexible CG iterations is ~100 launches of small kernels, whose issue costs
-/// more than their work on the coarse levels; replayed from a HIP graph it is one launch. A graph is valid as long as
-/// every kernel argument is: its key is the full record of them ( the hierarchy's levels, vectors and sizes, the options,
-/// the storage type ), written field by field ( no padding bytes ) and compared whole, so that two different argument sets
-/// never share a graph. The arena keeps the buffers of a solve of the same size, so Newton's successive systems ( two slots
-/// of rows ) replay two graphs per storage type. A few per thread are kept ( least recently used out ).
-struct GraphCache {
-    struct Entry { std::vector<unsigned char> key; hipGraphExec_t exec; hipGraph_t graph; uint64_t used; };
-    std::vector<Entry> entries;
-    uint64_t clock = 0;
-    ~GraphCache() {
-        for ( auto &e : entries ) { (void) hipGraphExecDestroy( e.exec ); (void) hipGraphDestroy( e.graph ); }
-    }
-    hipGraphExec_t find( const std::vector<unsigned char> &key ) {
-        for ( auto &e : entries ) if ( e.key == key ) { e.used = ++clock; return e.exec; }
-        return nullptr;
-    }
-    void put( const std::vector<unsigned char> &key, hipGraph_t g, hipGraphExec_t x ) {
-        if ( entries.size() >= 8 ) {
-            auto old = std::min_element( entries.begin(), entries.end(), []( const Entry &a, const Entry &b ) { return a.used < b.used; } );
-            (void) hipGraphExecDestroy( old->exec );
-            (void) hipGraphDestroy( old->graph );
-            entries.erase( old );
-        }
-        entries.push_back( Entry{ key, x, g, ++clock } );
-    }
-};
-thread_local GraphCache g_graphs;
-
-/// the stream graphs are captured on ( a capture needs a stream of its own: the legacy default stream cannot be
-/// captured ); one per thread, default priority
-struct CaptureStream {
-    hipStream_t s = nullptr;
-    ~CaptureStream() { if ( s ) (void) hipStreamDestroy( s ); }
-    hipStream_t get() {
-        if ( ! s && hipStreamCreateWithFlags( &s, hipStreamNonBlocking ) != hipSuccess ) { (void) hipGetLastError(); s = nullptr; }
-        return s;
-    }
-};
-thread_local CaptureStream g_capture;
-
-/// a graph's key: the values of the kernels' arguments appended one by one ( scalars and pointers, never a struct with
-/// padding )
-struct Key {
-    std::vector<unsigned char> b;
-    template<class T> void val( const T &v ) {
-        const unsigned char *c = reinterpret_cast<const unsigned char *>( &v );
-        b.insert( b.end(), c, c + sizeof( T ) );
-    }
+/// the graphs' key of this cycle: every field of its matrices and of the bottom kernel's levels
+struct KcycleKey : Key {
     template<class R> void mat( const MatT<R> &A ) {
         val( A.n ); val( A.step ); val( A.row_off ); val( A.row_cnt ); val( A.col ); val( A.val ); val( A.dia );
     }
@@ -827,13 +779,6 @@ struct Key {
             val( L.n ); val( L.cnt ); val( L.col ); val( L.val ); val( L.dia ); val( L.x ); val( L.t ); val( L.r );
         }
     }
-};
-
-/// what one flexible-CG solve reports
-struct FcgResult {
-    int its = 0;
-    bool bad = false, failed = false;    ///< no hierarchy ( a coarse row past its room ); a breakdown ( `p . q <= 0` )
-    double err = 0, true_err = 0;        ///< relative residual by the recurrence, and the true one
 };
 
 /// `y = x` in another float
@@ -955,7 +900,7 @@ FcgResult fcg_mg( const MatT<R> &A0m, const MatT<P> &A0p, I64 nnz, const R *b, R
     // the graph of a batch, found by the full record of every argument its kernels take
     hipGraphExec_t exec = nullptr;
     if ( o.graphs ) {
-        Key key;
+        KcycleKey key;
         key.val( int( sizeof( R ) ) ); key.val( int( sizeof( P ) ) );
         key.mat( A0 ); key.val( rp ); key.val( zp ); key.val( H.nl ); key.val( H.lb ); key.val( H.nc ); key.val( H.inv ); key.val( H.part ); key.val( H.kpart );
         for ( int l = 0; l < H.nl; ++l ) {
@@ -1039,34 +984,48 @@ int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, i
     bool done = false;
     double err = 1, true_err = 1;
     bool breakdown = false;
+    bool smoothed = o.smoothed && n > SA_MIN_ROWS;
+    float *valf = nullptr, *diaf = nullptr;
+    // one solve of the system ( `f32`: the cycle in FP32 ); false when its hierarchy could not be built
+    auto attempt = [&]( bool f32 ) {
+        const int left = f32 ? maxit : std::max( maxit - total, 4 );
+        FcgResult f;
+        if ( smoothed ) {
+            f = smoothed_solve( L, f32 ? valf : nullptr, f32 ? diaf : nullptr, b, d, tol, left, o, st, nb_levels, cs.last_its );
+            if ( ! f.bad ) cs.last_its = f.its;
+            smoothed = ! f.bad;                          // ( a coarse row past its room: the K-cycle from here on )
+        }
+        if ( ! smoothed ) {
+            if ( f32 ) {
+                MatT<float> Af;
+                Af.n = n; Af.step = L.step; Af.row_off = L.row_off; Af.row_cnt = L.row_cnt; Af.col = L.col; Af.val = valf; Af.dia = diaf;
+                f = fcg_mg<double, float>( A0, Af, L.nnz, b, d, tol, left, o, st, nb_levels, "mgm" );
+            } else
+                f = fcg_mg<double, double>( A0, A0, L.nnz, b, d, tol, left, o, st, nb_levels, "mg" );
+            if ( f.bad ) return false;
+        }
+        total += f.its;
+        err = f.err;
+        true_err = f.true_err;
+        breakdown = f.failed;
+        done = ! f.failed && f.err <= tol && f.true_err <= 10 * tol;
+        if ( f32 ) {
+            ++timing().mg32_solves;
+            timing().mg32_iterations += f.its;
+            if ( ! done ) { cs.nb_fp64_fallbacks += 1; ++timing().mg32_fallbacks; }
+        }
+        return true;
+    };
     if ( o.fp32 ) {
         // THE FP32 PRECONDITIONER: the hierarchy, its smoothing and its coarse solves in FP32 ( from an FP32 copy of the rows ),
         // the flexible CG, its SpMV and its vectors in FP64; the FP64 preconditioner when that solve does not converge
-        float *valf = A.get<float>( "mgm.valf", size_t( L.cap ) ), *diaf = A.get<float>( "mgm.diaf", size_t( n ) );
+        valf = A.get<float>( "mgm.valf", size_t( L.cap ) );
+        diaf = A.get<float>( "mgm.diaf", size_t( n ) );
         k_to_float_rows<<<blocks_for( n, 256 ), 256, 0, st>>>( n, L.row_off, L.row_cnt, L.step, L.val, L.dia, valf, diaf );
         check_launch( "k_to_float_rows" );
-        MatT<float> Af;
-        Af.n = n; Af.step = L.step; Af.row_off = L.row_off; Af.row_cnt = L.row_cnt; Af.col = L.col; Af.val = valf; Af.dia = diaf;
-        const FcgResult f = fcg_mg<double, float>( A0, Af, L.nnz, b, d, tol, maxit, o, st, nb_levels, "mgm" );
-        if ( f.bad ) return -2;
-        total += f.its;
-        err = f.err;
-        true_err = f.true_err;
-        breakdown = f.failed;
-        done = ! f.failed && f.err <= tol && f.true_err <= 10 * tol;
-        ++timing().mg32_solves;
-        timing().mg32_iterations += f.its;
-        if ( ! done ) { cs.nb_fp64_fallbacks += 1; ++timing().mg32_fallbacks; }
+        if ( ! attempt( true ) ) return -2;
     }
-    if ( ! done ) {
-        const FcgResult f = fcg_mg<double, double>( A0, A0, L.nnz, b, d, tol, std::max( maxit - total, 4 ), o, st, nb_levels, "mg" );
-        if ( f.bad ) return -2;
-        total += f.its;
-        err = f.err;
-        true_err = f.true_err;
-        breakdown = f.failed;
-        done = ! f.failed && f.err <= tol && f.true_err <= 10 * tol;
-    }
+    if ( ! done && ! attempt( false ) ) return -2;
     double *g = A.get<double>( "mg.g", 1 );
     k_read_gauge<<<1, 64, 0, st>>>( d, gauge, g );
     k_shift_gauge<<<blocks_for( n, 256 ), 256, 0, st>>>( n, d, g, gauge );

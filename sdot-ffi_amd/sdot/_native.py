@@ -520,8 +520,9 @@ def refresh_majorants_2d( tree, sorted_positions, sorted_weights ):
     return wa, wb
 
 
-def linear_solves_2d( row, col, val, dia, rhs, tol = 1e-6, method = "cg", kcycle = -1, nu = 0 ):
-    """`L d_j = rhs[ j ]` ( `SdotPlanNd._card_linear_solves` of the reference: `method` "cg" or "mg" )"""
+def linear_solves_2d( row, col, val, dia, rhs, tol = 1e-6, method = "cg", kcycle = -1, nu = 0, smoothed = False, fp32 = False ):
+    """`L d_j = rhs[ j ]` ( `SdotPlanNd._card_linear_solves` of the reference: `method` "cg" or "mg" ); with "mg", `smoothed` the
+    smoothed-aggregation cycle ( for rows in an order whose neighbours are near, as a solve's ranks ), `fp32` the cycle in FP32"""
     T = torch()
     row = on_device( row, T.int64 )
     col = on_device( col, T.int64 )
@@ -535,7 +536,7 @@ def linear_solves_2d( row, col, val, dia, rhs, tol = 1e-6, method = "cg", kcycle
     its = np.zeros( k )
     if method not in ( "cg", "mg" ):
         raise ValueError( f"linear_solves_2d: method 'cg' or 'mg' ( not { method!r} )" )
-    opts, optp = _host( [ n, k, 0 if method == "cg" else 1, tol, -1, 0, 0, 0, kcycle, nu ] )
+    opts, optp = _host( [ n, k, 0 if method == "cg" else 1, tol, 1 if smoothed else -1, int( fp32 ), 0, 0, kcycle, nu ] )
     _check( lib().sdot_amd_linear_solves_2d( _stream(), n, _ptr( row ), _ptr( col ), _ptr( val ), _ptr( dia ), _ptr( rhs.contiguous() ), k,
                                              optp, _ptr( sol ), its.ctypes.data_as( _P ) ) )
     return sol, its.astype( int )

@@ -1,0 +1,83 @@
+"""The smoothed-aggregation V-cycle ( the Newton systems' default preconditioner ) through `sdot_amd_linear_solves_2d`, on the
+Laplacians of power diagrams in tree order: against a dense solve where that is quick, against the Jacobi-PCG elsewhere."""
+import numpy as np
+import pytest
+
+import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+def _system( native, n, d, seed ):
+    """the Laplacian of a Voronoi diagram, rows in tree order, as CSR, and a right-hand side of zero sum"""
+    import torch
+    rng = np.random.default_rng( seed )
+    pos = rng.uniform( 0, 1, ( n, d ) )
+    if d == 2:
+        from sdot import UniformBox
+        order = native.build_tree_2d( pos )[ "seed_indices" ].cpu().numpy()
+        _, ( fi, fj, fc ) = native.measures_2d( pos, None, [ 0, 0, 1, 1 ], UniformBox( [ 0, 0 ], [ 1, 1 ] ), facets = True )
+    else:
+        # ( boxes of a few seeds in a serpentine order: near neighbours near, as the tree's ranks )
+        k = max( 1, round( ( n / 8 ) ** ( 1 / 3 ) ) )
+        c = np.floor( pos * k ).astype( int )
+        order = np.lexsort( ( c[ :, 2 ], c[ :, 1 ] // 2, c[ :, 0 ] // 2 ) )
+        _, ( fi, fj, fc ) = native.measures_3d( pos, None, [ 0, 0, 0, 1, 1, 1 ], None, facets = True )
+    rank = np.empty( n, np.int64 )
+    rank[ order ] = np.arange( n )
+    i, j, c = rank[ fi.cpu().numpy() ], rank[ fj.cpu().numpy() ], fc.cpu().numpy()
+    at = np.lexsort( ( j, i ) )
+    i, j, c = i[ at ], j[ at ], c[ at ]
+    row = np.concatenate( [ [ 0 ], np.cumsum( np.bincount( i, minlength = n ) ) ] )
+    dia = np.bincount( i, weights = c, minlength = n )
+    b = rng.normal( size = n )
+    return row, j, c, dia, torch.as_tensor( b - b.mean() )
+
+
+# the sizes: one level over the coarsest ( 65: the smallest the cycle takes ), a bottom of one level and of two, the first
+# aggregates of 4 and of 8 ( 8192 / 8193 ), a level between the finest and the bottom, 3D rows
+@pytest.mark.parametrize( "n, d", [ ( 65, 2 ), ( 256, 2 ), ( 261, 2 ), ( 2049, 2 ), ( 8192, 2 ), ( 8193, 2 ), ( 40_003, 2 ), ( 150_001, 2 ), ( 700, 3 ), ( 9_001, 3 ) ] )
+@pytest.mark.parametrize( "fp32", [ False, True ] )
+def test_smoothed_cycle_solves_the_laplacian( native, n, d, fp32 ):
+    print( f"case smoothed n={ n } d={ d } fp32={ fp32 }", flush = True )
+    row, col, val, dia, b = _system( native, n, d, n + d )
+    tol = 1e-10
+    x, its = native.linear_solves_2d( row, col, val, dia, b, tol = tol, method = "mg", smoothed = True, fp32 = fp32 )
+    x = x[ 0 ].cpu().numpy()
+    bh = b.numpy()
+    assert 0 < its[ 0 ] < 120
+    # the true residual: the recurrence's, at most `tol`, is accepted when the true one is within 10 times it
+    Ax = dia * x - np.bincount( np.repeat( np.arange( n ), np.diff( row ) ), weights = val * x[ col ], minlength = n )
+    assert np.linalg.norm( bh - Ax ) <= 10 * tol * np.linalg.norm( bh )
+    assert x[ 0 ] == 0
+    if n <= 2100:
+        M = np.diag( dia )
+        np.add.at( M, ( np.repeat( np.arange( n ), np.diff( row ) ), col ), -val )
+        ref = np.zeros( n )
+        ref[ 1: ] = np.linalg.solve( M[ 1:, 1: ], bh[ 1: ] )
+        # ( the error is at most the residual over the smallest eigenvalue of the grounded matrix )
+        lam = np.linalg.eigvalsh( ( M + M.T )[ 1:, 1: ] / 2 )[ 0 ]
+        assert np.linalg.norm( x - ref ) <= 10 * tol * np.linalg.norm( bh ) / lam + 1e-12 * np.linalg.norm( ref )
+
+
+def test_smoothed_cycle_is_bitwise_reproducible( native ):
+    row, col, val, dia, b = _system( native, 30_011, 2, 5 )
+    x = [ native.linear_solves_2d( row, col, val, dia, b, tol = 1e-8, method = "mg", smoothed = True, fp32 = True )[ 0 ].cpu().numpy() for _ in range( 3 ) ]
+    assert np.array_equal( x[ 0 ], x[ 1 ] ) and np.array_equal( x[ 0 ], x[ 2 ] )
+
+
+def test_rows_without_room_go_to_the_other_solvers( native ):
+    # seeds in a random order: aggregates of far seeds, whose coarse rows outgrow any room
+    n = 9_000
+    row, col, val, dia, b = _system( native, n, 2, 7 )
+    p = np.random.default_rng( 8 ).permutation( n )
+    inv = np.argsort( p )
+    i = np.repeat( np.arange( n ), np.diff( row ) )
+    i2, j2 = inv[ i ], inv[ col ]
+    at = np.lexsort( ( j2, i2 ) )
+    row2 = np.concatenate( [ [ 0 ], np.cumsum( np.bincount( i2, minlength = n ) ) ] )
+    x, its = native.linear_solves_2d( row2, j2[ at ], val[ at ], dia[ p ], b.numpy()[ p ], tol = 1e-9, method = "mg", smoothed = True, fp32 = True )
+    x = x[ 0 ].cpu().numpy()
+    assert its[ 0 ] > 0
+    r = b.numpy()[ p ] - ( dia[ p ] * x - np.bincount( i2, weights = val * x[ j2 ], minlength = n ) )
+    assert np.linalg.norm( r ) <= 1e-8 * np.linalg.norm( b.numpy() )
