@@ -821,7 +821,7 @@ int sdot_amd_refresh_majorants_2d( void *stream, long long n, long long nb_nodes
         k_i64_to_i32<<<blocks_for( nb_nodes, 256 ), 256, 0, st>>>( nb_nodes, node_end, t.node_end );
         k_seeds_from<<<blocks_for( n, 256 ), 256, 0, st>>>( n, sorted_positions, sorted_weights, t.seeds );
         check_launch( "refresh_majorants inputs" );
-        refresh_majorants( t, st );
+        refresh_majorants( t, st, true );
         k_majorants_out<<<blocks_for( nb_nodes, 256 ), 256, 0, st>>>( nb_nodes, t.nodes, node_wa, node_wb );
         check_launch( "k_majorants_out" );
         SDOT_HIP( hipStreamSynchronize( st ) );

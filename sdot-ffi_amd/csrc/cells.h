@@ -83,13 +83,11 @@ constexpr int ROW_STEP = 64;
 
 /// the vertex slots of the passes ( the first in LDS, the second in global slots )
 constexpr int CELL_BLOCK = 128;
-constexpr int CAP1 = 16;             ///< first pass, LDS
-#ifndef SDOT_AMD_CAPW
-#define SDOT_AMD_CAPW 16
-#endif
-/// the FP32 walk's LDS slots ( even, at most `CAP1` ): 12 bytes a slot, so its count sets the walk's waves per CU
-constexpr int CAPW = SDOT_AMD_CAPW;
-static_assert( CAPW % 2 == 0 && CAPW >= 6 && CAPW <= CAP1, "the FP32 walk's slots: even, from 6 to CAP1" );
+constexpr int WALK_BLOCK = 256;      ///< the first pass's walk by groups of lanes
+constexpr int WALK_16 = 1 << 15;     ///< sixteen lanes a cell up to this many cells, eight up to `WALK_8`, one beyond ( `launch_walk` )
+constexpr int WALK_8 = 1 << 18;
+constexpr I64 POLY_CHUNK = 1 << 20;  ///< the cells whose FP64 polygons are between the first pass's walk and its finish at a time
+constexpr int CAP1 = 16;             ///< first pass, registers of the cell's lanes
 constexpr int CAP2 = 96;             ///< second pass, LDS ( one wave per block )
 constexpr int CAP3 = 2048;           ///< third pass, global slots: the vertex limit of a cell
 constexpr int PASS2_BLOCKS = 1024;
@@ -103,9 +101,17 @@ enum CellMode { MODE_MASSES = 0, MODE_FACETS = 1, MODE_MOMENTS = 2, MODE_CELLS =
 /// `lo / hi`. Resets and uses the counters; the overflow pass is launched without a read back.
 /// `fp32`: the walk and the cuts in float, every vertex then re-solved in double from its two planes before the measures
 /// ( the cells past the first pass run the FP64 kernel either way ).
-/// `ovf_slots`: the lanes ( a multiple of 64 ) of the third pass, each with `CAP3` vertex slots in global memory.
+/// `ovf_slots`: the lanes ( a multiple of 64 ) of the third pass, each with `CAP3` vertex slots in global memory. `poly_chunk`: the
+/// cells of the FP64 first pass whose polygons are held at a time ( 324 bytes each ).
 void run_cells( const DevTree &t, const double *lo, const double *hi, const Density &dn, int mode, DiagramOut &out, hipStream_t st,
-                bool fp32 = false, int ovf_slots = OVF_SLOTS );
+                bool fp32 = false, int ovf_slots = OVF_SLOTS, I64 poly_chunk = POLY_CHUNK );
+
+/// the event counts of a diagram's passes are gathered in `EV_SHARDS` cache lines ( `[ shard ][ 8 ]` ), a block in its own: one line takes
+/// an atomic every ~12 ns from the whole chip ( five a wave: 64 us for a pass of 1024 waves with nothing to do, 19 of the 27 ms of 300k
+/// 3D cells, a wave each ). `event_shards` gives them cleared, `fold_events` adds them to `events` and clears them
+constexpr int EV_SHARDS = 64;
+unsigned long long *event_shards( hipStream_t st );
+void fold_events( unsigned long long *shards, unsigned long long *events, hipStream_t st );
 
 /// the device scratch a diagram needs besides its outputs ( overflow list and slots )
 void cells_scratch( DiagramOut &out, I64 n, const std::string &tag, hipStream_t st );

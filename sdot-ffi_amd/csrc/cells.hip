@@ -1,8 +1,10 @@
 // The cells of a 2D power diagram on CDNA4.
 //
-// ONE LANE PER CELL, the lanes of a wave holding consecutive tree ranks ( neighbours in space, so the
-// 64 walks of a wave touch the same nodes ). A cell is a convex polygon kept in LDS as three arrays
-// strided by the block ( `x[ i * BLOCK + lane ]` ), in the seed's frame ( a vertex is `x - p0` ).
+// A GROUP OF LANES PER CELL in the first pass ( `GroupCell` ): the polygon's vertices in the registers of the group's lanes, so
+// that a seed's side test, a node's pruning test and a cut each take all vertices at once, and the groups of a wave hold
+// consecutive tree ranks ( neighbours in space: their walks touch the same nodes ). The measures are then taken by one lane per
+// cell, the polygon in LDS as three arrays strided by the block ( `Store`: `x[ i * BLOCK + lane ]` ), which is also how the last
+// passes walk. Coordinates are in the seed's frame ( a vertex is `x - p0` ).
 // Reference semantics followed here ( paths under `src/sdot/include/sdot/` ):
 //   * the cut: `cell/Local2.h:206-298` ( in place, the outside a single cyclic run, intersections
 //     anchored on the inside vertex ), the several-runs rule `cell/Local2.h:300-315`;
@@ -16,7 +18,7 @@
 // An image density is integrated on the cell's edges ( Green: `mass = loop_integral F dy`,
 // `F( x, y ) = int_{x_ref}^x rho( s, y ) ds`, exact piece by piece since `F` is linear in `x` inside a
 // pixel ), so the cell is never cut by the pixel grid.
-// Cells that outgrow `CAP1` LDS slots are listed and redone by a second pass with global slots.
+// Cells that outgrow the first pass's 16 vertices are listed and redone by a second pass ( 96 ), then by a third ( global slots ).
 // Arithmetic is written with explicit `fma` and no contraction, the same expressions as the
 // oracle's, so a constant density gives the oracle's masses to the bit on the same tree.
 
@@ -70,8 +72,8 @@ __device__ void main_run( const S &c, int nb, T dx, T dy, T off, int &i1, int &n
 }
 
 /// the cut by `dx . v <= off`, in place; `CUT_NO_ROOM` leaves the cell intact
-template<class S, class T = typename S::T>
-__device__ int cut( const S &c, int &nb, int cap, T dx, T dy, T off, int pid, Ev &ev ) {
+template<int STRIDE, class T>
+__device__ int cut( const Store<STRIDE, T> &c, int &nb, int cap, T dx, T dy, T off, int pid, Ev &ev ) {
     // the signs, four vertices a step ( their reads issued together: the slots past `nb`, up to the next multiple of
     // four, exist since `cap` is one, and are masked ), with the mask of the outside ones among the first 64
     int nb_out = 0;
@@ -142,22 +144,28 @@ __device__ int cut( const S &c, int &nb, int cap, T dx, T dy, T off, int pid, Ev
     return CUT_DONE;
 }
 
-/// can a seed of node `r` still cut the cell of `( p0, w0 )`? ( exact: per-axis clamp )
-template<class S>
-__device__ __forceinline__ bool can_cut( const S &c, int nb, const NodeRec &r, double p0x, double p0y, double w0, Ev &ev ) {
-    ev.visits += 1;
-    const double hax = r.wa_x / 2, hay = r.wa_y / 2, cb = w0 - r.wb;
-    auto test = [&]( int i ) {
-        const double vx = double( c.X( i ) ), vy = double( c.Y( i ) );
+/// can a seed of node `r` still cut the cell of `( p0, w0 )` at its vertex `( vx, vy )`? ( exact: per-axis clamp )
+struct NodeTest {
+    const NodeRec &r;
+    double p0x, p0y, hax, hay, cb;
+    __device__ __forceinline__ NodeTest( const NodeRec &r_, double x, double y, double w0 )
+        : r( r_ ), p0x( x ), p0y( y ), hax( r_.wa_x / 2 ), hay( r_.wa_y / 2 ), cb( w0 - r_.wb ) {}
+    __device__ __forceinline__ bool operator()( double vx, double vy ) const {
         const double X = vx + p0x, Y = vy + p0y;
         double yx = X + hax, yy = Y + hay;
         yx = yx < r.lo_x ? r.lo_x : ( yx > r.hi_x ? r.hi_x : yx );
         yy = yy < r.lo_y ? r.lo_y : ( yy > r.hi_y ? r.hi_y : yy );
         const double ux = yx - X, uy = yy - Y;
         return cb + ux * ux - vx * vx - r.wa_x * yx + uy * uy - vy * vy - r.wa_y * yy <= 0;
-    };
+    }
+};
+
+/// a node's test on the vertices one by one
+template<class S, class F>
+__device__ __forceinline__ bool any_vertex( const S &c, int nb, const F &at, Ev &ev ) {
+    ev.visits += 1;
     for ( int i = 0; i < nb; i += 2 ) {                  // ( two vertices a step, their reads issued together; `cap` is even )
-        const bool t0 = test( i ), u1 = test( i + 1 ), t1 = i + 1 < nb && u1;
+        const bool t0 = at( c.X( i ), c.Y( i ) ), u1 = at( c.X( i + 1 ), c.Y( i + 1 ) ), t1 = i + 1 < nb && u1;
         if ( t0 ) { ev.prune += i + 1; return true; }
         if ( t1 ) { ev.prune += i + 2; return true; }
     }
@@ -186,44 +194,41 @@ __device__ __forceinline__ Frame32 frame32( double x, double y, double w ) {
     return f;
 }
 
-/// the test of `can_cut` on a float record: the node's outward-rounded box centred on the seed, its rounded-up majorant,
-/// in float. It answers "may cut" up to a margin of 1e-6 of the magnitude of its terms ( sixteen float epsilons, far above the
-/// roundings of the float vertex, of the centred box and of the majorant's constant ), so that it prunes no node the exact
+/// the same test on a float record: the node's outward-rounded box centred on the seed, its rounded-up majorant,
+/// in float. It answers "may cut" up to a margin of 1e-6 of the magnitude of its terms before they cancel ( sixteen float epsilons,
+/// far above the roundings of the float vertex, of the centred box and of the majorant ), so that it prunes no node the exact
 /// test would keep on the same polygon
-template<class S>
-__device__ __forceinline__ bool can_cut( const S &c, int nb, const NodeF &r, const Frame32 &f, Ev &ev ) {
-    ev.visits += 1;
-    const float lx = ( r.lo_x - f.xh ) - f.xl, ly = ( r.lo_y - f.yh ) - f.yl;
-    const float hx = ( r.hi_x - f.xh ) - f.xl, hy = ( r.hi_y - f.yh ) - f.yl;
-    const float cc = ( ( f.wh - r.wb ) + f.wl ) - ( r.wa_x * f.xh + r.wa_y * f.yh );
-    const float hax = 0.5f * r.wa_x, hay = 0.5f * r.wa_y, acc = fabsf( cc );
-    auto test = [&]( int i ) {
-        const float vx = float( c.X( i ) ), vy = float( c.Y( i ) );
+struct NodeTestF {
+    float lx, ly, hx, hy, cc, hax, hay, acc, wx, wy;
+    __device__ __forceinline__ NodeTestF( const NodeF &r, const Frame32 &f ) {
+        lx = ( r.lo_x - f.xh ) - f.xl; ly = ( r.lo_y - f.yh ) - f.yl;
+        hx = ( r.hi_x - f.xh ) - f.xl; hy = ( r.hi_y - f.yh ) - f.yl;
+        const float dx = ( f.xh - 0.5f * ( r.lo_x + r.hi_x ) ) + f.xl, dy = ( f.yh - 0.5f * ( r.lo_y + r.hi_y ) ) + f.yl;
+        const float dw = ( f.wh - r.wc ) + f.wl, bx = r.wa_x * dx, by = r.wa_y * dy;
+        cc = dw - ( bx + by );
+        acc = fabsf( dw ) + ( fabsf( bx ) + fabsf( by ) );
+        hax = 0.5f * r.wa_x; hay = 0.5f * r.wa_y;
+        wx = r.wa_x; wy = r.wa_y;
+    }
+    __device__ __forceinline__ bool operator()( float vx, float vy ) const {
         const float yx = fminf( fmaxf( vx + hax, lx ), hx ), yy = fminf( fmaxf( vy + hay, ly ), hy );
         const float ux = yx - vx, uy = yy - vy;
         const float p = ux * ux + uy * uy, q = vx * vx + vy * vy;
-        const float ax = r.wa_x * yx, ay = r.wa_y * yy;
+        const float ax = wx * yx, ay = wy * yy;
         const float sv = ( p - q ) + ( cc - ( ax + ay ) );
         const float tv = ( p + q ) + ( acc + ( fabsf( ax ) + fabsf( ay ) ) );
         return sv <= 1e-6f * tv;
-    };
-    for ( int i = 0; i < nb; i += 2 ) {                  // ( two vertices a step, their reads issued together; `cap` is even )
-        const bool t0 = test( i ), u1 = test( i + 1 ), t1 = i + 1 < nb && u1;
-        if ( t0 ) { ev.prune += i + 1; return true; }
-        if ( t1 ) { ev.prune += i + 2; return true; }
     }
-    ev.prune += nb;
-    return false;
-}
+};
 
-/// `can_cut` on a double record ( the seed itself in `p0x, p0y, w0` )
-template<class S>
-__device__ __forceinline__ bool can_cut( const S &c, int nb, const NodeRec &r, double p0x, double p0y, double w0, const Frame32 &, Ev &ev ) {
-    return can_cut( c, nb, r, p0x, p0y, w0, ev );
+/// can a seed of node `r` still cut the cell? ( the seed itself in `p0x, p0y, w0`; its float split in `f` )
+template<int STRIDE, class TT>
+__device__ __forceinline__ bool can_cut( const Store<STRIDE, TT> &c, int nb, const NodeRec &r, double p0x, double p0y, double w0, const Frame32 &, Ev &ev ) {
+    return any_vertex( c, nb, NodeTest( r, p0x, p0y, w0 ), ev );
 }
-template<class S>
-__device__ __forceinline__ bool can_cut( const S &c, int nb, const NodeF &r, double, double, double, const Frame32 &f, Ev &ev ) {
-    return can_cut( c, nb, r, f, ev );
+template<int STRIDE, class TT>
+__device__ __forceinline__ bool can_cut( const Store<STRIDE, TT> &c, int nb, const NodeF &r, double, double, double, const Frame32 &f, Ev &ev ) {
+    return any_vertex( c, nb, NodeTestF( r, f ), ev );
 }
 
 __device__ __forceinline__ double proximity( const NodeF &b, double p0x, double p0y ) {
@@ -238,6 +243,7 @@ struct Walk {
     const NodeF   *nodes32;                              ///< the float records ( the FP32 walk )
     const int     *node_end;                             ///< each node's end ( a float record's leaf )
     const double4 *seeds;
+    const int     *leaf_of;                              ///< each rank's leaf, counted from the left
     int depth;
 };
 
@@ -249,6 +255,225 @@ __device__ __forceinline__ bool node_live( const NodeF &r ) { return r.beg >= 0;
 __device__ __forceinline__ int node_stop( const Walk &, int, const NodeRec &r ) { return r.end; }
 __device__ __forceinline__ int node_stop( const Walk &wk, int m, const NodeF & ) { return wk.node_end[ m ]; }
 
+/// the cell the cuts start from: the domain polygon as it is ( its edges: `-5 - i` ) or the box ( its sides: bottom, right, top,
+/// left ); returns its vertex count, -1 when `cap` is too few
+template<int STRIDE, class TT>
+__device__ __forceinline__ int start_cell( const Store<STRIDE, TT> &c, int cap, const double *lo, const double *hi, const Polygon2 &dom, double p0x,
+                                           double p0y ) {
+    if ( dom.nb > 0 ) {
+        if ( dom.nb > cap ) return -1;
+        for ( int i = 0; i < dom.nb; ++i ) { c.X( i ) = TT( dom.x[ i ] - p0x ); c.Y( i ) = TT( dom.y[ i ] - p0y ); c.I( i ) = -5 - i; }
+        return dom.nb;
+    }
+    c.X( 0 ) = TT( lo[ 0 ] - p0x ); c.Y( 0 ) = TT( lo[ 1 ] - p0y );
+    c.X( 1 ) = TT( hi[ 0 ] - p0x ); c.Y( 1 ) = TT( lo[ 1 ] - p0y );
+    c.X( 2 ) = TT( hi[ 0 ] - p0x ); c.Y( 2 ) = TT( hi[ 1 ] - p0y );
+    c.X( 3 ) = TT( lo[ 0 ] - p0x ); c.Y( 3 ) = TT( hi[ 1 ] - p0y );
+    for ( int i = 0; i < 4; ++i ) c.I( i ) = -1 - i;
+    return 4;
+}
+
+// ---- a cell in the registers of a group of lanes ---------------------------------------------------------------------
+//
+// Vertex `i` on lane `i % G` of the group, in its register `i / G`. Every lane of the group runs the same walk ( the same loads,
+// from one cache line, and the same decisions: ballots and shuffles within the group ), and holds its own vertices. What bounds the
+// walk is its serial chain and the divergence between the cells of a wave: one lane per cell ran ~6 vertices one after the other in
+// every test, and 64 different walks a wave. The cut builds the same polygon, vertex for vertex in the same slots, with the same
+// arithmetic as `cut` on a `Store`: the cells are the same to the bit.
+
+using Mask32 = unsigned;
+using Mask64 = unsigned long long;
+using Mask128 = unsigned __int128;
+__device__ __forceinline__ int mask_count( Mask32 m ) { return __popc( m ); }
+__device__ __forceinline__ int mask_first( Mask32 m ) { return __ffs( int( m ) ) - 1; }
+__device__ __forceinline__ int mask_count( Mask64 m ) { return __popcll( m ); }
+__device__ __forceinline__ int mask_first( Mask64 m ) { return __ffsll( (long long) m ) - 1; }
+__device__ __forceinline__ int mask_count( Mask128 m ) { return __popcll( Mask64( m ) ) + __popcll( Mask64( m >> 64 ) ); }
+__device__ __forceinline__ int mask_first( Mask128 m ) { return Mask64( m ) ? mask_first( Mask64( m ) ) : 64 + mask_first( Mask64( m >> 64 ) ); }
+
+template<int G, int V, class TT>
+struct GroupCell {
+    using T = TT;
+    static constexpr int CAP = G * V;
+    using Mask = typename std::conditional<( CAP > 64 ), Mask128, typename std::conditional<( CAP > 32 ), Mask64, Mask32>::type>::type;
+    T   x[ V ], y[ V ];
+    int id[ V ];
+    int lane, first;                                     ///< the lane's place in its group, the group's first lane in its wave
+
+    __device__ __forceinline__ GroupCell() {
+        lane = threadIdx.x & ( G - 1 );
+        first = ( threadIdx.x & 63 ) & ~( G - 1 );
+    }
+    /// the vertices `i` for which `f( v )` holds on their lane ( `i = lane + v G` )
+    template<class F>
+    __device__ __forceinline__ Mask bits( F f ) const {
+        Mask m = 0;
+#pragma unroll
+        for ( int v = 0; v < V; ++v ) {
+            const Mask64 b = __ballot( f( v ) ) >> first;
+            m |= ( G == 64 ? Mask( b ) : Mask( unsigned( b ) & ( ( 1u << ( G & 31 ) ) - 1 ) ) ) << ( v * G );
+        }
+        return m;
+    }
+    /// vertex `i`'s value of `a`
+    template<class U>
+    __device__ __forceinline__ U get( const U ( &a )[ V ], int i ) const {
+        U r = __shfl( a[ 0 ], i & ( G - 1 ), G );
+#pragma unroll
+        for ( int v = 1; v < V; ++v ) { const U q = __shfl( a[ v ], i & ( G - 1 ), G ); r = i / G == v ? q : r; }
+        return r;
+    }
+};
+
+template<int G, int V, class T>
+__device__ __forceinline__ int start_cell( GroupCell<G, V, T> &c, int cap, const double *lo, const double *hi, const Polygon2 &dom, double p0x,
+                                           double p0y ) {
+    if ( dom.nb > 0 && dom.nb > cap ) return -1;
+#pragma unroll
+    for ( int v = 0; v < V; ++v ) {
+        const int i = c.lane + v * G;
+        if ( dom.nb > 0 ) {
+            c.x[ v ] = T( dom_at( dom.x, i ) - p0x );
+            c.y[ v ] = T( dom_at( dom.y, i ) - p0y );
+            c.id[ v ] = -5 - i;
+        } else {
+            c.x[ v ] = T( ( i == 1 || i == 2 ? hi[ 0 ] : lo[ 0 ] ) - p0x );
+            c.y[ v ] = T( ( i == 2 || i == 3 ? hi[ 1 ] : lo[ 1 ] ) - p0y );
+            c.id[ v ] = -1 - i;
+        }
+    }
+    return dom.nb > 0 ? dom.nb : 4;
+}
+
+/// the cut by `dx . v <= off` ( as `cut` on a `Store` )
+template<int G, int V, class T>
+__device__ __forceinline__ int cut( GroupCell<G, V, T> &c, int &nb, int cap, T dx, T dy, T off, int pid, Ev &ev ) {
+    using Mask = typename GroupCell<G, V, T>::Mask;
+    T s[ V ];
+#pragma unroll
+    for ( int v = 0; v < V; ++v ) s[ v ] = fma( dx, c.x[ v ], fma( dy, c.y[ v ], -off ) );
+    const Mask out = c.bits( [&]( int v ) { return c.lane + v * G < nb && s[ v ] > 0; } );
+    ev.side += nb;
+    if ( ! out ) return CUT_UNCHANGED;
+    int nb_out = mask_count( out );
+    if ( nb_out == nb ) { nb = 0; return CUT_EMPTY; }
+    const Mask full = nb == int( 8 * sizeof( Mask ) ) ? ~Mask( 0 ) : ( Mask( 1 ) << nb ) - 1;
+    const Mask starts = out & ~( ( ( out << 1 ) | ( out >> ( nb - 1 ) ) ) & full );
+    int i1 = mask_first( starts );
+    if ( mask_count( starts ) != 1 ) {                   // several runs: the one holding the largest `s` ( the first such vertex )
+        int a = c.lane;
+        T sa = c.lane < nb ? s[ 0 ] : -INFINITY;
+#pragma unroll
+        for ( int v = 1; v < V; ++v ) if ( c.lane + v * G < nb && s[ v ] > sa ) { a = c.lane + v * G; sa = s[ v ]; }
+        for ( int o = G / 2; o > 0; o >>= 1 ) {
+            const T so = __shfl_xor( sa, o, G );
+            const int ao = __shfl_xor( a, o, G );
+            if ( so > sa || ( so == sa && ao < a ) ) { sa = so; a = ao; }
+        }
+        i1 = a;
+        nb_out = 1;
+        for ( int n = 1, q = a ? a - 1 : nb - 1; n < nb && ( out >> q & 1 ); ++n, q = q ? q - 1 : nb - 1 ) i1 = q;
+        for ( int n = 1, q = a + 1 < nb ? a + 1 : 0; n < nb && ( out >> q & 1 ); ++n, q = q + 1 < nb ? q + 1 : 0 ) ++nb_out;
+        nb_out += a >= i1 ? a - i1 : a - i1 + nb;
+    }
+    const int nb_in = nb - nb_out, new_nb = nb_in + 2;
+    if ( new_nb > cap ) return CUT_NO_ROOM;
+    const int j0 = i1 ? i1 - 1 : nb - 1, j2 = i1 + nb_out - 1 >= nb ? i1 + nb_out - 1 - nb : i1 + nb_out - 1, j3 = j2 + 1 == nb ? 0 : j2 + 1;
+    // the two new vertices take the places `at` and `at + 1`; the vertices before keep theirs, those after follow
+    const bool wrap = i1 > j2;
+    const int at = wrap ? 0 : i1, shift = wrap ? j3 - 2 : nb_out - 2;
+    T nx[ V ], ny[ V ];
+    int ni[ V ];
+#pragma unroll
+    for ( int v = 0; v < V; ++v ) {
+        const int t = c.lane + v * G;
+        const bool A = t == at, B = t == at + 1;
+        int src = ! wrap && t < at ? t : t + shift;
+        src = src < 0 ? 0 : src >= G * V ? G * V - 1 : src;
+        const int in = A ? j0 : B ? j3 : src, ou = A ? i1 : B ? j2 : src;
+        const T xi = c.get( c.x, in ), yi = c.get( c.y, in ), si = c.get( s, in );
+        const T xo = c.get( c.x, ou ), yo = c.get( c.y, ou ), so = c.get( s, ou );
+        const int io = c.get( c.id, ou );
+        const T f = si / ( si - so );
+        nx[ v ] = A || B ? fma( xo - xi, f, xi ) : xi;
+        ny[ v ] = A || B ? fma( yo - yi, f, yi ) : yi;
+        ni[ v ] = A ? pid : io;
+    }
+#pragma unroll
+    for ( int v = 0; v < V; ++v ) { c.x[ v ] = nx[ v ]; c.y[ v ] = ny[ v ]; c.id[ v ] = ni[ v ]; }
+    nb = new_nb;
+    ev.newv += 2;
+    ev.cuts += 1;
+    return CUT_DONE;
+}
+
+/// the outcome of a pruning test on a group's vertices, and the vertices the one-by-one test would have looked at
+template<class Mask>
+__device__ __forceinline__ bool any_of( Mask hit, int nb, Ev &ev ) {
+    ev.prune += hit ? unsigned( mask_first( hit ) + 1 ) : unsigned( nb );
+    return bool( hit );
+}
+
+template<int G, int V, class T>
+__device__ __forceinline__ bool can_cut( const GroupCell<G, V, T> &c, int nb, const NodeRec &r, double p0x, double p0y, double w0, const Frame32 &, Ev &ev ) {
+    ev.visits += 1;
+    const NodeTest t( r, p0x, p0y, w0 );
+    return any_of( c.bits( [&]( int v ) { return c.lane + v * G < nb && t( double( c.x[ v ] ), double( c.y[ v ] ) ); } ), nb, ev );
+}
+template<int G, int V, class T>
+__device__ __forceinline__ bool can_cut( const GroupCell<G, V, T> &c, int nb, const NodeF &r, double, double, double, const Frame32 &f, Ev &ev ) {
+    ev.visits += 1;
+    const NodeTestF t( r, f );
+    return any_of( c.bits( [&]( int v ) { return c.lane + v * G < nb && t( float( c.x[ v ] ), float( c.y[ v ] ) ); } ), nb, ev );
+}
+
+/// the node at level `L` of a tree `depth` high on the way to leaf `j` ( a left child is 1 after its parent, a right one `2^height` )
+__device__ __forceinline__ int way_node( int j, int L, int depth ) {
+    const int pre = j >> ( depth - 1 - L );
+    return 2 * ( pre << ( depth - 1 - L ) ) + L - __popc( unsigned( pre ) );
+}
+
+/// whether the walk may start in the seed's own leaf. The float walk: always ( its test keeps what the exact one keeps ). The FP64
+/// walk by a group: the tests it would have made on the way down, a node a lane instead of one after the other, counted as it would
+/// have counted them; `false` ( the walk starts at the root ) if one of them or a tie sends it elsewhere first. One lane alone
+/// saves nothing by it
+template<int STRIDE, class TT>
+__device__ __forceinline__ bool own_way( const Store<STRIDE, TT> &, int, const Walk &, int, const double *, const double *, const Polygon2 &, double,
+                                         double, double, const NodeRec *, Ev & ) { return false; }
+template<class S>
+__device__ __forceinline__ bool own_way( const S &, int, const Walk &, int, const double *, const double *, const Polygon2 &, double, double, double,
+                                         const NodeF *, Ev & ) { return true; }
+template<int G, int V, class T>
+__device__ __forceinline__ bool own_way( const GroupCell<G, V, T> &c, int nb, const Walk &wk, int own, const double *lo, const double *hi,
+                                         const Polygon2 &dom, double p0x, double p0y, double w0, const NodeRec *kind, Ev &ev ) {
+    if ( dom.nb > 0 ) return false;
+    bool ok = true;
+    unsigned looked = 0;
+    for ( int L = c.lane; L < wk.depth; L += G ) {
+        const int m = way_node( own, L, wk.depth ), up = 1 << ( wk.depth - L );
+        const NodeRec r = node_at( wk, m, kind );
+        const NodeTest t( r, p0x, p0y, w0 );
+        int first = 4;
+#pragma unroll
+        for ( int i = 3; i >= 0; --i )
+            if ( t( ( i == 1 || i == 2 ? hi[ 0 ] : lo[ 0 ] ) - p0x, ( i >= 2 ? hi[ 1 ] : lo[ 1 ] ) - p0y ) ) first = i;
+        looked += first + 1;
+        ok = ok && first < 4;
+        if ( L > 0 ) {
+            const bool is_left = ! ( own >> ( wk.depth - 1 - L ) & 1 );
+            const NodeRec s = node_at( wk, is_left ? m - 1 + up : m - up + 1, kind );
+            const double pr = proximity( r, p0x, p0y ), ps = proximity( s, p0x, p0y );
+            ok = ok && ( is_left ? pr <= ps : ! ( ps <= pr ) );
+        }
+    }
+    const Mask64 all = __ballot( ok ) >> c.first;
+    if ( ( G == 64 ? all : all & ( ( Mask64( 1 ) << ( G & 63 ) ) - 1 ) ) != ( G == 64 ? ~Mask64( 0 ) : ( Mask64( 1 ) << ( G & 63 ) ) - 1 ) ) return false;
+    for ( int o = G / 2; o > 0; o >>= 1 ) looked += __shfl_xor( looked, o, G );
+    ev.visits += wk.depth;
+    ev.prune += looked;
+    return true;
+}
+
 /// builds the cell of rank `k` in `c`; returns the vertex count ( 0: empty ), or -1 when the slots
 /// were too few ( the cell is then left for the next pass ). One loop iteration does ONE thing of about
 /// the same cost -- a cut by one seed of the open leaf, or one node's test ( after a pop if needed ) --
@@ -256,32 +481,35 @@ __device__ __forceinline__ int node_stop( const Walk &wk, int m, const NodeF & )
 /// ahead of their use: a descent loads both children's records ( the nearer is the next node tested,
 /// from registers ), and a leaf's next seed is loaded while the current one cuts.
 template<class S, class ND = NodeRec>
-__device__ __forceinline__ int make_cell( const Walk &wk, int k, const double *lo, const double *hi, const Polygon2 &dom, const S &c, int cap,
-                                          Ev &ev ) {
+__device__ __forceinline__ int make_cell( const Walk &wk, int k, const double *lo, const double *hi, const Polygon2 &dom, S &c, int cap, Ev &ev ) {
     using T = typename S::T;
     const ND *kind = nullptr;                            // ( which records the walk reads: `NodeRec` or the float `NodeF` )
     const double4 p = wk.seeds[ k ];
     const double p0x = p.x, p0y = p.y, w0 = p.z;
     const Frame32 f32 = frame32( p0x, p0y, w0 );
-    int nb = 4;
-    if ( dom.nb > 0 ) {                                  // the polygon domain, laid down as it is ( its edges: `-5 - i` )
-        if ( dom.nb > cap ) return -1;
-        for ( int i = 0; i < dom.nb; ++i ) { c.X( i ) = T( dom.x[ i ] - p0x ); c.Y( i ) = T( dom.y[ i ] - p0y ); c.I( i ) = -5 - i; }
-        nb = dom.nb;
-    } else {
-        c.X( 0 ) = T( lo[ 0 ] - p0x ); c.Y( 0 ) = T( lo[ 1 ] - p0y );
-        c.X( 1 ) = T( hi[ 0 ] - p0x ); c.Y( 1 ) = T( lo[ 1 ] - p0y );
-        c.X( 2 ) = T( hi[ 0 ] - p0x ); c.Y( 2 ) = T( hi[ 1 ] - p0y );
-        c.X( 3 ) = T( lo[ 0 ] - p0x ); c.Y( 3 ) = T( hi[ 1 ] - p0y );
-        for ( int i = 0; i < 4; ++i ) c.I( i ) = -1 - i; // the box's sides: bottom, right, top, left
-    }
+    int nb = start_cell( c, cap, lo, hi, dom, p0x, p0y );
+    if ( nb < 0 ) return -1;
     int m = 0, h = wk.depth;
-    unsigned long long pend = 0, left = 0;
+    unsigned pend = 0, left = 0;                         // ( a tree is at most 29 high )
     int q = 0, qe = 0;                                   // the open leaf's remaining seeds
     bool visit = true;                                   // ( m, h ) is still to be tested
     ND rec;                                              // the record of ( m, h ) when the descent loaded it
     bool have = false;
     double4 nxt = make_double4( 0, 0, 0, 0 );            // the open leaf's seed `q`, loaded ahead
+    // THE WAY DOWN TO THE SEED'S OWN LEAF: every node on it holds the seed, so none is pruned, and the nearest child is the one that
+    // holds it ( a tie apart ): the walk starts in that leaf with every sibling on the way still pending
+    const int own = wk.leaf_of[ k ];
+    if ( own_way( c, nb, wk, own, lo, hi, dom, p0x, p0y, w0, kind, ev ) ) {
+        m = way_node( own, wk.depth - 1, wk.depth );
+        h = 1;
+        pend = ( 1u << wk.depth ) - 2;
+        left = ( ~unsigned( own ) << 1 ) & pend;
+        const ND r = node_at( wk, m, kind );
+        q = r.beg;
+        qe = node_stop( wk, m, r );
+        nxt = wk.seeds[ q ];
+        visit = false;
+    }
     // two inner loops, "while-while": the open leaf's seeds, then the walk down to the next leaf that may cut. A wave's
     // lanes run one kind of step at a time ( one loop with both kinds of step in it runs both bodies whenever its lanes
     // disagree ); each lane takes the same steps in the same order either way
@@ -300,13 +528,13 @@ __device__ __forceinline__ int make_cell( const Walk &wk, int k, const double *l
         for ( bool open = false; ! open; ) {
             if ( ! visit ) {                                  // pop: climb to the lowest pending height, take the sibling
                 if ( ! pend ) return nb;
-                const int hp = __ffsll( (long long) pend ) - 1;
+                const int hp = __ffs( int( pend ) ) - 1;
                 if ( h < hp ) {                              // up from `h` to `hp`: a left child's parent is 1 before it, a right
-                    const unsigned long long R = ( ( 1ull << hp ) - 1 ) & ~( ( 1ull << h ) - 1 );   // child's `2^height` before
-                    m -= __popcll( left & R ) + int( R & ~left );
+                    const unsigned R = ( ( 1u << hp ) - 1 ) & ~( ( 1u << h ) - 1 );   // child's `2^height` before
+                    m -= __popc( left & R ) + int( R & ~left );
                     h = hp;
                 }
-                const unsigned long long bit = 1ull << hp;
+                const unsigned bit = 1u << hp;
                 if ( left & bit ) { m = m - 1 + ( 1 << hp ); left &= ~bit; }
                 else              { m = m + 1 - ( 1 << hp ); left |= bit; }
                 pend &= ~bit;
@@ -324,7 +552,7 @@ __device__ __forceinline__ int make_cell( const Walk &wk, int k, const double *l
                     const int lc = m + 1, rc = m + ( 1 << ( h - 1 ) );
                     const ND rl = node_at( wk, lc, kind ), rr = node_at( wk, rc, kind );
                     const bool go_left = proximity( rl, p0x, p0y ) <= proximity( rr, p0x, p0y );
-                    const unsigned long long bit = 1ull << ( h - 1 );
+                    const unsigned bit = 1u << ( h - 1 );
                     pend |= bit;
                     left = go_left ? ( left | bit ) : ( left & ~bit );
                     m = go_left ? lc : rc;
@@ -483,14 +711,17 @@ __device__ __forceinline__ unsigned long long wave_sum64( unsigned long long v )
     return v;
 }
 
-/// the polygons of the FP32 kernel's walk, for its finish: slot `i` of rank `k` at `i n + k`
-struct Poly32 {
-    float *x, *y;
-    int   *id, *nb;
+/// the polygons of a first pass, from its walk to its finish: slot `i` of rank `k0 + k` at `i stride + k`
+template<class T>
+struct Poly {
+    T   *x, *y;
+    int *id, *nb;
+    I64 stride;
 };
 
 struct Params {
     Walk          wk;
+    unsigned long long *shards;                          ///< [ EV_SHARDS ][ 8 ] the event counts, a cache line each
     int           n;
     double        lo[ 2 ], hi[ 2 ];
     Density       dn;
@@ -649,22 +880,30 @@ __device__ void finish_cell( const Params &P, int k, const S &c, int nb, bool ac
 __device__ __forceinline__ void flush_events( const Params &P, const Ev &ev ) {
     const unsigned long long a = wave_sum64( ev.side ), b = wave_sum64( ev.prune ), c = wave_sum64( ev.newv );
     const unsigned long long d = wave_sum64( ev.visits ), e = wave_sum64( ev.cuts );
-    if ( ( threadIdx.x & 63 ) == 0 ) {
-        atomicAdd( &P.out.events[ 0 ], a );
-        atomicAdd( &P.out.events[ 1 ], b );
-        atomicAdd( &P.out.events[ 2 ], c );
-        atomicAdd( &P.out.events[ 3 ], d );
-        atomicAdd( &P.out.events[ 4 ], e );
+    if ( ( threadIdx.x & 63 ) == 0 && d ) {
+        unsigned long long *to = P.shards + 8 * ( blockIdx.x & ( EV_SHARDS - 1 ) );
+        atomicAdd( &to[ 0 ], a );
+        atomicAdd( &to[ 1 ], b );
+        atomicAdd( &to[ 2 ], c );
+        atomicAdd( &to[ 3 ], d );
+        atomicAdd( &to[ 4 ], e );
     }
 }
 
-/// the rank of the calling lane in a first pass: the blocks of one XCD take a contiguous range of ranks ( blocks are
-/// dealt round-robin to the 8 XCDs, each with its own L2 )
-__device__ __forceinline__ int pass1_rank() {
+__global__ __launch_bounds__( EV_SHARDS ) void k_fold_events( unsigned long long *shards, unsigned long long *events ) {
+    for ( int q = 0; q < 5; ++q ) {
+        const unsigned long long v = wave_sum64( shards[ 8 * threadIdx.x + q ] );
+        shards[ 8 * threadIdx.x + q ] = 0;
+        if ( threadIdx.x == 0 ) events[ q ] += v;
+    }
+}
+
+/// the block's place in a first pass: the blocks of one XCD take consecutive places ( blocks are dealt round-robin to the 8 XCDs,
+/// each with its own L2 )
+__device__ __forceinline__ int pass1_block() {
     const int nblk = int( gridDim.x ), b = int( blockIdx.x );
     const int per = nblk / 8, rem = nblk % 8, xcd = b % 8, slot = b / 8;
-    const int lb = xcd < rem ? xcd * ( per + 1 ) + slot : rem * ( per + 1 ) + ( xcd - rem ) * per + slot;
-    return lb * CELL_BLOCK + int( threadIdx.x );
+    return xcd < rem ? xcd * ( per + 1 ) + slot : rem * ( per + 1 ) + ( xcd - rem ) * per + slot;
 }
 
 /// the plane of a cut in double, from its identifier ( `gpu/Cell2D.cuh:946-971` ): the bisector with seed `id`,
@@ -699,51 +938,70 @@ __device__ __forceinline__ void plane_of( const Params &P, int id, double p0x, d
 
 } // namespace
 
-/// the first pass: one lane per cell, `CAP1` vertex slots in LDS
-__global__ __launch_bounds__( CELL_BLOCK ) void k_cells_pass1( Params P ) {
-    __shared__ double sx[ CAP1 * CELL_BLOCK ], sy[ CAP1 * CELL_BLOCK ];
-    __shared__ int sid[ CAP1 * CELL_BLOCK ];
-    const int k = pass1_rank();
-    const Store<CELL_BLOCK> c{ sx + threadIdx.x, sy + threadIdx.x, sid + threadIdx.x };
+/// THE FIRST PASS'S WALK, `G` lanes a cell with `V` vertices each ( `CAP1` in all ), over the ranks `[ k0, k1 )`: the polygon to `po`, its
+/// vertex count ( -1: listed for the second pass ). `T` float: the FP32 kernel's ( the seed's frame; each plane computed in double, then
+/// rounded; float node records )
+template<int G, int V, class T, class ND>
+__global__ __launch_bounds__( WALK_BLOCK ) void k_cells_walk( Params P, Poly<T> po, int k0, int k1 ) {
+    static_assert( G * V == CAP1, "the first pass's vertices" );
+    const int i = pass1_block() * ( WALK_BLOCK / G ) + int( threadIdx.x ) / G, k = k0 + i;
+    GroupCell<G, V, T> c;
     Ev ev;
-    int nb = 0;
-    bool active = k < P.n;
-    if ( active ) {
-        nb = make_cell( P.wk, k, P.lo, P.hi, P.dn.dom, c, CAP1, ev );
-        if ( nb < 0 ) {
-            const unsigned at = atomicAdd( &P.out.counters[ 1 ], 1u );
-            P.out.ovf_list[ at ] = k;
-            active = false;
+    if ( k < k1 ) {
+        const int nb = make_cell<GroupCell<G, V, T>, ND>( P.wk, k, P.lo, P.hi, P.dn.dom, c, CAP1, ev );
+        if ( c.lane == 0 ) {
+            po.nb[ i ] = nb;
+            if ( nb < 0 ) P.out.ovf_list[ atomicAdd( &P.out.counters[ 1 ], 1u ) ] = k;
         }
+#pragma unroll
+        for ( int v = 0; v < V; ++v )
+            if ( c.lane + v * G < nb ) {
+                const I64 at = ( c.lane + v * G ) * po.stride + i;
+                po.x[ at ] = c.x[ v ];
+                po.y[ at ] = c.y[ v ];
+                po.id[ at ] = c.id[ v ];
+            }
     }
-    finish_cell( P, k, c, nb, active, true );
+    if ( c.lane ) ev = Ev();                             // ( a group's lanes count the same events )
     flush_events( P, ev );
 }
 
-/// the first pass of the FP32 kernel: the walk and the cuts in float ( the seed's frame; each plane computed in double,
-/// then rounded ), `CAPW` float slots in LDS; the polygon ( float vertices, the cut of each edge ) to `po`, slot `i` of
-/// rank `k` at `i n + k`, and its vertex count ( -1: listed for the second pass, which runs the FP64 kernel )
-__global__ __launch_bounds__( CELL_BLOCK ) void k_cells_walk32( Params P, Poly32 po ) {
-    __shared__ float sx[ CAPW * CELL_BLOCK ], sy[ CAPW * CELL_BLOCK ];
-    __shared__ int sid[ CAPW * CELL_BLOCK ];
-    const int k = pass1_rank();
-    const Store<CELL_BLOCK, float> c{ sx + threadIdx.x, sy + threadIdx.x, sid + threadIdx.x };
+/// the same walk by one lane a cell, its vertices in LDS: for clouds that fill the chip, where the groups' repeated control costs
+/// more than the divergence it avoids
+template<class T, class ND>
+__global__ __launch_bounds__( CELL_BLOCK ) void k_cells_walk_lanes( Params P, Poly<T> po, int k0, int k1 ) {
+    __shared__ T sx[ CAP1 * CELL_BLOCK ], sy[ CAP1 * CELL_BLOCK ];
+    __shared__ int sid[ CAP1 * CELL_BLOCK ];
+    const int i = pass1_block() * CELL_BLOCK + int( threadIdx.x ), k = k0 + i;
+    Store<CELL_BLOCK, T> c{ sx + threadIdx.x, sy + threadIdx.x, sid + threadIdx.x };
     Ev ev;
-    if ( k < P.n ) {
-        const int nb = make_cell<Store<CELL_BLOCK, float>, NodeF>( P.wk, k, P.lo, P.hi, P.dn.dom, c, CAPW, ev );
-        if ( nb < 0 ) {
-            const unsigned at = atomicAdd( &P.out.counters[ 1 ], 1u );
-            P.out.ovf_list[ at ] = k;
-        }
-        po.nb[ k ] = nb;
-        for ( int i = 0; i < nb; ++i ) {
-            const size_t at = size_t( i ) * size_t( P.n ) + size_t( k );
-            po.x[ at ] = c.X( i );
-            po.y[ at ] = c.Y( i );
-            po.id[ at ] = c.I( i );
+    if ( k < k1 ) {
+        const int nb = make_cell<Store<CELL_BLOCK, T>, ND>( P.wk, k, P.lo, P.hi, P.dn.dom, c, CAP1, ev );
+        if ( nb < 0 ) P.out.ovf_list[ atomicAdd( &P.out.counters[ 1 ], 1u ) ] = k;
+        po.nb[ i ] = nb;
+        for ( int v = 0; v < nb; ++v ) {
+            const I64 at = v * po.stride + i;
+            po.x[ at ] = c.X( v );
+            po.y[ at ] = c.Y( v );
+            po.id[ at ] = c.I( v );
         }
     }
     flush_events( P, ev );
+}
+
+/// the end of the FP64 kernel's first pass, one lane a cell: its measures and facets
+__global__ __launch_bounds__( CELL_BLOCK ) void k_cells_finish( Params P, Poly<double> po, int k0, int k1 ) {
+    __shared__ double sx[ CAP1 * CELL_BLOCK ], sy[ CAP1 * CELL_BLOCK ];
+    __shared__ int sid[ CAP1 * CELL_BLOCK ];
+    const int i = pass1_block() * CELL_BLOCK + int( threadIdx.x ), k = k0 + i;
+    const Store<CELL_BLOCK> c{ sx + threadIdx.x, sy + threadIdx.x, sid + threadIdx.x };
+    const int nb = k < k1 ? po.nb[ i ] : -1;
+    for ( int e = 0; e < nb; ++e ) {
+        c.X( e ) = po.x[ e * po.stride + i ];
+        c.Y( e ) = po.y[ e * po.stride + i ];
+        c.I( e ) = po.id[ e * po.stride + i ];
+    }
+    finish_cell( P, k, c, nb, nb >= 0, true );
 }
 
 /// the end of the FP32 kernel's first pass: each vertex re-solved in double from the planes of the edge that arrives and
@@ -751,11 +1009,11 @@ __global__ __launch_bounds__( CELL_BLOCK ) void k_cells_walk32( Params P, Poly32
 /// ( `det^2 > 1e-12 |n_a|^2 |n_b|^2` ) and it lies within what the float vertex can be off by ( `|v - v_f|^2 det^2 <=
 /// 1e-8 L^2 |n_a|^2 |n_b|^2`, `L` the farthest corner of the box from the seed ); else the float vertex projected on the
 /// plane of the edge that leaves it. Then the cell's measures and facets in double, as the FP64 kernel's.
-__global__ __launch_bounds__( CELL_BLOCK ) void k_cells_finish32( Params P, Poly32 po ) {
+__global__ __launch_bounds__( CELL_BLOCK ) void k_cells_finish32( Params P, Poly<float> po ) {
     __shared__ double sx[ CAP1 * CELL_BLOCK ], sy[ CAP1 * CELL_BLOCK ];
     __shared__ int sid[ CAP1 * CELL_BLOCK ];
-    const int k = pass1_rank();
-    const Store<CELL_BLOCK> c{ sx + threadIdx.x, sy + threadIdx.x, sid + threadIdx.x };
+    const int k = pass1_block() * CELL_BLOCK + int( threadIdx.x );
+    Store<CELL_BLOCK> c{ sx + threadIdx.x, sy + threadIdx.x, sid + threadIdx.x };
     const bool live = k < P.n;
     const int nb = live ? po.nb[ k ] : 0;
     bool active = live && nb >= 0;
@@ -815,18 +1073,41 @@ __global__ void k_sym_check( int n, const int *row_off, const int *row_cnt, cons
     }
 }
 
+/// the cell of rank `k` by a whole wave, at most `CAP2` vertices, copied into the first lane's column of `c` ( every lane gets the
+/// vertex count; -1: too few slots )
+__device__ __forceinline__ int wave_cell( const Params &P, int k, const Store<64> &c, Ev &ev ) {
+    GroupCell<64, 2, double> g;
+    const int nb = make_cell<GroupCell<64, 2, double>, NodeRec>( P.wk, k, P.lo, P.hi, P.dn.dom, g, CAP2, ev );
+    const Store<64> d{ c.x - threadIdx.x, c.y - threadIdx.x, c.id - threadIdx.x };
+#pragma unroll
+    for ( int v = 0; v < 2; ++v ) {
+        const int i = int( threadIdx.x ) + 64 * v;
+        if ( i < nb ) { d.X( i ) = g.x[ v ]; d.Y( i ) = g.y[ v ]; d.I( i ) = g.id[ v ]; }
+    }
+    if ( threadIdx.x ) ev = Ev();
+    __syncthreads();
+    return nb;
+}
+
 /// the cells `k_sym_check` listed, redone by the FP64 kernel ( one lane per cell, `CAP2` slots in LDS ); each writes a new row
-/// and its measures over the FP32 ones. A cell past `CAP2` keeps its FP32 result. The list is short ( hundreds of cells ) and
-/// dealt one cell per wave before any wave takes a second: a wave's time is then one walk, not its lanes' divergent walks
-/// one after the other
+/// and its measures over the FP32 ones. A cell past `CAP2` keeps its FP32 result. A list of at most a cell per block ( hundreds of
+/// cells, the common case ) is walked by whole waves, a vertex a lane ( 1M cells: the redo and the second pass together 1.2 -> 0.5 ms a diagram ); a longer one by one lane per cell
 __global__ __launch_bounds__( 64 ) void k_cells_redo( Params P, const int *list, const unsigned *count_p ) {
     __shared__ double sx[ CAP2 * 64 ], sy[ CAP2 * 64 ];
     __shared__ int sid[ CAP2 * 64 ];
-    const Store<64> c{ sx + threadIdx.x, sy + threadIdx.x, sid + threadIdx.x };
+    Store<64> c{ sx + threadIdx.x, sy + threadIdx.x, sid + threadIdx.x };
     const unsigned count = *count_p;
+    Ev ev;
+    if ( count <= gridDim.x ) {
+        if ( blockIdx.x < count ) {
+            const int k = list[ blockIdx.x ], nb = wave_cell( P, k, c, ev );
+            finish_cell( P, k, c, nb, threadIdx.x == 0 && nb >= 0, false );
+            flush_events( P, ev );
+        }
+        return;
+    }
     const unsigned lanes = gridDim.x * 64;
     const unsigned rounds = ( count + lanes - 1 ) / lanes;
-    Ev ev;
     for ( unsigned r = 0; r < rounds; ++r ) {
         const unsigned idx = r * lanes + threadIdx.x * gridDim.x + blockIdx.x;   // consecutive cells to different waves
         const bool live = idx < count;
@@ -842,17 +1123,26 @@ __global__ __launch_bounds__( 64 ) void k_cells_redo( Params P, const int *list,
     flush_events( P, ev );
 }
 
-/// the second pass: the cells that outgrew `CAP1`, one lane per cell with `CAP2` slots in LDS, one wave per
-/// block and a fixed grid striding over the list ( its length only the device knows ), dealt one cell per wave first; the cells that
-/// outgrow `CAP2` too are listed again for the third pass
+/// the second pass: the cells that outgrew `CAP1`, with `CAP2` slots in LDS, one wave per block and a fixed grid striding over
+/// the list ( its length only the device knows ): whole waves a cell while there is a block for each, one lane per
+/// cell beyond; the cells that outgrow `CAP2` too are listed again for the third pass
 __global__ __launch_bounds__( 64 ) void k_cells_pass2( Params P ) {
     __shared__ double sx[ CAP2 * 64 ], sy[ CAP2 * 64 ];
     __shared__ int sid[ CAP2 * 64 ];
-    const Store<64> c{ sx + threadIdx.x, sy + threadIdx.x, sid + threadIdx.x };
+    Store<64> c{ sx + threadIdx.x, sy + threadIdx.x, sid + threadIdx.x };
     const unsigned count = P.out.counters[ 1 ];
+    Ev ev;
+    if ( count <= gridDim.x ) {
+        if ( blockIdx.x < count ) {
+            const int k = P.out.ovf_list[ blockIdx.x ], nb = wave_cell( P, k, c, ev );
+            if ( nb < 0 && threadIdx.x == 0 ) P.out.ovf_list[ P.n + int( atomicAdd( &P.out.counters[ 4 ], 1u ) ) ] = k;
+            finish_cell( P, k, c, nb, threadIdx.x == 0 && nb >= 0, false );
+            flush_events( P, ev );
+        }
+        return;
+    }
     const unsigned lanes = gridDim.x * 64;
     const unsigned rounds = ( count + lanes - 1 ) / lanes;
-    Ev ev;
     for ( unsigned r = 0; r < rounds; ++r ) {
         const unsigned idx = r * lanes + threadIdx.x * gridDim.x + blockIdx.x;   // consecutive cells to different waves
         const bool live = idx < count;
@@ -875,7 +1165,7 @@ __global__ __launch_bounds__( 64 ) void k_cells_pass2( Params P ) {
 /// the third pass: `CAP3` slots per cell in global memory, `slots` lanes ( the grid ); past that a cell is a failure
 __global__ __launch_bounds__( 64 ) void k_cells_pass3( Params P, double *gx, double *gy, int *gid, unsigned slots ) {
     const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-    const Store<1> c{ gx + size_t( slot ) * CAP3, gy + size_t( slot ) * CAP3, gid + size_t( slot ) * CAP3 };
+    Store<1> c{ gx + size_t( slot ) * CAP3, gy + size_t( slot ) * CAP3, gid + size_t( slot ) * CAP3 };
     const unsigned count = P.out.counters[ 4 ];
     const unsigned rounds = ( count + slots - 1 ) / slots;
     Ev ev;
@@ -935,6 +1225,23 @@ __global__ void k_reset_counters( unsigned *c ) {
     if ( threadIdx.x < 8 ) c[ threadIdx.x ] = 0;
 }
 
+__global__ void k_clear_shards( unsigned long long *shards ) { shards[ threadIdx.x ] = 0; }
+
+unsigned long long *event_shards( hipStream_t st ) {
+    bool fresh = false;
+    unsigned long long *s = arena().get<unsigned long long>( "ev.shards", 8 * EV_SHARDS, &fresh );
+    if ( fresh ) {
+        k_clear_shards<<<1, 8 * EV_SHARDS, 0, st>>>( s );
+        check_launch( "k_clear_shards" );
+    }
+    return s;
+}
+
+void fold_events( unsigned long long *shards, unsigned long long *events, hipStream_t st ) {
+    k_fold_events<<<1, EV_SHARDS, 0, st>>>( shards, events );
+    check_launch( "k_fold_events" );
+}
+
 __global__ void k_fill_u32( I64 n, unsigned *v, unsigned x ) {
     const I64 k = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
     if ( k < n ) v[ k ] = x;
@@ -976,8 +1283,23 @@ void set_domain( Density &dn, int nb, const double *xy ) {
     SDOT_CHECK( area > 0, "domain: the polygon is not counterclockwise" );
 }
 
+namespace {
+/// the first pass's walk over `[ k0, k1 )`, by the cells' count: a group shortens a cell's chain of tests and sets fewer different walks
+/// in one wave, one lane a cell repeats nothing. Measured, FP64 / FP32, uniform Voronoi cells, ms for 16 lanes, 8, one: 2k 0.09 / 0.10, 0.12 / 0.12,
+/// 0.30 / 0.30; 20k 0.17 / 0.16, 0.20 / 0.18, 0.44 / 0.40; 40k 0.29 / 0.25, 0.30 / 0.23, 0.52 / 0.43; 200k 1.22 / 0.98, 1.13 / 0.86, 1.21 / 0.88;
+/// 1M 6.2 / 4.7, 5.4 / 4.0, 4.6 / 3.0. ( Four lanes were never the fastest. )
+template<class T, class ND>
+void launch_walk( const Params &P, const Poly<T> &po, int k0, int k1, hipStream_t st ) {
+    const int m = k1 - k0;
+    if ( m <= WALK_16 )     k_cells_walk<16, 1, T, ND><<<blocks_for( I64( m ) * 16, WALK_BLOCK ), WALK_BLOCK, 0, st>>>( P, po, k0, k1 );
+    else if ( m <= WALK_8 ) k_cells_walk<8, 2, T, ND><<<blocks_for( I64( m ) * 8, WALK_BLOCK ), WALK_BLOCK, 0, st>>>( P, po, k0, k1 );
+    else                    k_cells_walk_lanes<T, ND><<<blocks_for( m, CELL_BLOCK ), CELL_BLOCK, 0, st>>>( P, po, k0, k1 );
+    check_launch( "k_cells_walk" );
+}
+} // namespace
+
 void run_cells( const DevTree &t, const double *lo, const double *hi, const Density &dn, int mode, DiagramOut &out, hipStream_t st, bool fp32,
-                int ovf_slots ) {
+                int ovf_slots, I64 poly_chunk ) {
     SDOT_CHECK( ovf_slots >= 64 && ovf_slots % 64 == 0, "cells: the third pass's lanes are a positive multiple of 64" );
     SDOT_CHECK( ! fp32 || t.nodes32, "cells: the FP32 walk needs the tree's float records" );
     Params P;
@@ -985,30 +1307,44 @@ void run_cells( const DevTree &t, const double *lo, const double *hi, const Dens
     P.wk.nodes32 = t.nodes32;
     P.wk.node_end = t.node_end;
     P.wk.seeds = t.seeds;
+    P.wk.leaf_of = t.leaf_of;
     P.wk.depth = t.depth;
     P.n = int( t.n );
     P.lo[ 0 ] = lo[ 0 ]; P.lo[ 1 ] = lo[ 1 ]; P.hi[ 0 ] = hi[ 0 ]; P.hi[ 1 ] = hi[ 1 ];
     P.dn = dn;
     P.out = out;
     P.mode = mode;
+    Arena &A = arena();
+    P.shards = event_shards( st );
     k_reset_counters<<<1, 64, 0, st>>>( out.counters );
     check_launch( "k_reset_counters" );
     Timing::Pending tp;
     bool timed = timing().begin( TK_CELLS, st, tp );
-    Arena &A = arena();
     if ( fp32 ) {
-        Poly32 po;
-        po.x = A.get<float>( "p32.x", size_t( CAPW ) * size_t( t.n ) );
-        po.y = A.get<float>( "p32.y", size_t( CAPW ) * size_t( t.n ) );
-        po.id = A.get<int>( "p32.id", size_t( CAPW ) * size_t( t.n ) );
+        Poly<float> po;
+        po.x = A.get<float>( "p32.x", size_t( CAP1 ) * size_t( t.n ) );
+        po.y = A.get<float>( "p32.y", size_t( CAP1 ) * size_t( t.n ) );
+        po.id = A.get<int>( "p32.id", size_t( CAP1 ) * size_t( t.n ) );
         po.nb = A.get<int>( "p32.nb", size_t( t.n ) );
-        k_cells_walk32<<<blocks_for( t.n, CELL_BLOCK ), CELL_BLOCK, 0, st>>>( P, po );
-        check_launch( "k_cells_walk32" );
+        po.stride = t.n;
+        launch_walk<float, NodeF>( P, po, 0, P.n, st );
         k_cells_finish32<<<blocks_for( t.n, CELL_BLOCK ), CELL_BLOCK, 0, st>>>( P, po );
         check_launch( "k_cells_finish32" );
     } else {
-        k_cells_pass1<<<blocks_for( t.n, CELL_BLOCK ), CELL_BLOCK, 0, st>>>( P );
-        check_launch( "k_cells_pass1" );
+        // the polygons pass through a buffer of at most `poly_chunk` cells
+        const I64 chunk = std::min<I64>( t.n, poly_chunk );
+        Poly<double> po;
+        po.x = A.get<double>( "p64.x", size_t( CAP1 ) * size_t( chunk ) );
+        po.y = A.get<double>( "p64.y", size_t( CAP1 ) * size_t( chunk ) );
+        po.id = A.get<int>( "p64.id", size_t( CAP1 ) * size_t( chunk ) );
+        po.nb = A.get<int>( "p64.nb", size_t( chunk ) );
+        po.stride = chunk;
+        for ( I64 k0 = 0; k0 < t.n; k0 += chunk ) {
+            const int k1 = int( std::min<I64>( k0 + chunk, t.n ) );
+            launch_walk<double, NodeRec>( P, po, int( k0 ), k1, st );
+            k_cells_finish<<<blocks_for( k1 - k0, CELL_BLOCK ), CELL_BLOCK, 0, st>>>( P, po, int( k0 ), k1 );
+            check_launch( "k_cells_finish" );
+        }
     }
     if ( timed ) timing().end( tp, st );
     timed = timing().begin( TK_CELLS_OVF, st, tp );
@@ -1041,6 +1377,7 @@ void run_cells( const DevTree &t, const double *lo, const double *hi, const Dens
                                                            out.facet_cap, &out.counters[ 7 ] );
         check_launch( "k_sym_rows" );
     }
+    fold_events( P.shards, out.events, st );
     if ( timed ) timing().end( tp, st );
 }
 

@@ -29,7 +29,7 @@ void solve_parts( I64 n, int dim, int density_kind, const double *o, int precisi
     // build's sort keys, sorted lists, segments and flags
     if ( d3 ) parts[ 0 ] = 96 * N + 48 * N + 12 * N + 8 * m + 32 * m + ( 16 + 3 + 3 ) * 8 * N +
                            ( 16 + 8 + 24 + 4 + 1 + 8 ) * m + 1024 * std::ceil( m / RS_TILE_B ) + 24 * half + 8 * N + 48 * N;
-    else      parts[ 0 ] = 64 * N + 32 * N + 32 * N + 12 * N + 8 * m + 32 * m + ( 11 + 2 + 3 ) * 8 * N +
+    else      parts[ 0 ] = 64 * N + 32 * N + 32 * N + 12 * N + 12 * m + 32 * m + ( 11 + 2 + 3 ) * 8 * N +
                            ( 16 + 24 + 4 + 1 + 8 ) * m + 1024 * std::ceil( m / RS_TILE_B ) + 24 * half + 8 * N + 32 * N;
     // two diagram slots: masses, row offsets and counts, diagonals, the rows ( 12 n + 4096 entries, 3D: 44 per seed ), the
     // overflow lists and counters
@@ -39,7 +39,9 @@ void solve_parts( I64 n, int dim, int density_kind, const double *o, int precisi
     const bool limits = ! d3 && o && int( o[ O_STEP ] ) == 1;
     if ( limits ) parts[ 2 ] = 2 * ( EDGE_CAP * 4 * m + 4 * m );
     // the FP32 kernel's polygons ( 2D, 'fp32' and 'mixed' ); 3D with a sum of Gaussians: each cell's polytope
-    if ( ! d3 && precision != 0 ) parts[ 3 ] = CAPW * 12 * m + 4 * m + 8 * m;   // ( and the FP64 redo's marks and list )
+    if ( ! d3 && precision != 0 ) parts[ 3 ] = CAP1 * 12 * m + 4 * m + 8 * m;   // ( and the FP64 redo's marks and list )
+    // the FP64 first pass's polygons ( every 2D solve ends with an FP64 diagram )
+    if ( ! d3 ) parts[ 3 ] += ( CAP1 * 20 + 4 ) * double( std::min<I64>( n, POLY_CHUNK ) );
     if ( d3 && ( density_kind == SDOT_AMD_GAUSSIANS || density_kind == SDOT_AMD_IMAGE ) ) parts[ 3 ] = 64 * m * ( 3 * 8 + 2 * 4 + 3 * 8 + 4 ) + 8 * m;
     // the third pass's vertex slots ( a fixed pool )
     parts[ 4 ] = d3 ? 0 : double( OVF_SLOTS ) * CAP3 * 20;

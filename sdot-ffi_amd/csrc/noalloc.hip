@@ -90,7 +90,7 @@ void measures_2d_noalloc( hipStream_t st, I64 n, const double *positions, const 
         check_launch( "k_fill_f64" );
         set_weights_rank( t, z, st );
     }
-    refresh_majorants( t, st );
+    refresh_majorants( t, st, events != nullptr );
     DiagramOut out;
     out.mass = A.get<double>( "na.mass", size_t( n ) );
     out.counters = A.get<unsigned>( "na.counters", 8 );
@@ -99,7 +99,7 @@ void measures_2d_noalloc( hipStream_t st, I64 n, const double *positions, const 
     k_zero_events<<<1, 64, 0, st>>>( out.events );
     check_launch( "k_zero_events" );
     const double lo[ 2 ] = { box[ 0 ], box[ 1 ] }, hi[ 2 ] = { box[ 2 ], box[ 3 ] };
-    run_cells( t, lo, hi, dn, MODE_MASSES, out, st, false, NOALLOC_OVF_LANES );
+    run_cells( t, lo, hi, dn, MODE_MASSES, out, st, false, NOALLOC_OVF_LANES, NOALLOC_POLY_CHUNK );
     k_rank_to_user<<<nbk, 256, 0, st>>>( n, t.order, out.mass, masses );
     check_launch( "k_rank_to_user" );
     unsigned *cnt = A.host<unsigned>( "na.hcnt", 8 );

@@ -366,7 +366,7 @@ __global__ void k_major_spread( const double4 *seeds, int n, const int *node_end
 
 /// the decision of every node ( `bsp_build_level.h:176-208` ) and its walk record
 __global__ void k_major_final( const double *S, int N, const double *fit, const unsigned long long *rk, const double *box, const int *beg,
-                               const int *end, NodeRec *nodes, NodeF *nodes32 ) {
+                               const int *end, double slack, double reach, NodeRec *nodes, NodeF *nodes32 ) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if ( m >= N ) return;
     NodeRec r;
@@ -386,8 +386,8 @@ __global__ void k_major_final( const double *S, int N, const double *fit, const 
             const double by_chance = sqrt( u > 0 ? u : 0.0 );
             bool well = true;
             const double reach_x = fmax( fabs( r.lo_x ), fabs( r.hi_x ) ), reach_y = fmax( fabs( r.lo_y ), fabs( r.hi_y ) );
-            if ( fabs( fx ) * ( r.hi_x - r.lo_x ) > 8 * spread || fabs( fx ) * reach_x > 100 * spread ) well = false;
-            if ( fabs( fy ) * ( r.hi_y - r.lo_y ) > 8 * spread || fabs( fy ) * reach_y > 100 * spread ) well = false;
+            if ( fabs( fx ) * ( r.hi_x - r.lo_x ) > 8 * spread || fabs( fx ) * reach_x > reach * spread ) well = false;
+            if ( fabs( fy ) * ( r.hi_y - r.lo_y ) > 8 * spread || fabs( fy ) * reach_y > reach * spread ) well = false;
             if ( well && rmax - rmin < 0.85 * by_chance * spread ) {
                 accept = true;
                 bb = rmax;
@@ -395,7 +395,7 @@ __global__ void k_major_final( const double *S, int N, const double *fit, const 
             }
         }
         if ( accept ) { r.wa_x = fx; r.wa_y = fy; }
-        r.wb = bb + 1e-6 * ( fabs( bb ) + spread + amax );
+        r.wb = bb + slack * ( fabs( bb ) + spread + amax );
     }
     nodes[ m ] = r;
     if ( nodes32 ) {
@@ -403,16 +403,19 @@ __global__ void k_major_final( const double *S, int N, const double *fit, const 
         f.lo_x = __double2float_rd( r.lo_x ); f.lo_y = __double2float_rd( r.lo_y );
         f.hi_x = __double2float_ru( r.hi_x ); f.hi_y = __double2float_ru( r.hi_y );
         f.wa_x = float( r.wa_x ); f.wa_y = float( r.wa_y );
-        // `( wa - wa_f ) . y` on the box, bounded by the farthest corner, goes into `wb` before it is rounded up
-        const double ex = fabs( r.wa_x - double( f.wa_x ) ) * fmax( fabs( r.lo_x ), fabs( r.hi_x ) );
-        const double ey = fabs( r.wa_y - double( f.wa_y ) ) * fmax( fabs( r.lo_y ), fabs( r.hi_y ) );
-        f.wb = __double2float_ru( r.wb + ex + ey );
+        // the majorant's value at the box's centre ( as the float walk computes it ), with what the slopes' rounding can change on the box
+        // and the rounding of these sums, then rounded up
+        const double cx = double( 0.5f * ( f.lo_x + f.hi_x ) ), cy = double( 0.5f * ( f.lo_y + f.hi_y ) );
+        const double ex = fabs( r.wa_x - double( f.wa_x ) ) * fmax( fabs( double( f.lo_x ) - cx ), fabs( double( f.hi_x ) - cx ) );
+        const double ey = fabs( r.wa_y - double( f.wa_y ) ) * fmax( fabs( double( f.lo_y ) - cy ), fabs( double( f.hi_y ) - cy ) );
+        const double ax = r.wa_x * cx, ay = r.wa_y * cy;
+        f.wc = __double2float_ru( r.wb + ax + ay + ex + ey + 1e-15 * ( fabs( r.wb ) + fabs( ax ) + fabs( ay ) ) );
         f.beg = r.beg < r.end ? r.beg : -1;
         nodes32[ m ] = f;
     }
 }
 
-void refresh_majorants( DevTree &t, hipStream_t st ) {
+void refresh_majorants( DevTree &t, hipStream_t st, bool reference ) {
     const int N = int( t.nb_nodes ), depth = t.depth;
     Timing::Pending tp;
     const bool timed = timing().begin( TK_MAJORANTS, st, tp );
@@ -431,7 +434,8 @@ void refresh_majorants( DevTree &t, hipStream_t st ) {
     check_launch( "k_major_fit" );
     k_major_spread<<<blocks_for( t.n, 256 ), 256, 0, st>>>( t.seeds, int( t.n ), t.node_end, depth, t.fit, N, t.rkeys );
     check_launch( "k_major_spread" );
-    k_major_final<<<blocks_for( N, 256 ), 256, 0, st>>>( t.stat, N, t.fit, t.rkeys, t.node_box, t.node_beg, t.node_end, t.nodes, t.nodes32 );
+    k_major_final<<<blocks_for( N, 256 ), 256, 0, st>>>( t.stat, N, t.fit, t.rkeys, t.node_box, t.node_beg, t.node_end, reference ? 1e-6 : 1e-12,
+                                                            reference ? 100.0 : 1e7, t.nodes, t.nodes32 );
     check_launch( "k_major_final" );
     if ( timed ) timing().end( tp, st );
 }

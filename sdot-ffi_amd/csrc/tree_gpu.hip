@@ -224,10 +224,11 @@ __global__ void k_children( int count, const int *beg, const int *end, const int
 }
 
 /// the leaves' seeds in ascending user index, and the outputs in rank order
-__global__ void k_leaves( int count, int first, const int *hbeg, const int *hend, int *ids ) {
+__global__ void k_leaves( int count, int first, const int *hbeg, const int *hend, int *ids, int *leaf_of ) {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if ( j >= count ) return;
     const int b = hbeg[ first + j ], e = hend[ first + j ];
+    if ( leaf_of ) for ( int i = b; i < e; ++i ) leaf_of[ i ] = j;
     for ( int i = b + 1; i < e; ++i ) {                   // insertion sort, a handful of seeds
         const int v = ids[ i ];
         int k = i;
@@ -421,7 +422,7 @@ void build_tree_device3( DevTree3 &t, I64 n, const double *pos, int leaf, hipStr
     }
     // 3. leaves, rank tables, preorder
     const int L = depth - 1;
-    k_leaves<<<blocks_for( I64( 1 ) << L, 256 ), 256, 0, st>>>( 1 << L, ( 1 << L ) - 1, hbeg, hend, lst[ 0 ] );
+    k_leaves<<<blocks_for( I64( 1 ) << L, 256 ), 256, 0, st>>>( 1 << L, ( 1 << L ) - 1, hbeg, hend, lst[ 0 ], nullptr );
     k_rank_tables3<<<nbk, 256, 0, st>>>( n, lst[ 0 ], pos, t.order, t.rank_of, t.seeds );
     for ( int l = 0; l < depth; ++l ) k_preorder<<<blocks_for( I64( 1 ) << l, 256 ), 256, 0, st>>>( l, depth, t.lvl_nodes );
     k_to_preorder3<<<blocks_for( N, 256 ), 256, 0, st>>>( N, t.lvl_nodes, hbeg, hend, hbox, t.node_beg, t.node_end, t.node_box );
@@ -445,6 +446,7 @@ void build_tree_device( DevTree &t, I64 n, const double *pos, int leaf, hipStrea
     t.lvl_nodes = A.get<int>( tag + ".lvl_nodes", size_t( N ) );
     t.order = A.get<int>( tag + ".order", size_t( n ) );
     t.rank_of = A.get<int>( tag + ".rank_of", size_t( n ) );
+    t.leaf_of = A.get<int>( tag + ".leaf_of", size_t( n ) );
     t.seeds = A.get<double4>( tag + ".seeds", size_t( n ) );
     t.stat = A.get<double>( tag + ".stat", size_t( N ) * 11 );
     t.fit = A.get<double>( tag + ".fit", size_t( N ) * 2 );
@@ -499,7 +501,7 @@ void build_tree_device( DevTree &t, I64 n, const double *pos, int leaf, hipStrea
     }
     // 3. leaves, rank tables, preorder
     const int L = depth - 1;
-    k_leaves<<<blocks_for( I64( 1 ) << L, 256 ), 256, 0, st>>>( 1 << L, ( 1 << L ) - 1, hbeg, hend, xid );
+    k_leaves<<<blocks_for( I64( 1 ) << L, 256 ), 256, 0, st>>>( 1 << L, ( 1 << L ) - 1, hbeg, hend, xid, t.leaf_of );
     k_rank_tables<<<nbk, 256, 0, st>>>( n, xid, pos, t.order, t.rank_of, t.seeds );
     for ( int l = 0; l < depth; ++l ) k_preorder<<<blocks_for( I64( 1 ) << l, 256 ), 256, 0, st>>>( l, depth, t.lvl_nodes );
     k_to_preorder<<<blocks_for( N, 256 ), 256, 0, st>>>( N, t.lvl_nodes, hbeg, hend, hbox, t.node_beg, t.node_end, t.node_box );
