@@ -23,14 +23,16 @@ double pad( double b ) { return std::ceil( std::max( b, 256.0 ) / 256.0 ) * 256.
 
 void solve_parts( I64 n, int dim, int density_kind, const double *o, int precision, double *parts ) {
     for ( int q = 0; q < SDOT_AMD_NB_MEMORY_PARTS; ++q ) parts[ q ] = 0;
-    const double N = double( ( I64( 1 ) << max_depth_for( n, 10 ) ) - 1 ), half = ( N + 1 ) / 2, m = double( n );
+    const double N = double( ( I64( 1 ) << max_depth_for( n, 10 ) ) - 1 ), m = double( n );
     const bool d3 = dim == 3;
     // the tree: records, boxes, slices, the level table, the permutation, the seeds, the majorants' moments; and its device
     // build's sort keys, sorted lists, segments and flags
-    if ( d3 ) parts[ 0 ] = 96 * N + 48 * N + 12 * N + 8 * m + 32 * m + ( 16 + 3 + 3 ) * 8 * N +
-                           ( 16 + 8 + 24 + 4 + 1 + 8 ) * m + 1024 * std::ceil( m / RS_TILE_B ) + 24 * half + 8 * N + 48 * N;
-    else      parts[ 0 ] = 64 * N + 32 * N + 32 * N + 12 * N + 12 * m + 32 * m + ( 11 + 2 + 3 ) * 8 * N +
-                           ( 16 + 24 + 4 + 1 + 8 ) * m + 1024 * std::ceil( m / RS_TILE_B ) + 24 * half + 8 * N + 32 * N;
+    // ( one workgroup builds a small cloud's tree in LDS: no build buffers )
+    const double d = dim, lists = d3 ? 3 : 1;
+    const double build = n <= 8192 ? 0 : d * ( 16 + 8 ) * m + ( 8 + 1 + 4 * lists ) * m + 1024 * d * std::ceil( m / RS_TILE_B ) + 16 * N + 16 * d * N +
+                                         4 * lists * std::ceil( m / 1024 );
+    if ( d3 ) parts[ 0 ] = 96 * N + 48 * N + 12 * N + 8 * m + 32 * m + ( 16 + 3 + 3 ) * 8 * N + build;
+    else      parts[ 0 ] = 64 * N + 32 * N + 32 * N + 12 * N + 12 * m + 32 * m + ( 11 + 2 + 3 ) * 8 * N + build;
     // two diagram slots: masses, row offsets and counts, diagonals, the rows ( 12 n + 4096 entries, 3D: 44 per seed ), the
     // overflow lists and counters
     const double cap = d3 ? std::ceil( m / 64 ) * 64 * 44 : ( ( o && o[ O_AGG_NB_DUPS ] > 0 ) ? 14 : 12 ) * m + 4096;

@@ -263,10 +263,7 @@ __global__ void k_major_leaves( const int *lvl_nodes, int first, int count, cons
 }
 
 /// one level up: a node's moments from its two children ( Chan et al.'s pairwise combination )
-__global__ void k_major_up( const int *lvl_nodes, int first, int count, int h, double *S, int N ) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if ( j >= count ) return;
-    const int node = lvl_nodes[ first + j ];
+__device__ __forceinline__ void merge_up( int node, int h, double *S, int N ) {
     const int lc = node + 1, rc = node + ( 1 << ( h - 1 ) );
     const Stat a = load_stat( S, N, lc ), b = load_stat( S, N, rc );
     Stat s;
@@ -288,6 +285,22 @@ __global__ void k_major_up( const int *lvl_nodes, int first, int count, int h, d
         s.wmax = fmax( a.wmax, b.wmax );
     }
     store_stat( S, N, node, s );
+}
+
+__global__ void k_major_up( const int *lvl_nodes, int first, int count, int h, double *S, int N ) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if ( j < count ) merge_up( lvl_nodes[ first + j ], h, S, N );
+}
+
+/// the levels `L` to the root, at most 256 nodes each, by one workgroup: a launch a level took ~4 us and as much again to start. ( 512 and
+/// 1024 nodes are more than a CU's share: 59 us for the eleven levels of 1M seeds, 20 for these nine )
+constexpr int TOP_LEVEL = 8;
+__global__ __launch_bounds__( 1 << TOP_LEVEL ) void k_major_top( const int *lvl_nodes, int L, int depth, double *S, int N ) {
+    for ( ; L >= 0; --L ) {
+        const int j = threadIdx.x;
+        if ( j < 1 << L ) merge_up( lvl_nodes[ ( 1 << L ) - 1 + j ], depth - L, S, N );
+        __syncthreads();                                 // ( one workgroup: its stores are seen by its own later loads )
+    }
 }
 
 /// the least-squares slope of every node ( Gauss with partial pivoting on the centred normal
@@ -425,10 +438,14 @@ void refresh_majorants( DevTree &t, hipStream_t st, bool reference ) {
         k_major_leaves<<<blocks_for( count, 256 ), 256, 0, st>>>( t.lvl_nodes, first, count, t.node_beg, t.node_end, t.seeds, t.stat, N );
         check_launch( "k_major_leaves" );
     }
-    for ( int L = depth - 2; L >= 0; --L ) {
+    for ( int L = depth - 2; L > TOP_LEVEL; --L ) {
         const int first = ( 1 << L ) - 1, count = 1 << L, h = depth - L;
         k_major_up<<<blocks_for( count, 256 ), 256, 0, st>>>( t.lvl_nodes, first, count, h, t.stat, N );
         check_launch( "k_major_up" );
+    }
+    if ( depth >= 2 ) {
+        k_major_top<<<1, 1 << TOP_LEVEL, 0, st>>>( t.lvl_nodes, std::min( depth - 2, TOP_LEVEL ), depth, t.stat, N );
+        check_launch( "k_major_top" );
     }
     k_major_fit<<<blocks_for( N, 256 ), 256, 0, st>>>( t.stat, N, t.fit, t.rkeys );
     check_launch( "k_major_fit" );

@@ -72,10 +72,7 @@ __global__ void k_major3_leaves( const int *lvl_nodes, int first, int count, con
     store3( S, N, node, s );
 }
 
-__global__ void k_major3_up( const int *lvl_nodes, int first, int count, int h, double *S, int N ) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if ( j >= count ) return;
-    const int node = lvl_nodes[ first + j ];
+__device__ __forceinline__ void merge_up3( int node, int h, double *S, int N ) {
     const int lc = node + 1, rc = node + ( 1 << ( h - 1 ) );
     const Stat3 a = load3( S, N, lc ), b = load3( S, N, rc );
     Stat3 s;
@@ -103,6 +100,22 @@ __global__ void k_major3_up( const int *lvl_nodes, int first, int count, int h, 
         s.v[ T_WMAX ] = fmax( a.v[ T_WMAX ], b.v[ T_WMAX ] );
     }
     store3( S, N, node, s );
+}
+
+__global__ void k_major3_up( const int *lvl_nodes, int first, int count, int h, double *S, int N ) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if ( j < count ) merge_up3( lvl_nodes[ first + j ], h, S, N );
+}
+
+/// the levels `L` to the root, at most 256 nodes each, by one workgroup: a launch a level took ~4 us and as much again to start. ( 512 and
+/// 1024 nodes are more than a CU's share: 59 us for the eleven levels of 1M seeds, 20 for these nine )
+constexpr int TOP_LEVEL = 8;
+__global__ __launch_bounds__( 1 << TOP_LEVEL ) void k_major3_top( const int *lvl_nodes, int L, int depth, double *S, int N ) {
+    for ( ; L >= 0; --L ) {
+        const int j = threadIdx.x;
+        if ( j < 1 << L ) merge_up3( lvl_nodes[ ( 1 << L ) - 1 + j ], depth - L, S, N );
+        __syncthreads();                                 // ( one workgroup: its stores are seen by its own later loads )
+    }
 }
 
 /// rows `i` and `j` of the 3 x 4 system swapped when `|A[ j ][ c ]| > |A[ i ][ c ]|` ( fixed indices: no scratch )
@@ -259,10 +272,14 @@ void refresh_majorants3( DevTree3 &t, hipStream_t st ) {
         k_major3_leaves<<<blocks_for( count, 256 ), 256, 0, st>>>( t.lvl_nodes, first, count, t.node_beg, t.node_end, t.seeds, t.stat, N );
         check_launch( "k_major3_leaves" );
     }
-    for ( int L = depth - 2; L >= 0; --L ) {
+    for ( int L = depth - 2; L > TOP_LEVEL; --L ) {
         const int first = ( 1 << L ) - 1, count = 1 << L, h = depth - L;
         k_major3_up<<<blocks_for( count, 256 ), 256, 0, st>>>( t.lvl_nodes, first, count, h, t.stat, N );
         check_launch( "k_major3_up" );
+    }
+    if ( depth >= 2 ) {
+        k_major3_top<<<1, 1 << TOP_LEVEL, 0, st>>>( t.lvl_nodes, std::min( depth - 2, TOP_LEVEL ), depth, t.stat, N );
+        check_launch( "k_major3_top" );
     }
     k_major3_fit<<<blocks_for( N, 256 ), 256, 0, st>>>( t.stat, N, t.fit, t.rkeys );
     check_launch( "k_major3_fit" );

@@ -3,16 +3,17 @@
 // user index ).
 //
 // How ( this build's own scheme; the reference's card builder is `gpu/Bsp2D.cuh:367` ):
-//   1. two stable LSD radix sorts of the seeds, by x and by y ( 64-bit order-preserving keys of the
-//      doubles, 8 passes of 8 bits; the in-tile rank of an element among its digit's is found with
-//      wave64 ballots, so a pass is histogram / scan / scatter );
-//   2. per level, every node's slice is a contiguous segment of BOTH sorted lists, so its box is read
-//      off the segment's ends ( first and last of the x list, of the y list ); the median cut on the
-//      longest axis takes the first half of that axis' list as is, and the other list is stably
-//      partitioned by the flags the cut writes ( an exclusive scan over all positions ) -- both lists
-//      stay sorted inside every child;
+//   1. a stable LSD radix sort of the seeds along each axis, the axes in the same launches ( 64-bit order-preserving keys of the
+//      doubles, 8 passes of 8 bits; the in-tile rank of an element among its digit's is found with wave64 ballots; a pass is
+//      histogram / scan of each digit's tiles / scatter );
+//   2. per level, every node's slice is a contiguous segment of EVERY sorted list, so its box is read off the segments' ends; the
+//      median cut on the longest axis takes the first half of that axis' list as is, and the other lists are stably partitioned by
+//      the flags the cut writes ( an exclusive scan over all positions ): the lists stay sorted inside every child. Five launches a
+//      level: the nodes, the flags, the scan in two, the partition, which also hands each position its child;
 //   3. the leaves' seeds sorted by user index, the preorder numbering and the rank tables.
-// Everything stays on the device; the host only issues launches ( their count is a function of `n` ).
+// Everything stays on the device; the host only issues launches ( their count is a function of `n` ) and waits for none of them.
+// A cloud of at most `SMALL_TREE` seeds is built by ONE workgroup with its lists in LDS ( `k_small_tree` ): its ~100 launches
+// took ~0.4 ms, whatever they did ( the line is what LDS holds: 64 KiB of keys, the lists and their partitions ).
 
 #include "tree.h"
 #include "tree3.h"
@@ -30,56 +31,80 @@ __device__ __forceinline__ unsigned long long dkey( double x ) {
     return ( u >> 63 ) ? ~u : ( u | 0x8000000000000000ull );
 }
 
-/// the keys of one axis ( `dim` coordinates a seed ), and the identity permutation
-__global__ void k_keys( I64 n, const double *pos, int dim, int axis, unsigned long long *key, int *val ) {
+/// the keys of every axis ( `dim` coordinates a seed; the grid's second index ), and the identity permutation
+__global__ void k_keys( I64 n, const double *pos, int dim, unsigned long long *key, int *val ) {
     const I64 i = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
     if ( i >= n ) return;
-    key[ i ] = dkey( pos[ dim * i + axis ] );
-    val[ i ] = int( i );
+    const int axis = blockIdx.y;
+    key[ axis * n + i ] = dkey( pos[ dim * i + axis ] );
+    val[ axis * n + i ] = int( i );
 }
 
-/// histogram of digit `shift` per tile: `hist[ digit * nt + tile ]`
-__global__ __launch_bounds__( RS_THREADS ) void k_rs_hist( I64 n, const unsigned long long *key, int shift, int nt, unsigned *hist ) {
+/// histogram of digit `shift` per tile: `hist[ ( axis 256 + digit ) nt + tile ]`
+__global__ __launch_bounds__( RS_THREADS ) void k_rs_hist( I64 n, const unsigned long long *keys, int shift, int nt, unsigned *hist ) {
     __shared__ unsigned h[ 256 ];
     h[ threadIdx.x ] = 0;
     __syncthreads();
+    const unsigned long long *key = keys + blockIdx.y * n;
     const I64 base = I64( blockIdx.x ) * RS_TILE;
     for ( int j = 0; j < RS_ITEMS; ++j ) {
         const I64 i = base + j * RS_THREADS + threadIdx.x;
         if ( i < n ) atomicAdd( &h[ ( key[ i ] >> shift ) & 255 ], 1u );
     }
     __syncthreads();
-    hist[ size_t( threadIdx.x ) * nt + blockIdx.x ] = h[ threadIdx.x ];
+    hist[ ( size_t( blockIdx.y ) * 256 + threadIdx.x ) * nt + blockIdx.x ] = h[ threadIdx.x ];
 }
 
-/// exclusive scan of `m` counts in one block ( digit-major: the offsets of each tile's digit run )
-__global__ __launch_bounds__( 1024 ) void k_scan_single( unsigned *v, int m ) {
-    __shared__ unsigned part[ 1024 ];
-    const int per = ( m + 1023 ) / 1024;
-    const int b = threadIdx.x * per, e = min( m, b + per );
-    unsigned s = 0;
-    for ( int i = b; i < e; ++i ) s += v[ i ];
-    part[ threadIdx.x ] = s;
+__device__ __forceinline__ unsigned wave_inclusive( unsigned v ) {
+    const int lane = threadIdx.x & 63;
+    for ( int o = 1; o < 64; o <<= 1 ) { const unsigned t = __shfl_up( v, o, 64 ); if ( lane >= o ) v += t; }
+    return v;
+}
+/// the exclusive prefix of `v` over the block's `T` threads, and the block's total ( `sh`: one word a wave )
+template<int T>
+__device__ __forceinline__ unsigned block_exclusive( unsigned v, unsigned *sh, unsigned &total ) {
+    const unsigned inc = wave_inclusive( v );
     __syncthreads();
-    for ( int off = 1; off < 1024; off <<= 1 ) {
-        const unsigned t = threadIdx.x >= unsigned( off ) ? part[ threadIdx.x - off ] : 0u;
-        __syncthreads();
-        part[ threadIdx.x ] += t;
-        __syncthreads();
+    if ( ( threadIdx.x & 63 ) == 63 ) sh[ threadIdx.x >> 6 ] = inc;
+    __syncthreads();
+    unsigned before = 0;
+    total = 0;
+    for ( int w = 0; w < T / 64; ++w ) { const unsigned x = sh[ w ]; before += w < int( threadIdx.x >> 6 ) ? x : 0; total += x; }
+    return before + inc - v;
+}
+
+/// the tiles' counts of one digit made offsets, its total kept ( one block a digit and axis; one block over all counts of 1M keys took
+/// 118 us a pass )
+__global__ __launch_bounds__( RS_THREADS ) void k_rs_scan( int nt, unsigned *hist, unsigned *total ) {
+    __shared__ unsigned sh[ RS_THREADS / 64 ];
+    unsigned *v = hist + ( size_t( blockIdx.y ) * 256 + blockIdx.x ) * nt;
+    unsigned carry = 0;
+    for ( int b = 0; b < nt; b += RS_THREADS ) {
+        const int i = b + int( threadIdx.x );
+        const unsigned x = i < nt ? v[ i ] : 0u;
+        unsigned t;
+        const unsigned e = block_exclusive<RS_THREADS>( x, sh, t );
+        if ( i < nt ) v[ i ] = carry + e;
+        carry += t;
     }
-    unsigned acc = threadIdx.x ? part[ threadIdx.x - 1 ] : 0u;
-    for ( int i = b; i < e; ++i ) { const unsigned x = v[ i ]; v[ i ] = acc; acc += x; }
+    if ( threadIdx.x == 0 ) total[ blockIdx.y * 256 + blockIdx.x ] = carry;
 }
 
 /// the stable scatter of one pass: a tile is read in rounds of 256 elements in order; inside a round the
 /// rank of an element among the same digit comes from wave ballots ( 8 bits -> the mask of its peers )
 /// plus the counts of the waves before it and of the earlier rounds
-__global__ __launch_bounds__( RS_THREADS ) void k_rs_scatter( I64 n, const unsigned long long *key, const int *val, int shift, int nt,
-                                                            const unsigned *offs, unsigned long long *key_out, int *val_out ) {
-    __shared__ unsigned running[ 256 ];
+__global__ __launch_bounds__( RS_THREADS ) void k_rs_scatter( I64 n, const unsigned long long *keys, const int *vals, int shift, int nt,
+                                                            const unsigned *offs, const unsigned *total, unsigned long long *keys_out, int *vals_out ) {
+    __shared__ unsigned running[ 256 ], sh[ RS_THREADS / 64 ];
     __shared__ unsigned wcount[ RS_THREADS / 64 ][ 256 ];
+    const unsigned long long *key = keys + blockIdx.y * n;
+    const int *val = vals + blockIdx.y * n;
+    unsigned long long *key_out = keys_out + blockIdx.y * n;
+    int *val_out = vals_out + blockIdx.y * n;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    running[ threadIdx.x ] = offs[ size_t( threadIdx.x ) * nt + blockIdx.x ];
+    unsigned all;
+    const unsigned first = block_exclusive<RS_THREADS>( total[ blockIdx.y * 256 + threadIdx.x ], sh, all );
+    running[ threadIdx.x ] = first + offs[ ( size_t( blockIdx.y ) * 256 + threadIdx.x ) * nt + blockIdx.x ];
     const I64 base = I64( blockIdx.x ) * RS_TILE;
     const unsigned long long lt = lane ? ( ~0ull >> ( 64 - lane ) ) : 0ull;
     for ( int j = 0; j < RS_ITEMS; ++j ) {
@@ -111,116 +136,125 @@ __global__ __launch_bounds__( RS_THREADS ) void k_rs_scatter( I64 n, const unsig
     }
 }
 
-struct Sorted { unsigned long long *key; int *val; };
-
-/// the stable sort of `n` ( key, id ) pairs by key; returns the buffers holding the result
-Sorted radix_sort( I64 n, unsigned long long *k0, int *v0, unsigned long long *k1, int *v1, unsigned *hist, hipStream_t st ) {
+/// the stable sorts of `axes` lists of `n` ( key, id ) pairs by key ( eight passes: the result is back in `k0`, `v0` )
+void radix_sort( I64 n, int axes, unsigned long long *k0, int *v0, unsigned long long *k1, int *v1, unsigned *hist, unsigned *total, hipStream_t st ) {
     const int nt = int( ( n + RS_TILE - 1 ) / RS_TILE );
     for ( int pass = 0; pass < 8; ++pass ) {
         const int shift = 8 * pass;
-        k_rs_hist<<<nt, RS_THREADS, 0, st>>>( n, k0, shift, nt, hist );
-        k_scan_single<<<1, 1024, 0, st>>>( hist, 256 * nt );
-        k_rs_scatter<<<nt, RS_THREADS, 0, st>>>( n, k0, v0, shift, nt, hist, k1, v1 );
+        k_rs_hist<<<dim3( nt, axes ), RS_THREADS, 0, st>>>( n, k0, shift, nt, hist );
+        k_rs_scan<<<dim3( 256, axes ), RS_THREADS, 0, st>>>( nt, hist, total );
+        k_rs_scatter<<<dim3( nt, axes ), RS_THREADS, 0, st>>>( n, k0, v0, shift, nt, hist, total, k1, v1 );
         std::swap( k0, k1 );
         std::swap( v0, v1 );
     }
     check_launch( "radix_sort" );
-    return Sorted{ k0, v0 };
 }
 
 // ---- the levels ------------------------------------------------------------------------------------------
 
-/// one node of level `L` ( heap index `first + j` ): its slice, box and cut
-__global__ void k_level_nodes( int count, int first, const int *beg, const int *end, const double *pos, const int *xid, const int *yid, int leaf,
-                               double *hbox, int *axis, int *mid, int *hbeg, int *hend ) {
+// ( every array over the lists holds `n` entries an axis )
+
+/// the slice of node `j` of level `L`, from its parent's slice and cut
+__device__ __forceinline__ void slice_of( int L, int j, I64 n, const int *hbeg, const int *hend, const int *hmid, int &b, int &e ) {
+    b = 0;
+    e = int( n );
+    if ( L == 0 ) return;
+    const int p = ( 1 << ( L - 1 ) ) - 1 + j / 2;
+    b = j & 1 ? hmid[ p ] : hbeg[ p ];
+    e = j & 1 ? hend[ p ] : hmid[ p ];
+}
+
+/// a node's box ( the ends of its segments of the lists ), the axis it is cut along ( the first longest ) and where ( its end: not cut )
+template<int D, class ID>
+__device__ __forceinline__ void node_cut( int b, int e, const double *pos, const ID *ids, I64 stride, int leaf, double *lo, double *hi, int &axis,
+                                          int &mid ) {
+    axis = 0;
+    mid = e;
+    for ( int d = 0; d < D; ++d ) lo[ d ] = hi[ d ] = 0;
+    if ( e <= b ) return;
+    for ( int d = 0; d < D; ++d ) {
+        lo[ d ] = pos[ D * size_t( ids[ d * stride + b ] ) + d ];
+        hi[ d ] = pos[ D * size_t( ids[ d * stride + e - 1 ] ) + d ];
+    }
+    for ( int d = 1; d < D; ++d ) if ( hi[ d ] - lo[ d ] > hi[ axis ] - lo[ axis ] ) axis = d;
+    if ( e - b > leaf && hi[ axis ] > lo[ axis ] ) mid = b + ( e - b ) / 2;
+}
+
+/// the nodes of level `L`, in heap order
+template<int D>
+__global__ void k_level_nodes( int L, I64 n, const double *pos, const int *ids, int leaf, double *hbox, int *haxis, int *hmid, int *hbeg, int *hend ) {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if ( j >= count ) return;
-    const int b = beg[ j ], e = end[ j ], node = first + j;
+    if ( j >= 1 << L ) return;
+    const int node = ( 1 << L ) - 1 + j;
+    int b, e, axis, mid;
+    slice_of( L, j, n, hbeg, hend, hmid, b, e );
+    double lo[ D ], hi[ D ];
+    node_cut<D>( b, e, pos, ids, n, leaf, lo, hi, axis, mid );
+    for ( int d = 0; d < D; ++d ) { hbox[ 2 * D * size_t( node ) + d ] = lo[ d ]; hbox[ 2 * D * size_t( node ) + D + d ] = hi[ d ]; }
     hbeg[ node ] = b;
     hend[ node ] = e;
-    double *bx = hbox + 4 * size_t( node );
-    if ( e <= b ) {
-        bx[ 0 ] = bx[ 1 ] = bx[ 2 ] = bx[ 3 ] = 0;
-        axis[ j ] = 0;
-        mid[ j ] = e;
-        return;
+    haxis[ node ] = axis;
+    hmid[ node ] = mid;
+}
+
+/// the side of every seed from its node's cut list: `flag[ id ] = position < mid`
+__global__ void k_flags( I64 n, int L, const int *seg, const int *haxis, const int *hmid, const int *ids, unsigned char *flag ) {
+    const I64 p = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
+    if ( p >= n ) return;
+    const int node = ( 1 << L ) - 1 + ( L ? seg[ p ] : 0 );
+    flag[ ids[ haxis[ node ] * n + p ] ] = p < hmid[ node ];
+}
+
+/// the lists a level partitions: in 2D the one that is not cut, position by position ( one scan ); in 3D all three, the cut one's partition
+/// being the identity
+template<int D>
+__device__ __forceinline__ I64 list_at( I64 n, I64 p, int axis ) { return D == 2 ? ( 1 - axis ) * n + p : blockIdx.y * n + p; }
+
+/// the exclusive scan of the left flags in the lists' order: inside each 1024 positions, and their sums
+template<int D>
+__global__ __launch_bounds__( 1024 ) void k_scan_blocks( I64 n, int L, const int *seg, const int *haxis, const int *ids, const unsigned char *flag,
+                                                       unsigned *s, unsigned *bsum ) {
+    __shared__ unsigned sh[ 16 ];
+    const I64 p = I64( blockIdx.x ) * 1024 + threadIdx.x;
+    unsigned v = 0;
+    if ( p < n ) v = flag[ ids[ list_at<D>( n, p, D == 2 ? haxis[ ( 1 << L ) - 1 + ( L ? seg[ p ] : 0 ) ] : 0 ) ] ];
+    unsigned total;
+    const unsigned e = block_exclusive<1024>( v, sh, total );
+    if ( p < n ) s[ blockIdx.y * n + p ] = e;
+    if ( threadIdx.x == 0 ) bsum[ blockIdx.y * gridDim.x + blockIdx.x ] = total;
+}
+
+/// the blocks' sums scanned, one block a list
+__global__ __launch_bounds__( 1024 ) void k_scan_sums( int m, unsigned *bsum ) {
+    __shared__ unsigned sh[ 16 ];
+    unsigned *v = bsum + size_t( blockIdx.x ) * m, carry = 0;
+    for ( int b = 0; b < m; b += 1024 ) {
+        const int i = b + int( threadIdx.x );
+        const unsigned x = i < m ? v[ i ] : 0u;
+        unsigned t;
+        const unsigned e = block_exclusive<1024>( x, sh, t );
+        if ( i < m ) v[ i ] = carry + e;
+        carry += t;
     }
-    const double lox = pos[ 2 * size_t( xid[ b ] ) ], hix = pos[ 2 * size_t( xid[ e - 1 ] ) ];
-    const double loy = pos[ 2 * size_t( yid[ b ] ) + 1 ], hiy = pos[ 2 * size_t( yid[ e - 1 ] ) + 1 ];
-    bx[ 0 ] = lox; bx[ 1 ] = loy; bx[ 2 ] = hix; bx[ 3 ] = hiy;
-    const int ax = ( hiy - loy > hix - lox ) ? 1 : 0;
-    axis[ j ] = ax;
-    const double lo = ax ? loy : lox, hi = ax ? hiy : hix;
-    mid[ j ] = ( e - b > leaf && hi > lo ) ? b + ( e - b ) / 2 : e;
 }
 
-/// which node of the level each position belongs to: `seg[ p ]`, from the slices
-__global__ void k_fill_seg( int count, const int *beg, const int *end, int *seg ) {
-    const int j = blockIdx.x;
-    const int b = beg[ j ], e = end[ j ];
-    for ( int p = b + threadIdx.x; p < e; p += blockDim.x ) seg[ p ] = j;
-}
-
-/// the side of every seed: from the cut axis' list, `flag[ id ] = position < mid`
-__global__ void k_flags( I64 n, const int *seg, const int *axis, const int *mid, const int *xid, const int *yid, unsigned char *flag ) {
+/// the stable partition of the lists inside every segment, and the next level's node of every position
+template<int D>
+__global__ void k_partition( I64 n, int L, const int *seg, const int *haxis, const int *hbeg, const int *hmid, const int *ids,
+                             const unsigned char *flag, const unsigned *s, const unsigned *bsum, int nsb, int *out, int *seg_out ) {
     const I64 p = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
     if ( p >= n ) return;
-    const int j = seg[ p ];
-    const int id = axis[ j ] ? yid[ p ] : xid[ p ];
-    flag[ id ] = p < mid[ j ];
-}
-
-/// the left flags of the OTHER list, in its order ( what the scan counts )
-__global__ void k_other_flags( I64 n, const int *seg, const int *axis, const int *xid, const int *yid, const unsigned char *flag, unsigned *f ) {
-    const I64 p = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
-    if ( p >= n ) return;
-    const int j = seg[ p ];
-    const int id = axis[ j ] ? xid[ p ] : yid[ p ];
-    f[ p ] = flag[ id ];
-}
-
-/// block sums, then their scan, then the scan of each block: an exclusive scan of `f` in `s`
-__global__ __launch_bounds__( 1024 ) void k_scan_blocks( I64 n, const unsigned *f, unsigned *s, unsigned *bsum ) {
-    __shared__ unsigned sh[ 1024 ];
-    const I64 i = I64( blockIdx.x ) * 1024 + threadIdx.x;
-    const unsigned v = i < n ? f[ i ] : 0u;
-    sh[ threadIdx.x ] = v;
-    __syncthreads();
-    for ( int off = 1; off < 1024; off <<= 1 ) {
-        const unsigned t = threadIdx.x >= unsigned( off ) ? sh[ threadIdx.x - off ] : 0u;
-        __syncthreads();
-        sh[ threadIdx.x ] += t;
-        __syncthreads();
-    }
-    if ( i < n ) s[ i ] = sh[ threadIdx.x ] - v;
-    if ( threadIdx.x == 1023 ) bsum[ blockIdx.x ] = sh[ 1023 ];
-}
-
-__global__ void k_scan_add( I64 n, unsigned *s, const unsigned *bsum ) {
-    const I64 i = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
-    if ( i < n ) s[ i ] += bsum[ i / 1024 ];
-}
-
-/// the stable partition of the other list inside every segment; the cut axis' list is already split
-__global__ void k_partition( I64 n, const int *seg, const int *axis, const int *beg, const int *mid, const int *xid, const int *yid,
-                             const unsigned char *flag, const unsigned *s, int *xo, int *yo ) {
-    const I64 p = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
-    if ( p >= n ) return;
-    const int j = seg[ p ];
-    const int ax = axis[ j ], b = beg[ j ], m = mid[ j ];
-    const int id = ax ? xid[ p ] : yid[ p ];
-    const unsigned left_before = s[ p ] - s[ b ];
-    const int q = flag[ id ] ? b + int( left_before ) : m + int( ( p - b ) - left_before );
-    if ( ax ) { yo[ p ] = yid[ p ]; xo[ q ] = id; }
-    else      { xo[ p ] = xid[ p ]; yo[ q ] = id; }
-}
-
-/// the next level's slices: `[ b, mid )` and `[ mid, e )`
-__global__ void k_children( int count, const int *beg, const int *end, const int *mid, int *nb, int *ne ) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if ( j >= count ) return;
-    nb[ 2 * j ] = beg[ j ]; ne[ 2 * j ] = mid[ j ];
-    nb[ 2 * j + 1 ] = mid[ j ]; ne[ 2 * j + 1 ] = end[ j ];
+    const int j = L ? seg[ p ] : 0, node = ( 1 << L ) - 1 + j;
+    const int b = hbeg[ node ], m = hmid[ node ], axis = haxis[ node ];
+    const unsigned *sl = s + blockIdx.y * n, *bl = bsum + size_t( blockIdx.y ) * nsb;
+    const I64 from = list_at<D>( n, p, axis );
+    const int id = ids[ from ];
+    const bool left = flag[ id ];
+    const unsigned before = ( sl[ p ] + bl[ p / 1024 ] ) - ( sl[ b ] + bl[ b / 1024 ] );
+    const int q = left ? b + int( before ) : m + int( ( p - b ) - before );
+    out[ from - p + q ] = id;
+    if ( D == 2 ) out[ axis * n + p ] = ids[ axis * n + p ];
+    if ( blockIdx.y == 0 ) seg_out[ p ] = 2 * j + ( p >= m );
 }
 
 /// the leaves' seeds in ascending user index, and the outputs in rank order
@@ -237,114 +271,198 @@ __global__ void k_leaves( int count, int first, const int *hbeg, const int *hend
     }
 }
 
+template<int D>
+__device__ __forceinline__ double4 seed_of( const double *pos, int u ) {
+    if ( D == 2 ) return make_double4( pos[ 2 * size_t( u ) ], pos[ 2 * size_t( u ) + 1 ], 0.0, 0.0 );
+    return make_double4( pos[ 3 * size_t( u ) ], pos[ 3 * size_t( u ) + 1 ], pos[ 3 * size_t( u ) + 2 ], 0.0 );
+}
+
+template<int D>
 __global__ void k_rank_tables( I64 n, const int *ids, const double *pos, int *order, int *rank_of, double4 *seeds ) {
     const I64 k = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
     if ( k >= n ) return;
     const int u = ids[ k ];
     order[ k ] = u;
     rank_of[ u ] = int( k );
-    seeds[ k ] = make_double4( pos[ 2 * size_t( u ) ], pos[ 2 * size_t( u ) + 1 ], 0.0, 0.0 );
+    seeds[ k ] = seed_of<D>( pos, u );
 }
 
-/// heap -> preorder for every node: `pre[ h ]`, computed level by level
-__global__ void k_preorder( int L, int depth, int *pre ) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if ( j >= ( 1 << L ) ) return;
-    // the path from the root: bit ( L - 1 - t ) of `j` is the side taken at level t
-    int p = 0;
-    for ( int t = 0; t < L; ++t ) {
-        const int hgt = depth - t;
-        p += ( ( j >> ( L - 1 - t ) ) & 1 ) ? ( 1 << ( hgt - 1 ) ) : 1;
-    }
-    pre[ ( 1 << L ) - 1 + j ] = p;
-}
+/// the preorder index of node `j` of level `L` in a tree `depth` high: a left child is 1 after its parent, a right one `2^( height - 1 )`
+__device__ __forceinline__ int preorder_of( int j, int L, int depth ) { return 2 * ( j << ( depth - 1 - L ) ) + L - __popc( unsigned( j ) ); }
 
-__global__ void k_to_preorder( I64 N, const int *pre, const int *hbeg, const int *hend, const double *hbox, int *beg, int *end, double *box ) {
+/// the tree's arrays from the heap's, in preorder, and the nodes level by level
+__global__ void k_to_preorder( I64 N, int depth, int box, const int *hbeg, const int *hend, const double *hbox, int *beg, int *end, double *out,
+                               int *lvl_nodes ) {
     const I64 h = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
     if ( h >= N ) return;
-    const int p = pre[ h ];
+    const int L = 31 - __clz( int( h ) + 1 ), p = preorder_of( int( h ) + 1 - ( 1 << L ), L, depth );
+    lvl_nodes[ h ] = p;
     beg[ p ] = hbeg[ h ];
     end[ p ] = hend[ h ];
-    for ( int c = 0; c < 4; ++c ) box[ 4 * size_t( p ) + c ] = hbox[ 4 * size_t( h ) + c ];
+    for ( int c = 0; c < box; ++c ) out[ box * size_t( p ) + c ] = hbox[ box * size_t( h ) + c ];
 }
 
-// ---- 3D: the same scheme with three sorted lists ----------------------------------------------------------------------
-//
-// Every node's slice is a contiguous segment of each of the three lists. The cut list ( the longest axis' ) decides each
-// seed's side; then EVERY list is stably partitioned by those sides ( for the cut list itself the partition is the identity:
-// its first half is the left child ), one exclusive scan per list.
+// ---- a small cloud's tree by one workgroup ----------------------------------------------------------------------------
 
-struct Lists3 { const int *id[ 3 ]; };
+constexpr int SMALL_TREE = 8192, SMALL_T = 1024, SMALL_NODES = 1024;
 
-/// one node of level `L` in 3D: its slice, box ( the ends of the three lists' segments ) and cut
-__global__ void k_level_nodes3( int count, int first, const int *beg, const int *end, const double *pos, Lists3 L, int leaf, double *hbox,
-                                int *axis, int *mid, int *hbeg, int *hend ) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if ( j >= count ) return;
-    const int b = beg[ j ], e = end[ j ], node = first + j;
-    hbeg[ node ] = b;
-    hend[ node ] = e;
-    double *bx = hbox + 6 * size_t( node );
-    if ( e <= b ) {
-        for ( int c = 0; c < 6; ++c ) bx[ c ] = 0;
-        axis[ j ] = 0;
-        mid[ j ] = e;
+struct SmallOut {
+    int *beg, *end, *lvl_nodes, *order, *rank_of, *leaf_of;
+    double *box;
+    double4 *seeds;
+};
+
+/// THE SAME TREE in one launch: each axis sorted by a bitonic network over ( key, user index ), the lists and their partitions in LDS,
+/// the levels separated by barriers, each thread eight consecutive positions of a scan. It is bound by its barriers and LDS: 2k seeds 114
+/// us, which made a call that measures 2k cells 0.79 -> 0.44 ms
+template<int D>
+__global__ __launch_bounds__( SMALL_T ) void k_small_tree( int n, const double *pos, int leaf, int depth, SmallOut out ) {
+    typedef unsigned short u16;
+    __shared__ unsigned long long keys[ SMALL_TREE ];
+    __shared__ u16 lists[ D ][ SMALL_TREE ];
+    __shared__ u16 nbeg[ SMALL_NODES ], nend[ SMALL_NODES ], nmid[ SMALL_NODES ], npre[ SMALL_NODES ], pbeg[ SMALL_NODES / 2 ], pend[ SMALL_NODES / 2 ],
+        pmid[ SMALL_NODES / 2 ];
+    __shared__ unsigned char naxis[ SMALL_NODES ];
+    __shared__ unsigned sh[ SMALL_T / 64 ];
+    const int tid = threadIdx.x;
+    int n2 = 2;
+    while ( n2 < n ) n2 *= 2;
+    for ( int d = 0; d < D; ++d ) {
+        u16 *id = lists[ d ];
+        for ( int i = tid; i < n2; i += SMALL_T ) { keys[ i ] = i < n ? dkey( pos[ D * i + d ] ) : ~0ull; id[ i ] = u16( i ); }
+        __syncthreads();
+        for ( int k = 2; k <= n2; k *= 2 )
+            for ( int j = k / 2; j > 0; j /= 2 ) {
+                for ( int t = tid; t < n2 / 2; t += SMALL_T ) {
+                    const int a = 2 * t - ( t & ( j - 1 ) ), b = a + j;
+                    const unsigned long long ka = keys[ a ], kb = keys[ b ];
+                    const u16 ia = id[ a ], ib = id[ b ];
+                    const bool greater = ka > kb || ( ka == kb && ia > ib );
+                    if ( greater == ! ( a & k ) ) { keys[ a ] = kb; keys[ b ] = ka; id[ a ] = ib; id[ b ] = ia; }
+                }
+                __syncthreads();
+            }
+    }
+    // ( the keys' room: the partitions' output, the segments, the flags )
+    u16 *alt = reinterpret_cast<u16 *>( keys );                       // [ D ][ SMALL_TREE ]
+    unsigned char *flag = reinterpret_cast<unsigned char *>( alt + 3 * SMALL_TREE );
+    u16 *cur = &lists[ 0 ][ 0 ];
+    const int p0 = 8 * tid;
+    int seg[ 8 ];
+    for ( int u = 0; u < 8; ++u ) seg[ u ] = 0;
+    for ( int L = 0; L < depth; ++L ) {
+        const int count = 1 << L;
+        if ( tid < count ) {
+            const int j = tid;
+            int b = 0, e = n, axis, mid;
+            if ( L ) {
+                b = j & 1 ? pmid[ j / 2 ] : pbeg[ j / 2 ];
+                e = j & 1 ? pend[ j / 2 ] : pmid[ j / 2 ];
+            }
+            double lo[ D ], hi[ D ];
+            node_cut<D>( b, e, pos, cur, SMALL_TREE, leaf, lo, hi, axis, mid );
+            const int p = preorder_of( j, L, depth );
+            out.lvl_nodes[ count - 1 + j ] = p;
+            out.beg[ p ] = b;
+            out.end[ p ] = e;
+            for ( int d = 0; d < D; ++d ) { out.box[ 2 * D * p + d ] = lo[ d ]; out.box[ 2 * D * p + D + d ] = hi[ d ]; }
+            nbeg[ j ] = u16( b );
+            nend[ j ] = u16( e );
+            nmid[ j ] = u16( mid );
+            naxis[ j ] = ( unsigned char )( axis );
+        }
+        __syncthreads();
+        if ( L + 1 == depth ) break;
+        for ( int u = 0; u < 8; ++u )
+            if ( p0 + u < n ) flag[ cur[ naxis[ seg[ u ] ] * SMALL_TREE + p0 + u ] ] = p0 + u < nmid[ seg[ u ] ];
+        __syncthreads();
+        for ( int d = 0; d < D; ++d ) {
+            const u16 *in = cur + d * SMALL_TREE;
+            u16 *to = alt + d * SMALL_TREE;
+            unsigned f = 0, c = 0, all;
+            for ( int u = 0; u < 8; ++u )
+                if ( p0 + u < n && flag[ in[ p0 + u ] ] ) { f |= 1u << u; ++c; }
+            const unsigned before = block_exclusive<SMALL_T>( c, sh, all );
+            // the prefix at each segment's start, from the thread that holds it
+            for ( int u = 0; u < 8; ++u )
+                if ( p0 + u < n && p0 + u == nbeg[ seg[ u ] ] ) npre[ seg[ u ] ] = u16( before + __popc( f & ( ( 1u << u ) - 1 ) ) );
+            __syncthreads();
+            for ( int u = 0; u < 8; ++u ) {
+                if ( p0 + u >= n ) continue;
+                const int j = seg[ u ], lb = int( before ) + __popc( f & ( ( 1u << u ) - 1 ) ) - npre[ j ];
+                to[ f >> u & 1 ? nbeg[ j ] + lb : nmid[ j ] + ( p0 + u - nbeg[ j ] ) - lb ] = in[ p0 + u ];
+            }
+            __syncthreads();
+        }
+        for ( int u = 0; u < 8; ++u )
+            if ( p0 + u < n ) seg[ u ] = 2 * seg[ u ] + ( p0 + u >= nmid[ seg[ u ] ] );
+        __syncthreads();
+        if ( tid < count ) { pbeg[ tid ] = nbeg[ tid ]; pend[ tid ] = nend[ tid ]; pmid[ tid ] = nmid[ tid ]; }
+        // ( the flags lie past the partitions' output and are written anew before the lists change places again )
+        for ( int d = 0; d < D; ++d )
+            for ( int i = tid; i < n; i += SMALL_T ) cur[ d * SMALL_TREE + i ] = alt[ d * SMALL_TREE + i ];
+        __syncthreads();
+    }
+    // the leaves' seeds in ascending user index, then the rank tables
+    if ( tid < 1 << ( depth - 1 ) ) {
+        const int b = nbeg[ tid ], e = nend[ tid ];
+        for ( int i = b + 1; i < e; ++i ) {
+            const u16 v = cur[ i ];
+            int k = i;
+            for ( ; k > b && cur[ k - 1 ] > v; --k ) cur[ k ] = cur[ k - 1 ];
+            cur[ k ] = v;
+        }
+        if ( out.leaf_of ) for ( int i = b; i < e; ++i ) out.leaf_of[ i ] = tid;
+    }
+    __syncthreads();
+    for ( int k = tid; k < n; k += SMALL_T ) {
+        const int u = cur[ k ];
+        out.order[ k ] = u;
+        out.rank_of[ u ] = k;
+        out.seeds[ k ] = seed_of<D>( pos, u );
+    }
+}
+
+/// the tree of `D`-dimensional seeds into the arrays of `o` ( see the file's header )
+template<int D>
+void build_into( const SmallOut &o, I64 n, const double *pos, int leaf, int depth, hipStream_t st ) {
+    const I64 N = ( I64( 1 ) << depth ) - 1;
+    if ( n <= SMALL_TREE && ( 1 << ( depth - 1 ) ) <= SMALL_NODES ) {
+        k_small_tree<D><<<1, SMALL_T, 0, st>>>( int( n ), pos, leaf, depth, o );
+        check_launch( "k_small_tree" );
         return;
     }
-    double lo[ 3 ], hi[ 3 ];
-    for ( int d = 0; d < 3; ++d ) {
-        lo[ d ] = pos[ 3 * size_t( L.id[ d ][ b ] ) + d ];
-        hi[ d ] = pos[ 3 * size_t( L.id[ d ][ e - 1 ] ) + d ];
-        bx[ d ] = lo[ d ];
-        bx[ 3 + d ] = hi[ d ];
+    Arena &A = arena();
+    // scratch ( one build at a time on a thread's arena ), `D` lists an array
+    unsigned long long *ka = A.get<unsigned long long>( "tb.ka", size_t( n ) * D ), *kb = A.get<unsigned long long>( "tb.kb", size_t( n ) * D );
+    int *va = A.get<int>( "tb.va", size_t( n ) * D ), *vb = A.get<int>( "tb.vb", size_t( n ) * D );
+    const int nt = int( ( n + RS_TILE - 1 ) / RS_TILE ), nsb = int( ( n + 1023 ) / 1024 ), lists = D == 2 ? 1 : D;
+    unsigned *hist = A.get<unsigned>( "tb.hist", size_t( 256 ) * nt * D ), *total = A.get<unsigned>( "tb.total", 256 * D );
+    int *hbeg = A.get<int>( "tb.hbeg", size_t( N ) ), *hend = A.get<int>( "tb.hend", size_t( N ) );
+    int *haxis = A.get<int>( "tb.haxis", size_t( N ) ), *hmid = A.get<int>( "tb.hmid", size_t( N ) );
+    double *hbox = A.get<double>( "tb.hbox", size_t( N ) * 2 * D );
+    int *seg = A.get<int>( "tb.seg", size_t( n ) ), *seg2 = A.get<int>( "tb.seg2", size_t( n ) );
+    unsigned char *flag = A.get<unsigned char>( "tb.flag", size_t( n ) );
+    unsigned *s = A.get<unsigned>( "tb.s", size_t( n ) * lists ), *bsum = A.get<unsigned>( "tb.bsum", size_t( nsb ) * lists );
+    const unsigned nbk = blocks_for( n, 256 );
+    k_keys<<<dim3( nbk, D ), 256, 0, st>>>( n, pos, D, ka, va );
+    radix_sort( n, D, ka, va, kb, vb, hist, total, st );
+    for ( int L = 0; L < depth; ++L ) {
+        k_level_nodes<D><<<blocks_for( I64( 1 ) << L, 256 ), 256, 0, st>>>( L, n, pos, va, leaf, hbox, haxis, hmid, hbeg, hend );
+        if ( L + 1 == depth ) break;
+        k_flags<<<nbk, 256, 0, st>>>( n, L, seg, haxis, hmid, va, flag );
+        k_scan_blocks<D><<<dim3( nsb, lists ), 1024, 0, st>>>( n, L, seg, haxis, va, flag, s, bsum );
+        k_scan_sums<<<lists, 1024, 0, st>>>( nsb, bsum );
+        k_partition<D><<<dim3( nbk, lists ), 256, 0, st>>>( n, L, seg, haxis, hbeg, hmid, va, flag, s, bsum, nsb, vb, seg2 );
+        check_launch( "tree level" );
+        std::swap( va, vb );
+        std::swap( seg, seg2 );
     }
-    int ax = 0;                                          // ( the first longest axis, as the host build picks it )
-    for ( int d = 1; d < 3; ++d ) if ( hi[ d ] - lo[ d ] > hi[ ax ] - lo[ ax ] ) ax = d;
-    axis[ j ] = ax;
-    mid[ j ] = ( e - b > leaf && hi[ ax ] > lo[ ax ] ) ? b + ( e - b ) / 2 : e;
-}
-
-/// the side of every seed from its node's cut list: `flag[ id ] = position < mid`
-__global__ void k_flags3( I64 n, const int *seg, const int *axis, const int *mid, Lists3 L, unsigned char *flag ) {
-    const I64 p = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
-    if ( p >= n ) return;
-    const int j = seg[ p ];
-    flag[ L.id[ axis[ j ] ][ p ] ] = p < mid[ j ];
-}
-
-/// the left flags of list `ids`, in its order
-__global__ void k_list_flags( I64 n, const int *ids, const unsigned char *flag, unsigned *f ) {
-    const I64 p = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
-    if ( p < n ) f[ p ] = flag[ ids[ p ] ];
-}
-
-/// the stable partition of list `ids` inside every segment by the flags ( `s` their exclusive scan in the list's order )
-__global__ void k_partition_list( I64 n, const int *seg, const int *beg, const int *mid, const int *ids, const unsigned char *flag,
-                                  const unsigned *s, int *out ) {
-    const I64 p = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
-    if ( p >= n ) return;
-    const int j = seg[ p ];
-    const int b = beg[ j ], m = mid[ j ], id = ids[ p ];
-    const unsigned left_before = s[ p ] - s[ b ];
-    out[ flag[ id ] ? b + int( left_before ) : m + int( ( p - b ) - left_before ) ] = id;
-}
-
-__global__ void k_rank_tables3( I64 n, const int *ids, const double *pos, int *order, int *rank_of, double4 *seeds ) {
-    const I64 k = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
-    if ( k >= n ) return;
-    const int u = ids[ k ];
-    order[ k ] = u;
-    rank_of[ u ] = int( k );
-    seeds[ k ] = make_double4( pos[ 3 * size_t( u ) ], pos[ 3 * size_t( u ) + 1 ], pos[ 3 * size_t( u ) + 2 ], 0.0 );
-}
-
-__global__ void k_to_preorder3( I64 N, const int *pre, const int *hbeg, const int *hend, const double *hbox, int *beg, int *end, double *box ) {
-    const I64 h = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
-    if ( h >= N ) return;
-    const int p = pre[ h ];
-    beg[ p ] = hbeg[ h ];
-    end[ p ] = hend[ h ];
-    for ( int c = 0; c < 6; ++c ) box[ 6 * size_t( p ) + c ] = hbox[ 6 * size_t( h ) + c ];
+    const int L = depth - 1;
+    k_leaves<<<blocks_for( I64( 1 ) << L, 256 ), 256, 0, st>>>( 1 << L, ( 1 << L ) - 1, hbeg, hend, va, o.leaf_of );
+    k_rank_tables<D><<<nbk, 256, 0, st>>>( n, va, pos, o.order, o.rank_of, o.seeds );
+    k_to_preorder<<<blocks_for( N, 256 ), 256, 0, st>>>( N, depth, 2 * D, hbeg, hend, hbox, o.beg, o.end, o.box, o.lvl_nodes );
+    check_launch( "tree finish" );
 }
 
 } // namespace
@@ -367,68 +485,7 @@ void build_tree_device3( DevTree3 &t, I64 n, const double *pos, int leaf, hipStr
     t.stat = A.get<double>( tag + ".stat3", size_t( N ) * 16 );
     t.fit = A.get<double>( tag + ".fit3", size_t( N ) * 3 );
     t.rkeys = A.get<unsigned long long>( tag + ".rkeys3", size_t( N ) * 3 );
-    // scratch ( shared with the 2D build's names: one build at a time on a thread's arena )
-    unsigned long long *ka = A.get<unsigned long long>( "tb.ka", size_t( n ) ), *kb = A.get<unsigned long long>( "tb.kb", size_t( n ) );
-    int *va = A.get<int>( "tb.va", size_t( n ) ), *vb = A.get<int>( "tb.vb", size_t( n ) );
-    int *lst[ 3 ], *lso[ 3 ];
-    for ( int d = 0; d < 3; ++d ) {
-        lst[ d ] = A.get<int>( "tb3.l" + std::to_string( d ), size_t( n ) );
-        lso[ d ] = A.get<int>( "tb3.o" + std::to_string( d ), size_t( n ) );
-    }
-    const int nt = int( ( n + RS_TILE - 1 ) / RS_TILE );
-    unsigned *hist = A.get<unsigned>( "tb.hist", size_t( 256 ) * nt );
-    const I64 half = I64( 1 ) << ( depth - 1 );
-    int *beg = A.get<int>( "tb.beg", size_t( half ) ), *end = A.get<int>( "tb.end", size_t( half ) );
-    int *nbeg = A.get<int>( "tb.nbeg", size_t( half ) ), *nend = A.get<int>( "tb.nend", size_t( half ) );
-    int *axis = A.get<int>( "tb.axis", size_t( half ) ), *mid = A.get<int>( "tb.mid", size_t( half ) );
-    int *hbeg = A.get<int>( "tb.hbeg", size_t( N ) ), *hend = A.get<int>( "tb.hend", size_t( N ) );
-    double *hbox = A.get<double>( "tb3.hbox", size_t( N ) * 6 );
-    int *seg = A.get<int>( "tb.seg", size_t( n ) );
-    unsigned char *flag = A.get<unsigned char>( "tb.flag", size_t( n ) );
-    unsigned *f = A.get<unsigned>( "tb.f", size_t( n ) ), *s = A.get<unsigned>( "tb.s", size_t( n ) );
-    const I64 nsb = ( n + 1023 ) / 1024;
-    unsigned *bsum = A.get<unsigned>( "tb.bsum", size_t( nsb ) );
-    const unsigned nbk = blocks_for( n, 256 );
-
-    // 1. the three sorted lists
-    for ( int ax = 0; ax < 3; ++ax ) {
-        k_keys<<<nbk, 256, 0, st>>>( n, pos, 3, ax, ka, va );
-        const Sorted r = radix_sort( n, ka, va, kb, vb, hist, st );
-        SDOT_HIP( hipMemcpyAsync( lst[ ax ], r.val, sizeof( int ) * size_t( n ), hipMemcpyDeviceToDevice, st ) );
-    }
-    // 2. the levels
-    const int zero = 0, nn = int( n );
-    SDOT_HIP( hipMemcpyAsync( beg, &zero, sizeof( int ), hipMemcpyHostToDevice, st ) );
-    SDOT_HIP( hipMemcpyAsync( end, &nn, sizeof( int ), hipMemcpyHostToDevice, st ) );
-    for ( int L = 0; L < depth; ++L ) {
-        const int count = 1 << L, first = count - 1;
-        k_level_nodes3<<<blocks_for( count, 256 ), 256, 0, st>>>( count, first, beg, end, pos, Lists3{ { lst[ 0 ], lst[ 1 ], lst[ 2 ] } }, leaf,
-                                                                  hbox, axis, mid, hbeg, hend );
-        if ( L + 1 == depth ) break;
-        k_fill_seg<<<count, 256, 0, st>>>( count, beg, end, seg );
-        k_flags3<<<nbk, 256, 0, st>>>( n, seg, axis, mid, Lists3{ { lst[ 0 ], lst[ 1 ], lst[ 2 ] } }, flag );
-        for ( int d = 0; d < 3; ++d ) {
-            k_list_flags<<<nbk, 256, 0, st>>>( n, lst[ d ], flag, f );
-            k_scan_blocks<<<unsigned( nsb ), 1024, 0, st>>>( n, f, s, bsum );
-            k_scan_single<<<1, 1024, 0, st>>>( bsum, int( nsb ) );
-            k_scan_add<<<nbk, 256, 0, st>>>( n, s, bsum );
-            k_partition_list<<<nbk, 256, 0, st>>>( n, seg, beg, mid, lst[ d ], flag, s, lso[ d ] );
-        }
-        for ( int d = 0; d < 3; ++d ) std::swap( lst[ d ], lso[ d ] );
-        k_children<<<blocks_for( count, 256 ), 256, 0, st>>>( count, beg, end, mid, nbeg, nend );
-        std::swap( beg, nbeg );
-        std::swap( end, nend );
-        check_launch( "3D tree level" );
-    }
-    // 3. leaves, rank tables, preorder
-    const int L = depth - 1;
-    k_leaves<<<blocks_for( I64( 1 ) << L, 256 ), 256, 0, st>>>( 1 << L, ( 1 << L ) - 1, hbeg, hend, lst[ 0 ], nullptr );
-    k_rank_tables3<<<nbk, 256, 0, st>>>( n, lst[ 0 ], pos, t.order, t.rank_of, t.seeds );
-    for ( int l = 0; l < depth; ++l ) k_preorder<<<blocks_for( I64( 1 ) << l, 256 ), 256, 0, st>>>( l, depth, t.lvl_nodes );
-    k_to_preorder3<<<blocks_for( N, 256 ), 256, 0, st>>>( N, t.lvl_nodes, hbeg, hend, hbox, t.node_beg, t.node_end, t.node_box );
-    check_launch( "3D tree finish" );
-    // `beg` / `end` came from host constants ( `zero`, `nn` ): the copies must be done before they go
-    SDOT_HIP( hipStreamSynchronize( st ) );
+    build_into<3>( SmallOut{ t.node_beg, t.node_end, t.lvl_nodes, t.order, t.rank_of, nullptr, t.node_box, t.seeds }, n, pos, leaf, depth, st );
 }
 
 void build_tree_device( DevTree &t, I64 n, const double *pos, int leaf, hipStream_t st, const std::string &tag ) {
@@ -451,63 +508,7 @@ void build_tree_device( DevTree &t, I64 n, const double *pos, int leaf, hipStrea
     t.stat = A.get<double>( tag + ".stat", size_t( N ) * 11 );
     t.fit = A.get<double>( tag + ".fit", size_t( N ) * 2 );
     t.rkeys = A.get<unsigned long long>( tag + ".rkeys", size_t( N ) * 3 );
-    // scratch
-    unsigned long long *ka = A.get<unsigned long long>( "tb.ka", size_t( n ) ), *kb = A.get<unsigned long long>( "tb.kb", size_t( n ) );
-    int *va = A.get<int>( "tb.va", size_t( n ) ), *vb = A.get<int>( "tb.vb", size_t( n ) );
-    int *xid = A.get<int>( "tb.xid", size_t( n ) ), *yid = A.get<int>( "tb.yid", size_t( n ) );
-    int *xo = A.get<int>( "tb.xo", size_t( n ) ), *yo = A.get<int>( "tb.yo", size_t( n ) );
-    const int nt = int( ( n + RS_TILE - 1 ) / RS_TILE );
-    unsigned *hist = A.get<unsigned>( "tb.hist", size_t( 256 ) * nt );
-    const I64 half = I64( 1 ) << ( depth - 1 );
-    int *beg = A.get<int>( "tb.beg", size_t( half ) ), *end = A.get<int>( "tb.end", size_t( half ) );
-    int *nbeg = A.get<int>( "tb.nbeg", size_t( half ) ), *nend = A.get<int>( "tb.nend", size_t( half ) );
-    int *axis = A.get<int>( "tb.axis", size_t( half ) ), *mid = A.get<int>( "tb.mid", size_t( half ) );
-    int *hbeg = A.get<int>( "tb.hbeg", size_t( N ) ), *hend = A.get<int>( "tb.hend", size_t( N ) );
-    double *hbox = A.get<double>( "tb.hbox", size_t( N ) * 4 );
-    int *seg = A.get<int>( "tb.seg", size_t( n ) );
-    unsigned char *flag = A.get<unsigned char>( "tb.flag", size_t( n ) );
-    unsigned *f = A.get<unsigned>( "tb.f", size_t( n ) ), *s = A.get<unsigned>( "tb.s", size_t( n ) );
-    const I64 nsb = ( n + 1023 ) / 1024;
-    unsigned *bsum = A.get<unsigned>( "tb.bsum", size_t( nsb ) );
-    const unsigned nbk = blocks_for( n, 256 );
-
-    // 1. the two sorted lists
-    for ( int ax = 0; ax < 2; ++ax ) {
-        k_keys<<<nbk, 256, 0, st>>>( n, pos, 2, ax, ka, va );
-        const Sorted r = radix_sort( n, ka, va, kb, vb, hist, st );
-        SDOT_HIP( hipMemcpyAsync( ax ? yid : xid, r.val, sizeof( int ) * size_t( n ), hipMemcpyDeviceToDevice, st ) );
-    }
-    // 2. the levels
-    const int zero = 0, nn = int( n );
-    SDOT_HIP( hipMemcpyAsync( beg, &zero, sizeof( int ), hipMemcpyHostToDevice, st ) );
-    SDOT_HIP( hipMemcpyAsync( end, &nn, sizeof( int ), hipMemcpyHostToDevice, st ) );
-    for ( int L = 0; L < depth; ++L ) {
-        const int count = 1 << L, first = count - 1;
-        k_level_nodes<<<blocks_for( count, 256 ), 256, 0, st>>>( count, first, beg, end, pos, xid, yid, leaf, hbox, axis, mid, hbeg, hend );
-        if ( L + 1 == depth ) break;
-        k_fill_seg<<<count, 256, 0, st>>>( count, beg, end, seg );
-        k_flags<<<nbk, 256, 0, st>>>( n, seg, axis, mid, xid, yid, flag );
-        k_other_flags<<<nbk, 256, 0, st>>>( n, seg, axis, xid, yid, flag, f );
-        k_scan_blocks<<<unsigned( nsb ), 1024, 0, st>>>( n, f, s, bsum );
-        k_scan_single<<<1, 1024, 0, st>>>( bsum, int( nsb ) );
-        k_scan_add<<<nbk, 256, 0, st>>>( n, s, bsum );
-        k_partition<<<nbk, 256, 0, st>>>( n, seg, axis, beg, mid, xid, yid, flag, s, xo, yo );
-        std::swap( xid, xo );
-        std::swap( yid, yo );
-        k_children<<<blocks_for( count, 256 ), 256, 0, st>>>( count, beg, end, mid, nbeg, nend );
-        std::swap( beg, nbeg );
-        std::swap( end, nend );
-        check_launch( "tree level" );
-    }
-    // 3. leaves, rank tables, preorder
-    const int L = depth - 1;
-    k_leaves<<<blocks_for( I64( 1 ) << L, 256 ), 256, 0, st>>>( 1 << L, ( 1 << L ) - 1, hbeg, hend, xid, t.leaf_of );
-    k_rank_tables<<<nbk, 256, 0, st>>>( n, xid, pos, t.order, t.rank_of, t.seeds );
-    for ( int l = 0; l < depth; ++l ) k_preorder<<<blocks_for( I64( 1 ) << l, 256 ), 256, 0, st>>>( l, depth, t.lvl_nodes );
-    k_to_preorder<<<blocks_for( N, 256 ), 256, 0, st>>>( N, t.lvl_nodes, hbeg, hend, hbox, t.node_beg, t.node_end, t.node_box );
-    check_launch( "tree finish" );
-    // `beg` / `end` came from host constants ( `zero`, `nn` ): the copies must be done before they go
-    SDOT_HIP( hipStreamSynchronize( st ) );
+    build_into<2>( SmallOut{ t.node_beg, t.node_end, t.lvl_nodes, t.order, t.rank_of, t.leaf_of, t.node_box, t.seeds }, n, pos, leaf, depth, st );
     t.h_lvl_nodes.clear();
 }
 
