@@ -107,7 +107,7 @@ void run_cells( const DevTree &t, const double *lo, const double *hi, const Dens
                 bool fp32 = false, int ovf_slots = OVF_SLOTS, I64 poly_chunk = POLY_CHUNK );
 
 /// the event counts of a diagram's passes are gathered in `EV_SHARDS` cache lines ( `[ shard ][ 8 ]` ), a block in its own: one line takes
-/// an atomic every ~12 ns from the whole chip ( five a wave: 64 us for a pass of 1024 waves with nothing to do, 19 of the 27 ms of 300k
+/// an atomic every ~12 ns from the whole chip ( five a wave: 64 us for a pass of 1024 waves with nothing to do, 0.3 of the 1.6 ms of 20k
 /// 3D cells, a wave each ). `event_shards` gives them cleared, `fold_events` adds them to `events` and clears them
 constexpr int EV_SHARDS = 64;
 unsigned long long *event_shards( hipStream_t st );

@@ -41,6 +41,7 @@ struct Params3 {
     DiagramOut      out;
     int             mode, room;
     PolyBuf         pb;
+    unsigned long long *shards;                          ///< the event counts ( `event_shards` )
 };
 
 /// what a wave keeps in LDS: its cell's faces, the staging of a cut, the walk's stack
@@ -761,11 +762,12 @@ __global__ __launch_bounds__( 64 * WAVES3 ) void k_cells3( Params3 P ) {
         wave_sync();
     }
     if ( lane == 0 ) {
-        atomicAdd( &P.out.events[ 0 ], ev_side );
-        atomicAdd( &P.out.events[ 1 ], ev_prune );
-        atomicAdd( &P.out.events[ 2 ], ev_new );
-        atomicAdd( &P.out.events[ 3 ], ev_visit );
-        atomicAdd( &P.out.events[ 4 ], ev_cut );
+        unsigned long long *to = P.shards + 8 * ( blockIdx.x & ( EV_SHARDS - 1 ) );
+        atomicAdd( &to[ 0 ], ev_side );
+        atomicAdd( &to[ 1 ], ev_prune );
+        atomicAdd( &to[ 2 ], ev_new );
+        atomicAdd( &to[ 3 ], ev_visit );
+        atomicAdd( &to[ 4 ], ev_cut );
     }
     const I64 row0 = I64( k0 / 64 ) * 64 * P.room + ( k0 & 63 );
     if ( status == C3_FAILED || status == C3_FULL ) {
@@ -917,77 +919,12 @@ struct Slot3 {
     int    nv, nf, res;
 };
 
-/// the rest of a cut once the signs `s` are known and one is positive ( lane 0 alone, on the slot in LDS ): the
-/// classification with the tie bound, the inside vertices renumbered, a new vertex per crossing edge, the new face
-/// closed -- the oracle's `cut3` step by step
-__device__ int cut_slot_rest( Slot3 &C, double nx, double ny, double nz, double off, int id, double vm, unsigned long long &ev_new ) {
-    const int nv = C.nv;
-    const double tie = 1e-13 * ( ( fabs( nx ) + fabs( ny ) + fabs( nz ) ) * vm + fabs( off ) );
-    int nin = 0;
-    for ( int v = 0; v < nv; ++v ) {
-        if ( ! ( C.s[ v ] > tie ) ) { C.s[ v ] = fmin( C.s[ v ], 0.0 ); C.idx[ v ] = nin++; }
-        else C.idx[ v ] = -1;
-    }
-    if ( nin == nv ) return C3_UNCHANGED;
-    if ( nin == 0 ) return C3_EMPTY;
-    if ( C.nf >= SLOT_F ) return C3_FULL;
-    const int fn = C.nf;
-    C.fx[ fn ] = nx; C.fy[ fn ] = ny; C.fz[ fn ] = nz; C.fo[ fn ] = off; C.fid[ fn ] = id;
-    for ( int v = 0; v < nv; ++v ) {                    // the inside vertices, their neighbours renumbered
-        const int i = C.idx[ v ];
-        if ( i < 0 ) continue;
-        C.X[ i ] = C.x[ v ]; C.Y[ i ] = C.y[ v ]; C.Z[ i ] = C.z[ v ];
-        for ( int j = 0; j < 3; ++j ) { C.PL[ 3 * i + j ] = C.pl[ 3 * v + j ]; C.NB[ 3 * i + j ] = C.idx[ C.nb[ 3 * v + j ] ]; }
-    }
-    int T = 0;
-    for ( int b = 0; b < nv; ++b ) {                    // a new vertex per crossing edge, in the order ( outside vertex, edge )
-        if ( C.idx[ b ] >= 0 ) continue;
-        for ( int k = 0; k < 3; ++k ) {
-            const int a = C.nb[ 3 * b + k ];
-            if ( C.idx[ a ] < 0 ) continue;
-            const int g = nin + T;
-            if ( g >= SLOT_V ) return C3_FULL;
-            const double sa = C.s[ a ], t = sa / ( sa - C.s[ b ] );
-            C.X[ g ] = fma( C.x[ b ] - C.x[ a ], t, C.x[ a ] );
-            C.Y[ g ] = fma( C.y[ b ] - C.y[ a ], t, C.y[ a ] );
-            C.Z[ g ] = fma( C.z[ b ] - C.z[ a ], t, C.z[ a ] );
-            const int p1 = C.pl[ 3 * b + ( k + 1 ) % 3 ], p2 = C.pl[ 3 * b + ( k + 2 ) % 3 ];
-            C.PL[ 3 * g ] = fn; C.PL[ 3 * g + 1 ] = p1; C.PL[ 3 * g + 2 ] = p2;
-            C.NB[ 3 * g ] = C.idx[ a ];
-            C.np1[ T ] = p1; C.np2[ T ] = p2;
-            const int ia = C.idx[ a ];
-            for ( int j = 0; j < 3; ++j )
-                if ( C.nb[ 3 * a + j ] == b ) C.NB[ 3 * ia + j ] = g;
-            ++T;
-        }
-    }
-    for ( int t0 = 0; t0 < T; ++t0 ) {                  // the new face closed
-        const int p1 = C.np1[ t0 ], p2 = C.np2[ t0 ];
-        int m1 = 0, m2 = 0, c1 = 0, c2 = 0;
-        for ( int t = 0; t < T; ++t ) {
-            if ( t == t0 ) continue;
-            if ( C.np1[ t ] == p2 || C.np2[ t ] == p2 ) { m1 = nin + t; ++c1; }
-            if ( C.np1[ t ] == p1 || C.np2[ t ] == p1 ) { m2 = nin + t; ++c2; }
-        }
-        if ( c1 != 1 || c2 != 1 ) return C3_FAILED;
-        C.NB[ 3 * ( nin + t0 ) + 1 ] = m1;
-        C.NB[ 3 * ( nin + t0 ) + 2 ] = m2;
-    }
-    const int m = nin + T;
-    for ( int v = 0; v < m; ++v ) {
-        C.x[ v ] = C.X[ v ]; C.y[ v ] = C.Y[ v ]; C.z[ v ] = C.Z[ v ];
-        for ( int j = 0; j < 3; ++j ) { C.pl[ 3 * v + j ] = C.PL[ 3 * v + j ]; C.nb[ 3 * v + j ] = C.NB[ 3 * v + j ]; }
-    }
-    C.nv = m;
-    C.nf = fn + 1;
-    ev_new += unsigned( T );
-    return C3_CUT;
-}
-
-/// the cut of an overflowed cell by its wave: the signs by every lane, the rest by lane 0 when a vertex is outside
+/// the cut of an overflowed cell by its wave, the oracle's `cut3` step by step with a lane a vertex ( `SLOT_V / 64` each ): the signs, the
+/// classification with the tie bound, the inside vertices renumbered, a new vertex per crossing edge in the order ( outside
+/// vertex, edge ), the new face closed, the cell copied back. ( One lane alone took ~40 us a cut of 70 vertices, 1.4 ms a cell. )
 __device__ int cut_slot( Slot3 &C, int lane, double nx, double ny, double nz, double off, int id, unsigned long long &ev_side,
                          unsigned long long &ev_new ) {
-    const int nv = C.nv;
+    const int nv = C.nv, fn = C.nf;
     ev_side += unsigned( nv );
     bool any = false;
     double vm = 0;
@@ -999,10 +936,89 @@ __device__ int cut_slot( Slot3 &C, int lane, double nx, double ny, double nz, do
     }
     if ( __ballot( any ) == 0 ) return C3_UNCHANGED;
     vm = wave_maxd( vm );
+    const double tie = 1e-13 * ( ( fabs( nx ) + fabs( ny ) + fabs( nz ) ) * vm + fabs( off ) );
+    const unsigned long long before = ( 1ull << lane ) - 1;
+    int nin = 0;
+    for ( int v0 = 0; v0 < nv; v0 += 64 ) {              // ( each lane on its own vertices' signs )
+        const int v = v0 + lane;
+        const bool in = v < nv && ! ( C.s[ v ] > tie );
+        const unsigned long long m = __ballot( in );
+        if ( v < nv ) {
+            C.idx[ v ] = in ? nin + __popcll( m & before ) : -1;
+            if ( in ) C.s[ v ] = fmin( C.s[ v ], 0.0 );
+        }
+        nin += __popcll( m );
+    }
+    if ( nin == nv ) return C3_UNCHANGED;
+    if ( nin == 0 ) return C3_EMPTY;
+    if ( fn >= SLOT_F ) return C3_FULL;
     __syncthreads();                                     // ( the block is the wave )
-    if ( lane == 0 ) C.res = cut_slot_rest( C, nx, ny, nz, off, id, vm, ev_new );
+    for ( int v = lane; v < nv; v += 64 ) {              // the inside vertices, their neighbours renumbered
+        const int i = C.idx[ v ];
+        if ( i < 0 ) continue;
+        C.X[ i ] = C.x[ v ]; C.Y[ i ] = C.y[ v ]; C.Z[ i ] = C.z[ v ];
+        for ( int j = 0; j < 3; ++j ) { C.PL[ 3 * i + j ] = C.pl[ 3 * v + j ]; C.NB[ 3 * i + j ] = C.idx[ C.nb[ 3 * v + j ] ]; }
+    }
     __syncthreads();
-    return C.res;
+    int T = 0;
+    for ( int v0 = 0; v0 < nv; v0 += 64 ) {              // a new vertex per crossing edge
+        const int b = v0 + lane;
+        const bool out = b < nv && C.idx[ b ] < 0;
+        int cnt = 0;
+        if ( out ) for ( int k = 0; k < 3; ++k ) cnt += C.idx[ C.nb[ 3 * b + k ] ] >= 0;
+        int inc = cnt;
+        for ( int d = 1; d < 64; d <<= 1 ) { const int t = __shfl_up( inc, d, 64 ); if ( lane >= d ) inc += t; }
+        const int all = __shfl( inc, 63, 64 );
+        if ( nin + T + all > SLOT_V ) return C3_FULL;
+        int at = T + inc - cnt;
+        if ( out )
+            for ( int k = 0; k < 3; ++k ) {
+                const int a = C.nb[ 3 * b + k ], ia = C.idx[ a ];
+                if ( ia < 0 ) continue;
+                const int g = nin + at;
+                const double sa = C.s[ a ], t = sa / ( sa - C.s[ b ] );
+                C.X[ g ] = fma( C.x[ b ] - C.x[ a ], t, C.x[ a ] );
+                C.Y[ g ] = fma( C.y[ b ] - C.y[ a ], t, C.y[ a ] );
+                C.Z[ g ] = fma( C.z[ b ] - C.z[ a ], t, C.z[ a ] );
+                const int p1 = C.pl[ 3 * b + ( k + 1 ) % 3 ], p2 = C.pl[ 3 * b + ( k + 2 ) % 3 ];
+                C.PL[ 3 * g ] = fn; C.PL[ 3 * g + 1 ] = p1; C.PL[ 3 * g + 2 ] = p2;
+                C.NB[ 3 * g ] = ia;
+                C.np1[ at ] = p1; C.np2[ at ] = p2;
+                for ( int j = 0; j < 3; ++j )
+                    if ( C.nb[ 3 * a + j ] == b ) C.NB[ 3 * ia + j ] = g;
+                ++at;
+            }
+        T += all;
+    }
+    __syncthreads();
+    bool open = false;
+    for ( int t0 = lane; t0 < T; t0 += 64 ) {            // the new face closed
+        const int p1 = C.np1[ t0 ], p2 = C.np2[ t0 ];
+        int m1 = 0, m2 = 0, c1 = 0, c2 = 0;
+        for ( int t = 0; t < T; ++t ) {
+            if ( t == t0 ) continue;
+            if ( C.np1[ t ] == p2 || C.np2[ t ] == p2 ) { m1 = nin + t; ++c1; }
+            if ( C.np1[ t ] == p1 || C.np2[ t ] == p1 ) { m2 = nin + t; ++c2; }
+        }
+        open |= c1 != 1 || c2 != 1;
+        C.NB[ 3 * ( nin + t0 ) + 1 ] = m1;
+        C.NB[ 3 * ( nin + t0 ) + 2 ] = m2;
+    }
+    if ( __any( open ) ) return C3_FAILED;
+    __syncthreads();
+    const int m = nin + T;
+    for ( int v = lane; v < m; v += 64 ) {
+        C.x[ v ] = C.X[ v ]; C.y[ v ] = C.Y[ v ]; C.z[ v ] = C.Z[ v ];
+        for ( int j = 0; j < 3; ++j ) { C.pl[ 3 * v + j ] = C.PL[ 3 * v + j ]; C.nb[ 3 * v + j ] = C.NB[ 3 * v + j ]; }
+    }
+    if ( lane == 0 ) {
+        C.fx[ fn ] = nx; C.fy[ fn ] = ny; C.fz[ fn ] = nz; C.fo[ fn ] = off; C.fid[ fn ] = id;
+        C.nv = m;
+        C.nf = fn + 1;
+    }
+    ev_new += unsigned( T );
+    __syncthreads();
+    return C3_CUT;
 }
 
 /// the second pass: the cells past the lanes of the first, one wave per cell with the cell in LDS ( up to `SLOT_V`
@@ -1080,7 +1096,11 @@ __global__ __launch_bounds__( 64 ) void k_cells3_pass2( Params3 P ) {
             top += 2;
             __syncthreads();
         }
-        if ( lane == 0 ) { atomicAdd( &P.out.events[ 0 ], ev_side ); atomicAdd( &P.out.events[ 2 ], ev_new ); }
+        if ( lane == 0 ) {
+            unsigned long long *to = P.shards + 8 * ( blockIdx.x & ( EV_SHARDS - 1 ) );
+            atomicAdd( &to[ 0 ], ev_side );
+            atomicAdd( &to[ 2 ], ev_new );
+        }
         const I64 row0 = I64( k0 / 64 ) * 64 * P.room + ( k0 & 63 );
         if ( status == C3_FAILED || status == C3_FULL ) {
             if ( lane == 0 ) record_failure( P, k0, row0, status == C3_FULL ? 1 : 2 );
@@ -1194,6 +1214,7 @@ void run_cells_3d( const DevTree3 &t, const double *lo, const double *hi, const 
     P.out = out;
     P.mode = mode;
     P.room = room;
+    P.shards = event_shards( st );
     k_reset_counters3<<<1, 64, 0, st>>>( out.counters );
     check_launch( "k_reset_counters3" );
     Timing::Pending tp;
@@ -1219,6 +1240,7 @@ void run_cells_3d( const DevTree3 &t, const double *lo, const double *hi, const 
     if ( timed ) timing().end( tp, st );
     k_cells3_pass2<<<PASS2_BLOCKS3, 64, 0, st>>>( P );
     check_launch( "k_cells3_pass2" );
+    fold_events( P.shards, out.events, st );
 }
 
 } // namespace sdot_amd
