@@ -87,17 +87,6 @@ __device__ __forceinline__ double gauss_peak( double m, double s ) {
     return m / ( 2.5066282746310002 * 2.5066282746310002 * 2.5066282746310002 * s * s * s );
 }
 
-__device__ double rho_at( const Density3 &dn, double x, double y, double z ) {
-    if ( dn.kind == 0 ) return dn.rho;
-    double r = 0;
-    for ( int q = 0; q < dn.ng; ++q ) {
-        const double *g = dn.gauss + 5 * q;
-        const double s = g[ 3 ], dx = x - g[ 0 ], dy = y - g[ 1 ], dz = z - g[ 2 ];
-        r += gauss_peak( g[ 4 ], s ) * exp( -( dx * dx + dy * dy + dz * dz ) / ( 2 * s * s ) );
-    }
-    return r;
-}
-
 /// `int_0^1 exp( -u t^2 ) t^2 dt`, `e = exp( -u )`: below 1 the series `sum_k ( -u )^k / ( k! ( 2 k + 3 ) )` to `k = 19` by
 /// Horner ( the next term is below 3e-20 of the sum ), else `( sqrt( pi ) erf( sqrt u ) / 4 - sqrt( u ) e / 2 ) / u^1.5`
 __device__ __forceinline__ double radial_h( double u, double e ) {
@@ -337,6 +326,57 @@ __device__ CellSums image_terms( const Density3 &dn, const double4 &p0, bool fac
 }
 
 
+/// the 14-point rule on the tetrahedron `( A, g, v, o )` of volume `vol` ( seed frame, the seed at `p0` ) against a sum of Gaussians: the
+/// mass and the moments into `S`. The Gaussians outside, so that each one's peak and width divide once per tetrahedron
+__device__ __forceinline__ void gauss_rule14( const Density3 &dn, const double4 &p0, V3 A, V3 g, V3 v, V3 o, double vol, CellSums &S ) {
+    const double r1 = 0.0927352503108912264, r1w = 0.0734930431163619495;
+    const double r2 = 0.3108859192633006098, r2w = 0.1126879257180158507;
+    const double r3 = 0.0455037041256496494, r3w = 0.0425460207770814664;
+    for ( int q = 0; q < dn.ng; ++q ) {
+        const double *ga = dn.gauss + 5 * q;
+        const double s = ga[ 3 ], top = vol * gauss_peak( ga[ 4 ], s ), inv = 1 / ( 2 * s * s );
+        const double mx = ga[ 0 ] - p0.x, my = ga[ 1 ] - p0.y, mz = ga[ 2 ] - p0.z;
+#pragma unroll 1
+        for ( int qq = 0; qq < 14; ++qq ) {
+            double b0, b1, b2, b3, wq;
+            if ( qq < 8 ) {
+                const double a = qq < 4 ? r1 : r2;
+                wq = qq < 4 ? r1w : r2w;
+                const int jj = qq & 3;
+                b0 = jj == 0 ? 1 - 3 * a : a; b1 = jj == 1 ? 1 - 3 * a : a; b2 = jj == 2 ? 1 - 3 * a : a; b3 = jj == 3 ? 1 - 3 * a : a;
+            } else {
+                const int pr = qq - 8;                   // pairs ( 0 1 ) ( 0 2 ) ( 0 3 ) ( 1 2 ) ( 1 3 ) ( 2 3 )
+                const int i0 = pr < 3 ? 0 : pr < 5 ? 1 : 2, i1 = pr < 3 ? pr + 1 : pr < 5 ? pr - 1 : 3;
+                wq = r3w;
+                b0 = ( i0 == 0 || i1 == 0 ) ? r3 : 0.5 - r3; b1 = ( i0 == 1 || i1 == 1 ) ? r3 : 0.5 - r3;
+                b2 = ( i0 == 2 || i1 == 2 ) ? r3 : 0.5 - r3; b3 = ( i0 == 3 || i1 == 3 ) ? r3 : 0.5 - r3;
+            }
+            const double x = b0 * A.x + b1 * g.x + b2 * v.x + b3 * o.x;
+            const double y = b0 * A.y + b1 * g.y + b2 * v.y + b3 * o.y;
+            const double z = b0 * A.z + b1 * g.z + b2 * v.z + b3 * o.z;
+            const double dx = x - mx, dy = y - my, dz = z - mz;
+            const double w = wq * top * exp( -( dx * dx + dy * dy + dz * dz ) * inv );
+            S.mass += w;
+            S.mx += w * x; S.my += w * y; S.mz += w * z;
+            S.m2 += w * ( x * x + y * y + z * z );
+        }
+    }
+}
+
+/// the corners of the `k`-th of the `BOX_SUB^2` equal parts of the triangle `( g, v, o )` ( its rows have 7, 5, 3 and 1 )
+__device__ __forceinline__ void sub_triangle( int k, V3 g, V3 v, V3 o, V3 &P0, V3 &P1, V3 &P2 ) {
+    static_assert( BOX_SUB == 4, "the rows below" );
+    const int i = k < 7 ? 0 : k < 12 ? 1 : k < 15 ? 2 : 3, r = k - ( k < 7 ? 0 : k < 12 ? 7 : k < 15 ? 12 : 15 );
+    const int j = r / 2, down = r & 1;
+    auto at = [&]( int a, int b ) {
+        return V3{ g.x + ( v.x - g.x ) * a / BOX_SUB + ( o.x - g.x ) * b / BOX_SUB, g.y + ( v.y - g.y ) * a / BOX_SUB + ( o.y - g.y ) * b / BOX_SUB,
+                   g.z + ( v.z - g.z ) * a / BOX_SUB + ( o.z - g.z ) * b / BOX_SUB };
+    };
+    P0 = at( down ? i + 1 : i, j );
+    P1 = at( i + 1, down ? j + 1 : j );
+    P2 = at( i, j + 1 );
+}
+
 /// the triangle `( g, v, o )` of a face of outward unit normal `u`, and the tetrahedron it makes with the cell's mean
 /// vertex `A` ( seed frame; the seed at `p0` ): the facet's `int rho`, the mass ( a constant: the tetrahedron's volume; a
 /// sum of Gaussians: the flux through the triangle ), the moments ( the tetrahedron's )
@@ -388,32 +428,7 @@ __device__ __forceinline__ CellSums edge_terms( const Density3 &dn, const double
                 }
         return S;
     }
-    // the 14-point rule on the tetrahedron ( A, g, v, o )
-    const double r1 = 0.0927352503108912264, r1w = 0.0734930431163619495;
-    const double r2 = 0.3108859192633006098, r2w = 0.1126879257180158507;
-    const double r3 = 0.0455037041256496494, r3w = 0.0425460207770814664;
-    for ( int qq = 0; qq < 14; ++qq ) {
-        double b0, b1, b2, b3, wq;
-        if ( qq < 8 ) {
-            const double a = qq < 4 ? r1 : r2;
-            wq = qq < 4 ? r1w : r2w;
-            const int jj = qq & 3;
-            b0 = jj == 0 ? 1 - 3 * a : a; b1 = jj == 1 ? 1 - 3 * a : a; b2 = jj == 2 ? 1 - 3 * a : a; b3 = jj == 3 ? 1 - 3 * a : a;
-        } else {
-            const int pr = qq - 8;                       // pairs ( 0 1 ) ( 0 2 ) ( 0 3 ) ( 1 2 ) ( 1 3 ) ( 2 3 )
-            const int i0 = pr < 3 ? 0 : pr < 5 ? 1 : 2, i1 = pr < 3 ? pr + 1 : pr < 5 ? pr - 1 : 3;
-            wq = r3w;
-            b0 = ( i0 == 0 || i1 == 0 ) ? r3 : 0.5 - r3; b1 = ( i0 == 1 || i1 == 1 ) ? r3 : 0.5 - r3;
-            b2 = ( i0 == 2 || i1 == 2 ) ? r3 : 0.5 - r3; b3 = ( i0 == 3 || i1 == 3 ) ? r3 : 0.5 - r3;
-        }
-        const double x = b0 * A.x + b1 * g.x + b2 * v.x + b3 * o.x;
-        const double y = b0 * A.y + b1 * g.y + b2 * v.y + b3 * o.y;
-        const double z = b0 * A.z + b1 * g.z + b2 * v.z + b3 * o.z;
-        const double w = wq * vol * rho_at( dn, p0.x + x, p0.y + y, p0.z + z );
-        S.mass += w;
-        S.mx += w * x; S.my += w * y; S.mz += w * z;
-        S.m2 += w * ( x * x + y * y + z * z );
-    }
+    gauss_rule14( dn, p0, A, g, v, o, vol, S );
     return S;
 }
 
@@ -598,79 +613,87 @@ __device__ __forceinline__ double proximity3( const NodeRec3 &r, double px, doub
     return s;
 }
 
-/// a cell's faces in the wave's LDS ( the first pass ) or in the polytope buffer ( the measure kernel )
-struct LdsFaces {
-    const WaveLds &L;
-    __device__ double x( int f ) const { return L.fx[ f ]; }
-    __device__ double y( int f ) const { return L.fy[ f ]; }
-    __device__ double z( int f ) const { return L.fz[ f ]; }
-    __device__ int id( int f ) const { return L.fid[ f ]; }
-};
-struct BufFaces {
-    const PolyBuf &B;
-    I64 base;
-    __device__ double x( int f ) const { return B.fx[ base + f ]; }
-    __device__ double y( int f ) const { return B.fy[ base + f ]; }
-    __device__ double z( int f ) const { return B.fz[ base + f ]; }
-    __device__ int id( int f ) const { return B.fid[ base + f ]; }
-};
-
-/// the measures of a built cell, one wave ( this lane's vertex in `c` ), written to the outputs
-template<bool GAUSS, class Faces>
-__device__ void measure_cell( const Params3 &P, const Faces &F, const Cell3 &c, int lane, int k0, const double4 &p0, I64 row0 ) {
-    // the measures: face by face ( the faces in cut order, as the oracle lists the facets )
-    const bool act = lane < c.nv;
+/// the measures of a built cell against a constant density, one wave ( this lane's vertex in `c`; the faces and the cut's staging in `L` ),
+/// written to the outputs. The faces' mean vertices by a lane a face, the triangles ( mean vertex, edge ) by the lanes of their lower
+/// vertices, six at most each, a facet's parts summed in vertex order by the face's lane: instructions bound it, and face by face
+/// over the whole wave it was a third of them ( `k_cells3`, 300k cells: 27.4 -> 20.4 ms )
+__device__ void measure_flat( const Params3 &P, WaveLds &L, const Cell3 &c, int lane, int k0, const double4 &p0, I64 row0 ) {
+    const bool act = lane < c.nv, facets = P.mode == MODE_FACETS, moments = P.mode == MODE_MOMENTS;
+    const int nf = c.nv > 0 ? c.nf : 0;
     const double inv_nv = c.nv > 0 ? 1.0 / c.nv : 0.0;
-    const double Ax = wave_total( act ? c.x : 0.0 ) * inv_nv, Ay = wave_total( act ? c.y : 0.0 ) * inv_nv, Az = wave_total( act ? c.z : 0.0 ) * inv_nv;
-    double wx[ 3 ], wy[ 3 ], wz[ 3 ];
-    int nk[ 3 ];
-#pragma unroll
-    for ( int k = 0; k < 3; ++k ) {
-        nk[ k ] = byte_of( c.nb, k );
-        wx[ k ] = __shfl( c.x, nk[ k ], 64 ); wy[ k ] = __shfl( c.y, nk[ k ], 64 ); wz[ k ] = __shfl( c.z, nk[ k ], 64 );
+    const V3 Av{ wave_total( act ? c.x : 0.0 ) * inv_nv, wave_total( act ? c.y : 0.0 ) * inv_nv, wave_total( act ? c.z : 0.0 ) * inv_nv };
+    wave_sync();
+    if ( act ) { L.sx[ lane ] = c.x; L.sy[ lane ] = c.y; L.sz[ lane ] = c.z; L.spl[ lane ] = c.pl; }
+    wave_sync();
+    // a face a lane
+    int cnt = 0;
+    double norm = 1;
+    if ( lane < nf ) {
+        double gx = 0, gy = 0, gz = 0;
+        for ( int v = 0; v < c.nv; ++v ) {
+            const int pl = L.spl[ v ];
+            if ( byte_of( pl, 0 ) != lane && byte_of( pl, 1 ) != lane && byte_of( pl, 2 ) != lane ) continue;
+            ++cnt;
+            gx += L.sx[ v ]; gy += L.sy[ v ]; gz += L.sz[ v ];
+        }
+        const double fx = L.fx[ lane ], fy = L.fy[ lane ], fz = L.fz[ lane ];
+        norm = sqrt( fx * fx + fy * fy + fz * fz );
+        const double inv = 1.0 / cnt;                    // ( a face without a vertex: never read )
+        L.fx[ lane ] = gx * inv; L.fy[ lane ] = gy * inv; L.fz[ lane ] = gz * inv;
+        L.used[ lane ] = cnt >= 3;
     }
-    const bool facets = P.mode == MODE_FACETS, moments = P.mode == MODE_MOMENTS;
-    const V3 Av{ Ax, Ay, Az };
+    wave_sync();
+    // a vertex a lane
     CellSums S;
-    double dia = 0;
-    int q = 0;
-    for ( int f = 0; f < ( c.nv > 0 ? c.nf : 0 ); ++f ) {
-        int j = -1;
-        if ( act ) j = byte_of( c.pl, 0 ) == f ? 0 : byte_of( c.pl, 1 ) == f ? 1 : byte_of( c.pl, 2 ) == f ? 2 : -1;
-        const int cntf = __popcll( __ballot( j >= 0 ) );
-        if ( cntf < 3 ) continue;
-        const V3 g{ wave_total( j >= 0 ? c.x : 0.0 ) / cntf, wave_total( j >= 0 ? c.y : 0.0 ) / cntf, wave_total( j >= 0 ? c.z : 0.0 ) / cntf };
-        const double fnx = F.x( f ), fny = F.y( f ), fnz = F.z( f );
-        const int fid = F.id( f );
-        const double dn = sqrt( fnx * fnx + fny * fny + fnz * fnz );
-        const V3 u{ fnx / dn, fny / dn, fnz / dn };
-        S.part = 0;
-        if ( j >= 0 ) {
-            const V3 v{ c.x, c.y, c.z };
+    double part[ 3 ] = { 0, 0, 0 };
+    if ( act ) {
+        const V3 v{ c.x, c.y, c.z };
+#pragma unroll
+        for ( int j = 0; j < 3; ++j ) {
+            const int f = byte_of( c.pl, j );
+            if ( ! L.used[ f ] ) continue;
+            const V3 g{ L.fx[ f ], L.fy[ f ], L.fz[ f ] };
 #pragma unroll
             for ( int e = 1; e <= 2; ++e ) {             // the two edges of the face at this vertex, each counted by its lower lane
-                const int ks = ( j + e ) % 3;           // ( selects, not an index: no scratch )
-                const int w = ks == 0 ? nk[ 0 ] : ks == 1 ? nk[ 1 ] : nk[ 2 ];
+                const int w = byte_of( c.nb, ( j + e ) % 3 );
                 if ( ! ( lane < w ) ) continue;
-                const V3 o{ ks == 0 ? wx[ 0 ] : ks == 1 ? wx[ 1 ] : wx[ 2 ], ks == 0 ? wy[ 0 ] : ks == 1 ? wy[ 1 ] : wy[ 2 ],
-                            ks == 0 ? wz[ 0 ] : ks == 1 ? wz[ 1 ] : wz[ 2 ] };
-                const CellSums d = edge_terms<GAUSS>( P.dn, p0, facets, moments, fid < 0, Av, g, v, o, u );
-                S.part += d.part; S.mass += d.mass; S.mx += d.mx; S.my += d.my; S.mz += d.mz; S.m2 += d.m2;
+                const V3 o{ L.sx[ w ], L.sy[ w ], L.sz[ w ] };
+                const CellSums d = edge_terms<false>( P.dn, p0, facets, moments, false, Av, g, v, o, v );
+                part[ j ] += d.part; S.mass += d.mass; S.mx += d.mx; S.my += d.my; S.mz += d.mz; S.m2 += d.m2;
             }
         }
-        if ( facets && fid >= 0 ) {
-            const double cf = wave_total( S.part ) / ( 2 * dn );
-            if ( lane == 0 && q < P.room ) {
-                P.out.col[ row0 + I64( q ) * 64 ] = fid;
-                P.out.val[ row0 + I64( q ) * 64 ] = cf;
+    }
+    double dia = 0;
+    int nq = 0;
+    if ( facets ) {
+        wave_sync();
+        if ( act ) { L.sx[ lane ] = part[ 0 ]; L.sy[ lane ] = part[ 1 ]; L.sz[ lane ] = part[ 2 ]; }
+        wave_sync();
+        double cf = 0;
+        bool has = false;
+        if ( cnt >= 3 && L.fid[ lane ] >= 0 ) {          // ( `cnt` of a lane past the faces is 0 )
+            double sp = 0;
+            for ( int v = 0; v < c.nv; ++v ) {
+                const int pl = L.spl[ v ];
+                if ( byte_of( pl, 0 ) == lane ) sp += L.sx[ v ];
+                else if ( byte_of( pl, 1 ) == lane ) sp += L.sy[ v ];
+                else if ( byte_of( pl, 2 ) == lane ) sp += L.sz[ v ];
             }
-            dia += cf;
-            ++q;
+            cf = sp / ( 2 * norm );
+            has = true;
         }
+        const unsigned long long mh = __ballot( has );
+        const int q = __popcll( mh & ( ( 1ull << lane ) - 1 ) );
+        nq = __popcll( mh );
+        if ( has && q < P.room ) {
+            P.out.col[ row0 + I64( q ) * 64 ] = L.fid[ lane ];
+            P.out.val[ row0 + I64( q ) * 64 ] = cf;
+        }
+        dia = wave_total( cf );
     }
     S.mass = wave_total( S.mass );
     if ( moments ) { S.mx = wave_total( S.mx ); S.my = wave_total( S.my ); S.mz = wave_total( S.mz ); S.m2 = wave_total( S.m2 ); }
-    if ( lane == 0 ) write_cell( P, k0, p0, S, dia, q, row0 );
+    if ( lane == 0 ) write_cell( P, k0, p0, S, dia, nq, row0 );
 }
 
 template<bool SPLIT>
@@ -786,7 +809,7 @@ __global__ __launch_bounds__( 64 * WAVES3 ) void k_cells3( Params3 P ) {
         if ( lane == 0 ) { P.pb.nv[ k0 ] = status == C3_EMPTY ? 0 : c.nv; P.pb.nf[ k0 ] = c.nf; }
         return;
     }
-    measure_cell<false>( P, LdsFaces{ L }, c, lane, k0, p0, row0 );
+    measure_flat( P, L, c, lane, k0, p0, row0 );
 }
 
 /// what a wave of the measure kernel keeps in LDS: the cell's vertices, its faces ( area centroid, unit normal, the norm of
@@ -803,8 +826,10 @@ struct MeasLds {
 
 /// the second kernel of a sum of Gaussians: the cells the first pass kept, one wave each. The triangles of the cell ( a
 /// face's area centroid and one of its edges, `3 nv` of them ) are spread over the lanes, each face's sums taken in a fixed
-/// order: the same terms as the face-by-face loop of the first pass, with every lane at work
-template<bool IMAGE>
+/// order. For a flux against Gaussians a box face's triangles come in `BOX_SUB^2` parts, a part a lane: on one lane they were 16 rules
+/// while the wave waited, in a quarter of 10k cells ( a diagram 2.04 -> 0.41 ms ). `MOMENTS` is a form of its own for its registers
+enum { MEASURE_FLUX, MEASURE_MOMENTS, MEASURE_IMAGE };
+template<int FORM>
 __global__ __launch_bounds__( 64 * WAVES3 ) void k_cells3_measure( Params3 P ) {
     __shared__ MeasLds lds[ WAVES3 ];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -836,44 +861,62 @@ __global__ __launch_bounds__( 64 * WAVES3 ) void k_cells3_measure( Params3 P ) {
         M.fok[ lane ] = cnt >= 3;
     }
     wave_sync();
-    // the triangles: each edge of a face counted by its lower vertex
+    // the triangles: each edge of a face counted by its lower vertex; the box faces' last ( their count in the upper half )
     int cnt = 0;
     if ( act )
         for ( int j = 0; j < 3; ++j ) {
             const int f = byte_of( pl, j );
             if ( ! M.fok[ f ] ) continue;
-            cnt += int( lane < byte_of( nb, ( j + 1 ) % 3 ) ) + int( lane < byte_of( nb, ( j + 2 ) % 3 ) );
+            const int edges = int( lane < byte_of( nb, ( j + 1 ) % 3 ) ) + int( lane < byte_of( nb, ( j + 2 ) % 3 ) );
+            cnt += M.fid[ f ] < 0 ? edges << 16 : edges;
         }
     int inc = cnt;
     for ( int d = 1; d < 64; d <<= 1 ) {
         const int t = __shfl_up( inc, d, 64 );
         if ( lane >= d ) inc += t;
     }
-    const int T = __shfl( inc, 63, 64 );
+    const int all = __shfl( inc, 63, 64 ), inner = all & 0xffff, T = inner + ( all >> 16 );
     if ( act ) {
-        int t = inc - cnt;
+        int ti = ( inc - cnt ) & 0xffff, tb = inner + ( ( inc - cnt ) >> 16 );
         for ( int j = 0; j < 3; ++j ) {
             const int f = byte_of( pl, j );
             if ( ! M.fok[ f ] ) continue;
             for ( int e = 1; e <= 2; ++e ) {
                 const int w = byte_of( nb, ( j + e ) % 3 );
-                if ( lane < w ) { M.tf[ t ] = f; M.tv[ t ] = lane; M.tw[ t ] = w; ++t; }
+                if ( ! ( lane < w ) ) continue;
+                const int t = M.fid[ f ] < 0 ? tb++ : ti++;
+                M.tf[ t ] = f; M.tv[ t ] = lane; M.tw[ t ] = w;
             }
         }
     }
     wave_sync();
     const bool facets = P.mode == MODE_FACETS, moments = P.mode == MODE_MOMENTS;
     CellSums S;
-    for ( int t = lane; t < T; t += 64 ) {
-        const int f = M.tf[ t ], v = M.tv[ t ], w = M.tw[ t ];
-        const CellSums d = IMAGE ? image_terms( P.dn, p0, facets, moments, Av.x, V3{ M.gx[ f ], M.gy[ f ], M.gz[ f ] },
-                                                V3{ M.px[ v ], M.py[ v ], M.pz[ v ] }, V3{ M.px[ w ], M.py[ w ], M.pz[ w ] },
-                                                V3{ M.ux[ f ], M.uy[ f ], M.uz[ f ] } )
-                                 : edge_terms<true>( P.dn, p0, facets, moments, M.fid[ f ] < 0, Av, V3{ M.gx[ f ], M.gy[ f ], M.gz[ f ] },
-                                             V3{ M.px[ v ], M.py[ v ], M.pz[ v ] }, V3{ M.px[ w ], M.py[ w ], M.pz[ w ] },
-                                             V3{ M.ux[ f ], M.uy[ f ], M.uz[ f ] } );
-        M.tpart[ t ] = d.part;
-        S.mass += d.mass; S.mx += d.mx; S.my += d.my; S.mz += d.mz; S.m2 += d.m2;
+    constexpr int PARTS = FORM == MEASURE_FLUX ? BOX_SUB * BOX_SUB : 1;
+    const int items = inner + PARTS * ( T - inner );
+    for ( int i = lane; i < items; i += 64 ) {
+        const int t = i < inner ? i : inner + ( i - inner ) / PARTS;
+        const int f = M.tf[ t ], a = M.tv[ t ], b = M.tw[ t ];
+        const V3 g{ M.gx[ f ], M.gy[ f ], M.gz[ f ] }, v{ M.px[ a ], M.py[ a ], M.pz[ a ] }, o{ M.px[ b ], M.py[ b ], M.pz[ b ] };
+        const V3 u{ M.ux[ f ], M.uy[ f ], M.uz[ f ] };
+        if ( FORM == MEASURE_FLUX ) {
+            const double ux = v.x - g.x, uy = v.y - g.y, uz = v.z - g.z, tx = o.x - g.x, ty = o.y - g.y, tz = o.z - g.z;
+            const double cx = uy * tz - uz * ty, cy = uz * tx - ux * tz, cz = ux * ty - uy * tx;
+            double ar = 0.5 * sqrt( cx * cx + cy * cy + cz * cz );
+            V3 P0 = g, P1 = v, P2 = o;
+            if ( i >= inner ) {
+                sub_triangle( ( i - inner ) % PARTS, g, v, o, P0, P1, P2 );
+                ar /= PARTS;
+            }
+            double part = 0;
+            gauss_rule7( P.dn, p0, P0, P1, P2, ar, u, part, S.mass );
+            if ( i < inner ) M.tpart[ t ] = part;
+        } else {
+            const CellSums d = FORM == MEASURE_IMAGE ? image_terms( P.dn, p0, facets, moments, Av.x, g, v, o, u )
+                                                     : edge_terms<true>( P.dn, p0, false, true, false, Av, g, v, o, u );
+            M.tpart[ t ] = d.part;
+            S.mass += d.mass; S.mx += d.mx; S.my += d.my; S.mz += d.mz; S.m2 += d.m2;
+        }
     }
     wave_sync();
     // the facets: a face's parts summed in triangle order by its lane, the rows' entries in face order
@@ -882,7 +925,7 @@ __global__ __launch_bounds__( 64 * WAVES3 ) void k_cells3_measure( Params3 P ) {
     bool has = false;
     if ( facets && lane < nf && M.fok[ lane ] && M.fid[ lane ] >= 0 ) {
         double sp = 0;
-        for ( int t = 0; t < T; ++t ) if ( M.tf[ t ] == lane ) sp += M.tpart[ t ];
+        for ( int t = 0; t < inner; ++t ) if ( M.tf[ t ] == lane ) sp += M.tpart[ t ];
         cf = sp / ( 2 * M.dn[ lane ] );
         has = true;
     }
@@ -1230,8 +1273,10 @@ void run_cells_3d( const DevTree3 &t, const double *lo, const double *hi, const 
         P.pb.nv = A.get<int>( "cells3.nv", size_t( t.n ) ); P.pb.nf = A.get<int>( "cells3.nf", size_t( t.n ) );
         k_cells3<true><<<blocks_for( t.n, WAVES3 ), 64 * WAVES3, 0, st>>>( P );
         check_launch( "k_cells3" );
-        if ( dn.kind == 1 ) k_cells3_measure<true><<<blocks_for( t.n, WAVES3 ), 64 * WAVES3, 0, st>>>( P );
-        else                k_cells3_measure<false><<<blocks_for( t.n, WAVES3 ), 64 * WAVES3, 0, st>>>( P );
+        const unsigned blocks = blocks_for( t.n, WAVES3 );
+        if ( dn.kind == 1 )              k_cells3_measure<MEASURE_IMAGE><<<blocks, 64 * WAVES3, 0, st>>>( P );
+        else if ( mode == MODE_MOMENTS ) k_cells3_measure<MEASURE_MOMENTS><<<blocks, 64 * WAVES3, 0, st>>>( P );
+        else                             k_cells3_measure<MEASURE_FLUX><<<blocks, 64 * WAVES3, 0, st>>>( P );
         check_launch( "k_cells3_measure" );
     } else {
         k_cells3<false><<<blocks_for( t.n, WAVES3 ), 64 * WAVES3, 0, st>>>( P );
