@@ -50,7 +50,6 @@ struct WaveLds {
     int    fid[ CELL3_FACES ];
     double sx[ CELL3_VERTICES ], sy[ CELL3_VERTICES ], sz[ CELL3_VERTICES ];
     int    spl[ CELL3_VERTICES ], snb[ CELL3_VERTICES ];
-    int    np1[ CELL3_VERTICES ], np2[ CELL3_VERTICES ];
     int    stk_m[ STACK3 ], stk_h[ STACK3 ];
     int    used[ CELL3_FACES ];
 };
@@ -488,16 +487,30 @@ __device__ void compact_faces( WaveLds &L, Cell3 &c, int lane ) {
     c.nf = __popcll( mu );
 }
 
-/// the cut by `n . v <= off` ( face id `id` ), the oracle's `cut3` with the lanes of a wave
-__device__ int cut_cell( WaveLds &L, Cell3 &c, int lane, double nx, double ny, double nz, double off, int id, unsigned long long &ev_side,
-                         unsigned long long &ev_new ) {
+/// a bound of the coordinates of the cell's vertices from its seed: the cuts only take from the box, a new vertex lies between two others up to
+/// the rounding of its `fma`
+__device__ __forceinline__ double box_bound( const Params3 &P, const double4 &p0 ) {
+    const double x = fmax( fabs( P.hi[ 0 ] - p0.x ), fabs( P.lo[ 0 ] - p0.x ) ), y = fmax( fabs( P.hi[ 1 ] - p0.y ), fabs( P.lo[ 1 ] - p0.y ) );
+    return 1.0000001 * fmax( fmax( x, y ), fmax( fabs( P.hi[ 2 ] - p0.z ), fabs( P.lo[ 2 ] - p0.z ) ) );
+}
+
+/// the cut by `n . v <= off` ( face id `id` ), the oracle's `cut3` with the lanes of a wave. A cell has ~32 of them, a chain of dependent
+/// steps across lanes that bounds the kernel: the tie bound takes `vm_bound`, a bound of the vertices' coordinates, and their largest
+/// only where a vertex is that near the plane; the crossings' scan is two ballots; the new face's edges meet in a table of
+/// faces. ( As three wave-wide reductions and scans and a loop over the new vertices: 300k cells 20.4 ms, 17.3 so )
+__device__ int cut_cell( WaveLds &L, Cell3 &c, int lane, double vm_bound, double nx, double ny, double nz, double off, int id,
+                         unsigned long long &ev_side, unsigned long long &ev_new ) {
     const bool act = lane < c.nv;
     double s = act ? fma( nx, c.x, fma( ny, c.y, fma( nz, c.z, -off ) ) ) : -1.0;
     ev_side += unsigned( c.nv );
     if ( __ballot( s > 0 ) == 0 ) return C3_UNCHANGED;
     // a vertex on the plane up to the rounding of `s` stays inside ( where more than three planes meet )
-    const double vm = wave_maxd( act ? fmax( fabs( c.x ), fmax( fabs( c.y ), fabs( c.z ) ) ) : 0.0 );
-    const double tie = 1e-13 * ( ( fabs( nx ) + fabs( ny ) + fabs( nz ) ) * vm + fabs( off ) );
+    const double n1a = fabs( nx ) + fabs( ny ) + fabs( nz );
+    double tie = 1e-13 * ( n1a * vm_bound + fabs( off ) );
+    if ( __ballot( s > 0 && s <= tie ) ) {               // ( else no bound below this one parts the vertices otherwise )
+        const double vm = wave_maxd( act ? fmax( fabs( c.x ), fmax( fabs( c.y ), fabs( c.z ) ) ) : 0.0 );
+        tie = 1e-13 * ( n1a * vm + fabs( off ) );
+    }
     const bool out = act && s > tie;
     if ( ! out ) s = fmin( s, 0.0 );
     const unsigned long long mo = __ballot( out );
@@ -509,16 +522,13 @@ __device__ int cut_cell( WaveLds &L, Cell3 &c, int lane, double nx, double ny, d
     if ( c.nf >= CELL3_FACES ) return C3_FULL;
     const int n0 = byte_of( c.nb, 0 ), n1 = byte_of( c.nb, 1 ), n2 = byte_of( c.nb, 2 );
     const int cnt = out ? int( ( mi >> n0 ) & 1 ) + int( ( mi >> n1 ) & 1 ) + int( ( mi >> n2 ) & 1 ) : 0;
-    int inc = cnt;
-    for ( int d = 1; d < 64; d <<= 1 ) {
-        const int t = __shfl_up( inc, d, 64 );
-        if ( lane >= d ) inc += t;
-    }
-    const int excl = inc - cnt, T = __shfl( inc, 63, 64 ), nin = __popcll( mi );
+    const unsigned long long c0 = __ballot( cnt & 1 ), c1 = __ballot( cnt & 2 ), before = ( 1ull << lane ) - 1;
+    const int excl = __popcll( c0 & before ) + 2 * __popcll( c1 & before ), T = __popcll( c0 ) + 2 * __popcll( c1 ), nin = __popcll( mi );
     if ( nin + T > CELL3_VERTICES ) return C3_FULL;
     const int fn = c.nf;
     wave_sync();
     if ( lane == 0 ) { L.fx[ fn ] = nx; L.fy[ fn ] = ny; L.fz[ fn ] = nz; L.fo[ fn ] = off; L.fid[ fn ] = id; }
+    L.used[ lane ] = 0;                                  // ( the faces' new vertices: their count, and the sum of their numbers )
     // the neighbours' positions, signs, neighbour lists and scan offsets ( every lane shuffles: no lane is masked )
     double ax[ 3 ], ay[ 3 ], az[ 3 ], as[ 3 ];
     int bn[ 3 ], bex[ 3 ];
@@ -530,6 +540,7 @@ __device__ int cut_cell( WaveLds &L, Cell3 &c, int lane, double nx, double ny, d
         bn[ k ] = __shfl( c.nb, nk[ k ], 64 );
         bex[ k ] = __shfl( excl, nk[ k ], 64 );
     }
+    wave_sync();
     if ( out ) {                                         // the new vertices of this outside vertex's crossing edges
         int j = 0;
 #pragma unroll
@@ -544,8 +555,9 @@ __device__ int cut_cell( WaveLds &L, Cell3 &c, int lane, double nx, double ny, d
             const int p1 = byte_of( c.pl, ( k + 1 ) % 3 ), p2 = byte_of( c.pl, ( k + 2 ) % 3 );
             L.spl[ g ] = fn | ( p1 << 8 ) | ( p2 << 16 );
             L.snb[ g ] = __popcll( mi & ( ( 1ull << a ) - 1 ) );
-            L.np1[ g - nin ] = p1;
-            L.np2[ g - nin ] = p2;
+            const int mark = ( 1 << 16 ) + g;
+            atomicAdd( &L.used[ p1 ], mark );
+            atomicAdd( &L.used[ p2 ], mark );
         }
     } else if ( act ) {                                  // an inside vertex: its slot and its neighbours renumbered
         const int ia = __popcll( mi & ( ( 1ull << lane ) - 1 ) );
@@ -578,15 +590,9 @@ __device__ int cut_cell( WaveLds &L, Cell3 &c, int lane, double nx, double ny, d
     if ( lane < nin + T ) {
         nbv = L.snb[ lane ];
         if ( lane >= nin ) {
-            const int t0 = lane - nin, p1 = L.np1[ t0 ], p2 = L.np2[ t0 ];
-            int m1 = 0, m2 = 0, c1 = 0, c2 = 0;
-            for ( int t = 0; t < T; ++t ) {
-                if ( t == t0 ) continue;
-                const int q1 = L.np1[ t ], q2 = L.np2[ t ];
-                if ( q1 == p2 || q2 == p2 ) { m1 = nin + t; ++c1; }
-                if ( q1 == p1 || q2 == p1 ) { m2 = nin + t; ++c2; }
-            }
-            broken = c1 != 1 || c2 != 1;
+            const int pl = L.spl[ lane ], q1 = L.used[ byte_of( pl, 1 ) ], q2 = L.used[ byte_of( pl, 2 ) ];
+            const int m1 = ( q2 & 0xffff ) - lane, m2 = ( q1 & 0xffff ) - lane;
+            broken = q1 >> 16 != 2 || q2 >> 16 != 2;
             nbv = ( nbv & 255 ) | ( m1 << 8 ) | ( m2 << 16 );
         }
     }
@@ -727,6 +733,7 @@ __global__ __launch_bounds__( 64 * WAVES3 ) void k_cells3( Params3 P ) {
             L.fid[ lane ] = hi ? -2 - 2 * d : -1 - 2 * d;
         }
     }
+    const double vm_bound = box_bound( P, p0 );
     int status = C3_CUT;
     // the walk: nearest child first, a node pruned when no vertex can be cut by a seed under its majorant
     int top = 0;
@@ -765,7 +772,7 @@ __global__ __launch_bounds__( 64 * WAVES3 ) void k_cells3( Params3 P ) {
                     if ( k == k0 ) continue;
                     const double dx = readlane_d( sq.x, j ) - p0.x, dy = readlane_d( sq.y, j ) - p0.y, dz = readlane_d( sq.z, j ) - p0.z;
                     const double off = ( ( w0 - readlane_d( sq.w, j ) ) + ( dx * dx + dy * dy + dz * dz ) ) / 2;
-                    const int res = cut_cell( L, c, lane, dx, dy, dz, off, k, ev_side, ev_new );
+                    const int res = cut_cell( L, c, lane, vm_bound, dx, dy, dz, off, k, ev_side, ev_new );
                     if ( res == C3_CUT ) ++ev_cut;
                     if ( res == C3_EMPTY || res == C3_FAILED || res == C3_FULL ) { status = res; break; }
                 }
@@ -953,33 +960,38 @@ struct Slot3 {
     double x[ SLOT_V ], y[ SLOT_V ], z[ SLOT_V ], s[ SLOT_V ];
     int    pl[ 3 * SLOT_V ], nb[ 3 * SLOT_V ];
     double X[ SLOT_V ], Y[ SLOT_V ], Z[ SLOT_V ];
-    int    PL[ 3 * SLOT_V ], NB[ 3 * SLOT_V ], idx[ SLOT_V ], np1[ SLOT_V ], np2[ SLOT_V ];
+    int    PL[ 3 * SLOT_V ], NB[ 3 * SLOT_V ], idx[ SLOT_V ];
     double fx[ SLOT_F ], fy[ SLOT_F ], fz[ SLOT_F ], fo[ SLOT_F ];
     int    fid[ SLOT_F ];
     int    stk_m[ STACK3 ], stk_h[ STACK3 ];
     int    tf[ 3 * SLOT_V ], tv[ 3 * SLOT_V ], tw[ 3 * SLOT_V ];   ///< the measures' triangles ( face, vertices ), `3 nv` at most
     double tp[ 3 * SLOT_V ];                                       ///< their facet parts
-    int    nv, nf, res;
+    int    nv, nf;
 };
+static_assert( SLOT_F <= 3 * SLOT_V, "a cut's table of faces lies in the triangles' room" );
 
 /// the cut of an overflowed cell by its wave, the oracle's `cut3` step by step with a lane a vertex ( `SLOT_V / 64` each ): the signs, the
 /// classification with the tie bound, the inside vertices renumbered, a new vertex per crossing edge in the order ( outside
 /// vertex, edge ), the new face closed, the cell copied back. ( One lane alone took ~40 us a cut of 70 vertices, 1.4 ms a cell. )
-__device__ int cut_slot( Slot3 &C, int lane, double nx, double ny, double nz, double off, int id, unsigned long long &ev_side,
+__device__ int cut_slot( Slot3 &C, int lane, double vm_bound, double nx, double ny, double nz, double off, int id, unsigned long long &ev_side,
                          unsigned long long &ev_new ) {
     const int nv = C.nv, fn = C.nf;
     ev_side += unsigned( nv );
-    bool any = false;
-    double vm = 0;
+    const double n1a = fabs( nx ) + fabs( ny ) + fabs( nz );
+    double tie = 1e-13 * ( n1a * vm_bound + fabs( off ) );
+    bool any = false, near = false;
     for ( int v = lane; v < nv; v += 64 ) {
         const double sv = fma( nx, C.x[ v ], fma( ny, C.y[ v ], fma( nz, C.z[ v ], -off ) ) );
         C.s[ v ] = sv;
         any |= sv > 0;
-        vm = fmax( vm, fmax( fabs( C.x[ v ] ), fmax( fabs( C.y[ v ] ), fabs( C.z[ v ] ) ) ) );
+        near |= sv > 0 && sv <= tie;
     }
     if ( __ballot( any ) == 0 ) return C3_UNCHANGED;
-    vm = wave_maxd( vm );
-    const double tie = 1e-13 * ( ( fabs( nx ) + fabs( ny ) + fabs( nz ) ) * vm + fabs( off ) );
+    if ( __ballot( near ) ) {                            // ( the vertices' own largest coordinate, as in `cut_cell` )
+        double vm = 0;
+        for ( int v = lane; v < nv; v += 64 ) vm = fmax( vm, fmax( fabs( C.x[ v ] ), fmax( fabs( C.y[ v ] ), fabs( C.z[ v ] ) ) ) );
+        tie = 1e-13 * ( n1a * wave_maxd( vm ) + fabs( off ) );
+    }
     const unsigned long long before = ( 1ull << lane ) - 1;
     int nin = 0;
     for ( int v0 = 0; v0 < nv; v0 += 64 ) {              // ( each lane on its own vertices' signs )
@@ -996,6 +1008,7 @@ __device__ int cut_slot( Slot3 &C, int lane, double nx, double ny, double nz, do
     if ( nin == 0 ) return C3_EMPTY;
     if ( fn >= SLOT_F ) return C3_FULL;
     __syncthreads();                                     // ( the block is the wave )
+    for ( int f = lane; f < fn; f += 64 ) C.tf[ f ] = 0; // ( the faces' new vertices: their count, and the sum of their numbers )
     for ( int v = lane; v < nv; v += 64 ) {              // the inside vertices, their neighbours renumbered
         const int i = C.idx[ v ];
         if ( i < 0 ) continue;
@@ -1009,11 +1022,10 @@ __device__ int cut_slot( Slot3 &C, int lane, double nx, double ny, double nz, do
         const bool out = b < nv && C.idx[ b ] < 0;
         int cnt = 0;
         if ( out ) for ( int k = 0; k < 3; ++k ) cnt += C.idx[ C.nb[ 3 * b + k ] ] >= 0;
-        int inc = cnt;
-        for ( int d = 1; d < 64; d <<= 1 ) { const int t = __shfl_up( inc, d, 64 ); if ( lane >= d ) inc += t; }
-        const int all = __shfl( inc, 63, 64 );
+        const unsigned long long c0 = __ballot( cnt & 1 ), c1 = __ballot( cnt & 2 );
+        const int all = __popcll( c0 ) + 2 * __popcll( c1 );
         if ( nin + T + all > SLOT_V ) return C3_FULL;
-        int at = T + inc - cnt;
+        int at = T + __popcll( c0 & before ) + 2 * __popcll( c1 & before );
         if ( out )
             for ( int k = 0; k < 3; ++k ) {
                 const int a = C.nb[ 3 * b + k ], ia = C.idx[ a ];
@@ -1026,7 +1038,9 @@ __device__ int cut_slot( Slot3 &C, int lane, double nx, double ny, double nz, do
                 const int p1 = C.pl[ 3 * b + ( k + 1 ) % 3 ], p2 = C.pl[ 3 * b + ( k + 2 ) % 3 ];
                 C.PL[ 3 * g ] = fn; C.PL[ 3 * g + 1 ] = p1; C.PL[ 3 * g + 2 ] = p2;
                 C.NB[ 3 * g ] = ia;
-                C.np1[ at ] = p1; C.np2[ at ] = p2;
+                const int mark = ( 1 << 16 ) + g;
+                atomicAdd( &C.tf[ p1 ], mark );
+                atomicAdd( &C.tf[ p2 ], mark );
                 for ( int j = 0; j < 3; ++j )
                     if ( C.nb[ 3 * a + j ] == b ) C.NB[ 3 * ia + j ] = g;
                 ++at;
@@ -1035,17 +1049,11 @@ __device__ int cut_slot( Slot3 &C, int lane, double nx, double ny, double nz, do
     }
     __syncthreads();
     bool open = false;
-    for ( int t0 = lane; t0 < T; t0 += 64 ) {            // the new face closed
-        const int p1 = C.np1[ t0 ], p2 = C.np2[ t0 ];
-        int m1 = 0, m2 = 0, c1 = 0, c2 = 0;
-        for ( int t = 0; t < T; ++t ) {
-            if ( t == t0 ) continue;
-            if ( C.np1[ t ] == p2 || C.np2[ t ] == p2 ) { m1 = nin + t; ++c1; }
-            if ( C.np1[ t ] == p1 || C.np2[ t ] == p1 ) { m2 = nin + t; ++c2; }
-        }
-        open |= c1 != 1 || c2 != 1;
-        C.NB[ 3 * ( nin + t0 ) + 1 ] = m1;
-        C.NB[ 3 * ( nin + t0 ) + 2 ] = m2;
+    for ( int g = nin + lane; g < nin + T; g += 64 ) {   // the new face closed
+        const int q1 = C.tf[ C.PL[ 3 * g + 1 ] ], q2 = C.tf[ C.PL[ 3 * g + 2 ] ];
+        open |= q1 >> 16 != 2 || q2 >> 16 != 2;
+        C.NB[ 3 * g + 1 ] = ( q2 & 0xffff ) - g;
+        C.NB[ 3 * g + 2 ] = ( q1 & 0xffff ) - g;
     }
     if ( __any( open ) ) return C3_FAILED;
     __syncthreads();
@@ -1074,6 +1082,7 @@ __global__ __launch_bounds__( 64 ) void k_cells3_pass2( Params3 P ) {
         const int k0 = P.out.ovf_list[ it ];
         const double4 p0 = P.seeds[ k0 ];
         const double w0 = p0.w;
+        const double vm_bound = box_bound( P, p0 );
         unsigned long long ev_side = 0, ev_new = 0;
         __syncthreads();
         if ( lane < 8 ) {
@@ -1123,7 +1132,7 @@ __global__ __launch_bounds__( 64 ) void k_cells3_pass2( Params3 P ) {
                     const double4 q = P.seeds[ k ];
                     const double dx = q.x - p0.x, dy = q.y - p0.y, dz = q.z - p0.z;
                     const double off = ( ( w0 - q.w ) + ( dx * dx + dy * dy + dz * dz ) ) / 2;
-                    const int res = cut_slot( C, lane, dx, dy, dz, off, k, ev_side, ev_new );
+                    const int res = cut_slot( C, lane, vm_bound, dx, dy, dz, off, k, ev_side, ev_new );
                     if ( res == C3_EMPTY || res == C3_FAILED || res == C3_FULL ) { status = res; break; }
                 }
                 continue;
