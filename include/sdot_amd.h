@@ -49,7 +49,8 @@ void        sdot_amd_release( void );
  * `sdot_amd_kernel_times` returns, per index, the summed milliseconds and the launches timed, the
  * algorithmic bytes of the timed SpMV launches, and the cell kernels' event counters summed over every
  * diagram since the last reset ( HOST [ 5 ]: side tests, pruning vertex tests, new vertices, node
- * visits, cuts ); `reset` clears them afterwards. */
+ * visits, cuts ); `reset` clears them afterwards. In 2D these are the counts of the walk as solves run it, whose majorants prune more
+ * than the reference's; an entry point that is asked for `events` counts the walk under the reference's. */
 int sdot_amd_set_timing( int on );
 int sdot_amd_kernel_times( double *ms, long long *launches, double *spmv_bytes, unsigned long long *events, int reset );
 
@@ -386,6 +387,13 @@ int sdot_amd_build_tree_2d( void *stream, long long n, const double *positions, 
                             long long *seed_indices, long long *rank_of, long long *node_begin, long long *node_end,
                             long long *node_left, long long *node_right, double *node_box );
 
+/* WHETHER TWO ROWS OF A CLOUD MAY BE EQUAL: `*found` = 1 when two 64-bit prints of the rows' bits ( `-0.0` as `0.0` ) are equal, 0 when the
+ * cloud surely has no exact duplicate ( the first step of the search of `src/sdot/SdotPlanNd.py:124-155` ). Returns at once; the
+ * answer is there when the stream has run.
+ *   positions DEVICE [ n ][ dim ], table DEVICE [ slots ] ( scratch; a power of two, at least 2 n ), found DEVICE [ 1 ] */
+int sdot_amd_equal_prints( void *stream, long long n, int dim, const double *positions, unsigned long long *table, long long slots,
+                           int *found );
+
 /* THE MAJORANTS: for every node of a tree built as above, `( wa, wb )` with `w_k <= wa . p_k + wb` on
  * its seeds ( affine least-squares fit kept when it tightens the spread, else constant ).
  * Replaces `bsp_refresh_majorants_card_2d` -> `sdot::gpu2d::refresh_majorants`
@@ -405,7 +413,8 @@ int sdot_amd_refresh_majorants_2d( void *stream, long long n, long long nb_nodes
  * Replaces `sdotplan_card_linear_2d` -> `sdot::gpu2d::linear_solves`
  * ( src/sdot/include/sdot/gpu/Newton2D.cuh:1916, called from src/sdot/SdotPlanNd.py:204-236 ).
  *   row DEVICE [ n + 1 ] int64, col DEVICE [ nnz ] int64, val DEVICE [ nnz ], dia DEVICE [ n ]
- *   rhs DEVICE [ k ][ n ], options HOST [ 10 ] ( n, k, method, tol, ... as the reference; tol used )
+ *   rhs DEVICE [ k ][ n ], options HOST [ 10 ] ( n, k, method, tol, ... as the reference; with method 1, options[ 4 ] = 1 takes the
+ *       smoothed-aggregation V-cycle, options[ 5 ] = 1 its levels in FP32 )
  *   solution DEVICE [ k ][ n ] ( output ), iterations HOST [ k ] ( output, -1: failed )
  */
 int sdot_amd_linear_solves_2d( void *stream, long long n, const long long *row, const long long *col, const double *val,

@@ -163,6 +163,37 @@ void preorder_tables( int depth, std::vector<int> &pre, std::vector<int> &height
         for ( I64 i = ( I64( 1 ) << level ) - 1; i < ( I64( 1 ) << ( level + 1 ) ) - 1; ++i ) height[ size_t( pre[ size_t( i ) ] ) ] = depth - level;
 }
 
+/// splitmix64's finalizer ( a bijection )
+__device__ __forceinline__ unsigned long long mix64( unsigned long long z ) {
+    z = ( z ^ ( z >> 30 ) ) * 0xBF58476D1CE4E5B9ull;
+    z = ( z ^ ( z >> 27 ) ) * 0x94D049BB133111EBull;
+    return z ^ ( z >> 31 );
+}
+
+__global__ void k_clear_prints( I64 slots, unsigned long long *table, int *found ) {
+    const I64 i = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
+    if ( i < slots ) table[ i ] = 0;
+    if ( i == 0 ) *found = 0;
+}
+
+/// each row's 64-bit print into a table at most half full ( linear probing, 0 an empty slot ); `found` when two rows have the same. Bound
+/// by the table's scattered atomics. ( Prints of 1M rows sorted on the host instead, with the copy to it: ~45 ms a solve )
+__global__ void k_insert_prints( I64 n, int dim, const double *pos, unsigned long long *table, I64 mask, int *found ) {
+    const I64 i = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
+    if ( i >= n || *static_cast<volatile int *>( found ) ) return;
+    unsigned long long h = 0;
+    for ( int d = 0; d < dim; ++d ) {
+        const double x = pos[ i * dim + d ];
+        h = mix64( h ^ static_cast<unsigned long long>( __double_as_longlong( x == 0 ? 0.0 : x ) ) );   // ( -0.0 as 0.0 )
+    }
+    const unsigned long long key = h ? h : 1;
+    for ( I64 probe = 0; probe <= mask; ++probe ) {
+        const unsigned long long was = atomicCAS( &table[ ( I64( h ) + probe ) & mask ], 0ull, key );
+        if ( was == 0 ) return;
+        if ( was == key ) { *found = 1; return; }
+    }
+}
+
 __global__ void k_i32_to_i64( I64 n, const int *a, long long *b ) {
     const I64 i = I64( blockIdx.x ) * blockDim.x + threadIdx.x;
     if ( i < n ) b[ i ] = a[ i ];
@@ -787,6 +818,17 @@ int sdot_amd_build_tree_2d( void *stream, long long n, const double *positions, 
         if ( node_right ) SDOT_HIP( hipMemcpyAsync( node_right, rgt.data(), sizeof( long long ) * size_t( N ), hipMemcpyHostToDevice, st ) );
         if ( node_box ) SDOT_HIP( hipMemcpyAsync( node_box, t.node_box, sizeof( double ) * size_t( N ) * 4, hipMemcpyDeviceToDevice, st ) );
         SDOT_HIP( hipStreamSynchronize( st ) );
+    } );
+}
+
+int sdot_amd_equal_prints( void *stream, long long n, int dim, const double *positions, unsigned long long *table, long long slots, int *found ) {
+    return guarded( [&] {
+        SDOT_CHECK( n >= 1 && dim >= 1 && positions && table && found, "equal_prints: n >= 1, dim >= 1 and the arrays are required" );
+        SDOT_CHECK( slots >= 2 * n && ( slots & ( slots - 1 ) ) == 0, "equal_prints: the table's slots are a power of two, at least 2 n" );
+        hipStream_t st = hipStream_t( stream );
+        k_clear_prints<<<blocks_for( slots, 256 ), 256, 0, st>>>( slots, table, found );
+        k_insert_prints<<<blocks_for( n, 256 ), 256, 0, st>>>( n, dim, positions, table, slots - 1, found );
+        check_launch( "k_insert_prints" );
     } );
 }
 

@@ -5,7 +5,7 @@
 
 namespace sdot_amd {
 
-/// the largest cloud the fixed scratch serves, and the scratch's size per GPU ( the tree and its build ~165 B a seed, the
+/// the largest cloud the fixed scratch serves, and the scratch's size per GPU ( the tree and its build ~185 B a seed, the
 /// rank-order masses, overflow lists and zero weights ~24 B a seed, the overflow slots of `NOALLOC_OVF_LANES` lanes ~2.6 MB,
 /// with room to spare )
 constexpr I64    NOALLOC_MAX_SEEDS = I64( 1 ) << 17;

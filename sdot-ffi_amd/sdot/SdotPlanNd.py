@@ -45,10 +45,13 @@ def exact_duplicates( positions ):
     """THE EXACT DUPLICATES of a cloud `[ n, d ]`: `( dup, rep )`, each seed whose position an earlier one already holds and
     the smallest index at that position, both increasing with `dup` ( empty `int64` arrays when there is none; `-0.0` and
     `0.0` alike ). Reference `src/sdot/SdotPlanNd.py:124-155`. A 64-bit print of each row's bits, sorted: when no two prints
-    are equal there is no duplicate; otherwise the rows whose prints collide are grouped exactly."""
+    are equal there is no duplicate; otherwise the rows whose prints collide are grouped exactly. A cloud on the device has its
+    prints compared there, and comes to the host only when two are equal."""
+    none = ( np.zeros( 0, dtype = np.int64 ), np.zeros( 0, dtype = np.int64 ) )
+    if getattr( positions, "is_cuda", False ) and positions.numel() > 0 and not _native.equal_prints( positions ):
+        return none
     P = np.ascontiguousarray( _host( positions ), dtype = np.float64 )
     n = P.shape[ 0 ]
-    none = ( np.zeros( 0, dtype = np.int64 ), np.zeros( 0, dtype = np.int64 ) )
     if n < 2:
         return none
     P = P.reshape( n, -1 ) + 0.0

@@ -28,7 +28,7 @@ CARD_OPTIONS = [ "tol_abs", "tol_rel", "t_min", "mult_ok", "factor", "maxit", "m
 #: what the library exports ( every symbol of `include/sdot_amd.h` )
 EXPORTS = [ "sdot_amd_abi_version", "sdot_amd_last_error", "sdot_amd_device_bytes", "sdot_amd_release", "sdot_amd_set_timing",
             "sdot_amd_kernel_times", "sdot_amd_measures_2d",
-            "sdot_amd_solve_2d", "sdot_amd_tree_nodes", "sdot_amd_build_tree_2d", "sdot_amd_refresh_majorants_2d",
+            "sdot_amd_solve_2d", "sdot_amd_tree_nodes", "sdot_amd_build_tree_2d", "sdot_amd_equal_prints", "sdot_amd_refresh_majorants_2d",
             "sdot_amd_linear_solves_2d", "sdot_amd_solve_2d_batch", "sdot_amd_server_start", "sdot_amd_server_submit",
             "sdot_amd_server_wait", "sdot_amd_server_stop", "sdot_amd_measures_3d", "sdot_amd_solve_3d",
             "sdot_amd_solve_2d_precision", "sdot_amd_graph_counts", "sdot_amd_solve_bytes", "sdot_amd_server_submit_nd", "sdot_amd_server_info",
@@ -96,6 +96,8 @@ def lib():
         L.sdot_amd_solve_2d_precision.argtypes = [ _P, _LL, _P, _P, _P, _P, _LL, _P, _P, _I, _D, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I ]
         L.sdot_amd_solve_2d_domain.argtypes = [ _P, _LL, _P, _P, _P, _P, _LL, _P, _P, _I, _D, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P ]
         L.sdot_amd_solve_2d_domain.restype = _I
+        L.sdot_amd_equal_prints.argtypes = [ _P, _LL, _I, _P, _P, _LL, _P ]
+        L.sdot_amd_equal_prints.restype = _I
         L.sdot_amd_build_tree_2d.argtypes = [ _P, _LL, _P, _I, _P, _P, _P, _P, _P, _P, _P ]
         L.sdot_amd_refresh_majorants_2d.argtypes = [ _P, _LL, _LL, _P, _P, _P, _P, _P, _P, _P ]
         L.sdot_amd_linear_solves_2d.argtypes = [ _P, _LL, _P, _P, _P, _P, _P, _LL, _P, _P, _P ]
@@ -491,6 +493,20 @@ def solve_2d_batch( instances, options, streams = 8, precision = 0 ):
         out.append( dict( weights = weights[ a:b ], cell_masses = masses[ a:b ], barycenters = bary[ a:b ], stats = stats[ i ],
                           cost = float( costs[ i ] ), error = tuple( int( v ) for v in errors[ i ] ), times = tuple( times[ i ] ) ) )
     return out
+
+
+def equal_prints( positions ):
+    """whether two rows of `positions[ n, d ]` ( a device tensor ) have the same 64-bit print; not: the rows are all different"""
+    T = torch()
+    pos = on_device( positions )
+    pos = pos.reshape( pos.shape[ 0 ], -1 )
+    n, slots = pos.shape[ 0 ], 2
+    while slots < 2 * n:
+        slots *= 2
+    table = T.empty( slots, dtype = T.int64, device = device() )
+    found = T.empty( 1, dtype = T.int32, device = device() )
+    _check( lib().sdot_amd_equal_prints( _stream(), n, pos.shape[ 1 ], _ptr( pos ), _ptr( table ), slots, _ptr( found ) ) )
+    return bool( found.item() )
 
 
 def build_tree_2d( positions, leaf = 10 ):
