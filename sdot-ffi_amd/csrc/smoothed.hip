@@ -10,8 +10,8 @@
 //   * `P = ( I - 2/3 D^-1 A ) P0`, a row's entries below 0.1 of its largest dropped ( 0.2 where rows are long, in 3D: there the
 //     coarse rows would grow past 100 entries ), the rest scaled to a unit sum ( `k_prolongator` ); the restriction is `P^T`,
 //     listed per coarse row in increasing order of the fine rows;
-//   * the Galerkin row `P^T A P` by one wave: its columns found by an LDS hash, each column's sum then taken by ONE lane over the
-//     terms in their fixed order, so the result does not depend on the hash's races ( `k_galerkin` );
+//   * the Galerkin row `P^T A P` by one wave: its columns found by an LDS hash, each column's sum taken in whole numbers of
+//     a bound's 2^-57, so the result does not depend on the hash's races ( `k_galerkin` );
 //   * two damped Jacobi sweeps before ( from zero: one pass ) and after, Chebyshev dampings; the correction scaled by 1.2, which
 //     saves 10 % of the iterations ( 1.15 to 1.45 measured alike ), as truncated prolongations under-correct;
 //   * THE BOTTOM: the first level of at most 2048 rows is one product with a dense operator, the V-cycle over the levels below
@@ -259,92 +259,69 @@ __device__ __forceinline__ int sorted_list( I64 I, I64 nf, const int *pn, const 
 }
 
 /// THE GALERKIN ROWS, one wave a coarse row ( see the file's header ): the terms `P_iI a_ij P_jK` of the fine rows `i` of its list, eight
-/// lanes a fine row, staged in LDS with their column's number ( an LDS hash of the columns met so far, room for at most `SA_SMAX + 1` );
-/// then each lane adds up the terms of its own columns in the staged order, four terms a read ( one at a time, the loop waited out
-/// an LDS latency a term: 1M rows 5.0 -> 1.9 ms a hierarchy ). `state[ S_BAD ]` when a list or a row outgrows its room
+/// lanes a fine row, added in LDS at their column's place in a hash of the columns met ( at most `SA_SMAX + 1` ). The sums are 64-bit
+/// whole numbers of `2^-57` of a bound of the row's terms ( `P`'s rows sum to 1, a row of `A` to at most twice its diagonal: there are four
+/// bits for what is off this ), so that the atomics' order does not matter: the row is the same in every run, and each sum is within
+/// `2^-58` of the bound a term, where a sum in double rounds by `2^-53` of itself. `state[ S_BAD ]` when a list or a row outgrows its room.
+/// ( Terms staged in LDS and added up by their column's lane, every lane looking at every term: 1M rows 2.05 ms a hierarchy, 0.90 so )
 template<class P>
 __global__ __launch_bounds__( 64 ) void k_galerkin( Rows<P> A, const int *pn, const int *pcol, const P *pval, int *tn, int *tcol, P *tval, int room,
                                                    int *ccnt, int *ccol, P *cval, P *cdia, P *cdinv, double *state ) {
-    __shared__ int si[ SA_TMAX ], hk[ SA_HASH ], hi[ SA_HASH ], ck[ SA_SMAX + 1 ], nkeys;
-    __shared__ __attribute__(( aligned( 16 ) )) int ti[ 64 * SA_PMAX + 4 ];
-    __shared__ __attribute__(( aligned( 16 ) )) double tv[ 64 * SA_PMAX + 4 ];
+    __shared__ unsigned long long sum[ SA_HASH ];
     __shared__ double sw[ SA_TMAX ];
+    __shared__ int raw[ SA_TMAX ], si[ SA_TMAX ], hk[ SA_HASH ], ck[ SA_SMAX + 1 ], at[ SA_SMAX + 1 ], nkeys;
     const int lane = threadIdx.x;
     const I64 I = xcd_block();
     const bool over = tn[ I ] > SA_TMAX;
-    for ( int h = lane; h < SA_HASH; h += 64 ) hk[ h ] = -1;
+    for ( int h = lane; h < SA_HASH; h += 64 ) { hk[ h ] = -1; sum[ h ] = 0; }
     if ( lane == 0 ) nkeys = 0;
-    const int cnt = sorted_list( I, A.n, pn, pcol, pval, tn, tcol, tval, ti, si, sw );
-    double acc[ 4 ] = { 0, 0, 0, 0 };
+    const int cnt = sorted_list( I, A.n, pn, pcol, pval, tn, tcol, tval, raw, si, sw );
+    double bound = 0;
+    for ( int k = lane; k < cnt; k += 64 ) bound += 2 * fabs( sw[ k ] * double( A.dia[ si[ k ] ] ) );
+    for ( int o = 32; o; o >>= 1 ) bound += __shfl_xor( bound, o, 64 );
+    const int ex = bound > 0 && bound < 1e300 ? ilogb( bound ) + 1 : 0;
+    const double scale = ldexp( 1.0, 57 - ex ), unit = ldexp( 1.0, ex - 57 );
     const int g = lane >> 3, sub = lane & 7;
-    for ( int base = 0; base < cnt; base += 8 ) {
-        const bool valid = base + g < cnt;
-        const int i = valid ? si[ base + g ] : 0;
-        const double wi = valid ? sw[ base + g ] : 0.0;
-        const int rc = valid ? A.cnt[ i ] : -1;
-        const I64 b = valid ? A.base( i ) : 0;
-        for ( int q0 = 0; __any( q0 <= rc ); q0 += 8 ) {
-            const int q = q0 + sub;
-            int j = i, np = 0;
-            double a = 0;
-            if ( q <= rc ) {
+    for ( int base = 0; base < cnt && nkeys <= SA_SMAX + 1; base += 8 ) {   // ( past any room the hash would fill up )
+        if ( base + g < cnt ) {
+            const int i = si[ base + g ];
+            const double wi = sw[ base + g ] * scale;
+            const int rc = A.cnt[ i ];
+            const I64 b = A.base( i );
+            for ( int q = sub; q <= rc; q += 8 ) {
+                int j = i;
+                double a;
                 if ( q < rc ) { j = A.col[ b + I64( q ) * A.step ]; a = -double( A.val[ b + I64( q ) * A.step ] ); }
                 else a = double( A.dia[ i ] );
-                np = pn[ j ];
-            }
-            int inc = np;
-            for ( int o = 1; o < 64; o <<= 1 ) { const int v = __shfl_up( inc, o, 64 ); if ( lane >= o ) inc += v; }
-            const int total = __shfl( inc, 63, 64 );
-            for ( int e = 0, at = inc - np; e < np; ++e, ++at ) {
-                const int K = pcol[ I64( e ) * A.n + j ];
-                tv[ at ] = wi * a * double( pval[ I64( e ) * A.n + j ] );
-                unsigned h = ( unsigned( K ) * 2654435761u ) >> 23;
-                int slot = -1;
-                for ( int probe = 0; probe < SA_HASH; ++probe, h = ( h + 1 ) & ( SA_HASH - 1 ) ) {
-                    const int prev = atomicCAS( &hk[ h ], -1, K );
-                    if ( prev == -1 ) {
-                        const int id = atomicAdd( &nkeys, 1 );
-                        hi[ h ] = id;
-                        if ( id <= SA_SMAX ) ck[ id ] = K;
+                const int np = pn[ j ];
+                for ( int e = 0; e < np; ++e ) {
+                    const int K = pcol[ I64( e ) * A.n + j ];
+                    const long long term = __double2ll_rn( wi * a * double( pval[ I64( e ) * A.n + j ] ) );
+                    unsigned h = ( unsigned( K ) * 2654435761u ) >> 23;
+                    for ( int probe = 0; probe < SA_HASH; ++probe, h = ( h + 1 ) & ( SA_HASH - 1 ) ) {
+                        int prev = hk[ h ];
+                        if ( prev == -1 ) {
+                            prev = atomicCAS( &hk[ h ], -1, K );
+                            if ( prev == -1 ) {
+                                const int id = atomicAdd( &nkeys, 1 );
+                                if ( id <= SA_SMAX ) { ck[ id ] = K; at[ id ] = int( h ); }
+                                prev = K;
+                            }
+                        }
+                        if ( prev == K ) { atomicAdd( &sum[ h ], static_cast<unsigned long long>( term ) ); break; }
                     }
-                    if ( prev == -1 || prev == K ) { slot = int( h ); break; }
                 }
-                ti[ at ] = slot;
             }
-            __syncthreads();
-            const int keys = nkeys;
-            if ( keys > SA_SMAX + 1 ) { base = cnt; break; }    // ( past any room: the hash would fill up )
-            const int padded = ( total + 3 ) & ~3;
-            for ( int t = lane; t < padded; t += 64 ) {
-                ti[ t ] = t < total ? hi[ ti[ t ] ] : SA_HASH;
-                if ( t >= total ) tv[ t ] = 0;
-            }
-            __syncthreads();
-            for ( int t = 0; t < padded; t += 4 ) {
-                const int4 id = *reinterpret_cast<const int4 *>( ti + t );
-                const double2 v0 = *reinterpret_cast<const double2 *>( tv + t ), v1 = *reinterpret_cast<const double2 *>( tv + t + 2 );
-                acc[ 0 ] += id.x == lane ? v0.x : 0.0; acc[ 0 ] += id.y == lane ? v0.y : 0.0;
-                acc[ 0 ] += id.z == lane ? v1.x : 0.0; acc[ 0 ] += id.w == lane ? v1.y : 0.0;
-                if ( keys > 64 )
-#pragma unroll
-                    for ( int u = 1; u < 4; ++u ) {
-                        const int m = lane + 64 * u;
-                        acc[ u ] += id.x == m ? v0.x : 0.0; acc[ u ] += id.y == m ? v0.y : 0.0;
-                        acc[ u ] += id.z == m ? v1.x : 0.0; acc[ u ] += id.w == m ? v1.y : 0.0;
-                    }
-            }
-            __syncthreads();
         }
+        __syncthreads();
     }
     const int m = min( nkeys, SA_SMAX + 1 );
     bool diag = false;
-#pragma unroll
-    for ( int u = 0; u < 4; ++u ) {
-        const int id = lane + 64 * u;
-        if ( id >= m ) continue;
+    for ( int id = lane; id < m; id += 64 ) {
         const int K = ck[ id ];
+        const double v = double( static_cast<long long>( sum[ at[ id ] ] ) ) * unit;
         if ( K == int( I ) ) {
-            const P d = P( acc[ u ] > 0 ? acc[ u ] : 1.0 );
+            const P d = P( v > 0 ? v : 1.0 );
             cdia[ I ] = d;
             cdinv[ I ] = P( 1.0 / double( d ) );
             diag = true;
@@ -352,7 +329,7 @@ __global__ __launch_bounds__( 64 ) void k_galerkin( Rows<P> A, const int *pn, co
         }
         int r = 0;
         for ( int k = 0; k < m; ++k ) r += ck[ k ] < K && ck[ k ] != int( I );
-        if ( r < room ) { ccol[ I * room + r ] = K; cval[ I * room + r ] = P( -acc[ u ] ); }
+        if ( r < room ) { ccol[ I * room + r ] = K; cval[ I * room + r ] = P( -v ); }
     }
     const bool has_diag = __any( diag );
     if ( lane == 0 ) {
