@@ -284,7 +284,7 @@ def bench_3d( args ):
                                 n = args.n, tol_abs = args.tol, start = "cold ( Voronoi ), tree included", step = "trials", continuation = "auto",
                                 linear = "jacobi-pcg" if args.linear == "cg" else "multigrid flexible CG", cells = "fp64" ),
                  roofline = roof_cells,
-                 roofline_secondary = dict( kernel = "k_cg_spmv_dot" if args.linear == "cg" else "k_fcg_spmv", bound = "hbm", achieved = spmv_gbs, peak = HBM_PEAK_GBS, unit = "GB/s",
+                 roofline_secondary = dict( kernel = "k_cg_spmv_dot" if args.linear == "cg" else "k_direction", bound = "hbm", achieved = spmv_gbs, peak = HBM_PEAK_GBS, unit = "GB/s",
                                   frac = spmv_gbs / HBM_PEAK_GBS, traffic = None, avg_launch_ms = spmv_avg_ms, launches_timed = spmv_launches,
                                   bytes_per_launch = spmv_bytes / max( spmv_launches, 1 ) ),
                  cells = dict( kernels_ms_per_diagram = cells_ms / max( cells_launches, 1 ), diagrams = cells_launches,
@@ -376,7 +376,7 @@ def main():
     target = sdot.Image( img_h, origin = [ 0, 0 ], frame = np.eye( 2 ) / args.res )
     settings = sdot.Iterative( tol = args.tol, continuation = args.continuation, on_failure = "ignore", precision = args.precision,
                                tuning = sdot.Tuning( step = args.step, linear_solver = args.linear, linear_tol = args.linear_tol ) )
-    linear = "jacobi-pcg" if args.linear == "cg" else "multigrid flexible CG ( aggregates of 8 tree ranks, degree-2 Chebyshev smoothing, K-cycle on levels 1-2 )"
+    linear = "jacobi-pcg" if args.linear == "cg" else "multigrid flexible CG ( smoothed aggregation over tree ranks, V-cycle, degree-2 Chebyshev smoothing )"
     print( f"bench: n = { args.n }, image { args.res }^2, tol { args.tol }", file = sys.stderr, flush = True )
 
     def step():
@@ -415,20 +415,20 @@ def main():
     kf = _KERNEL_FLOAT[ args.precision ]
     k32 = kf == _native.FP32 or ( kf == _native.MIXED and st[ "it_double" ] < 0 )
     if k32:
-        t_walk, t_fin = measured_traffic( "k_cells_walk32", args ), measured_traffic( "k_cells_finish32", args )
-        roof_cells = dict( kernel = "k_cells_walk32 + k_cells_finish32", bound = "fp32-valu", achieved = cells_tf, peak = FP32_PEAK_TFLOPS,
+        t_walk, t_fin = measured_traffic( "k_cells_walk_lanes", args ), measured_traffic( "k_cells_finish32", args )
+        roof_cells = dict( kernel = "k_cells_walk ( FP32 ) + k_cells_finish32", bound = "fp32-valu", achieved = cells_tf, peak = FP32_PEAK_TFLOPS,
                            unit = "TFLOP/s", frac = cells_tf / FP32_PEAK_TFLOPS,
                            traffic = None if t_walk is None or t_fin is None else t_walk + t_fin, avg_launch_ms = cells_avg_ms,
                            launches = cells_launches, flops_per_launch = flops / max( cells_launches, 1 ) )
     else:
-        roof_cells = dict( kernel = "k_cells_pass1", bound = "fp64-valu", achieved = cells_tf, peak = FP64_PEAK_TFLOPS, unit = "TFLOP/s",
-                           frac = cells_tf / FP64_PEAK_TFLOPS, traffic = measured_traffic( "k_cells_pass1", args ), avg_launch_ms = cells_avg_ms,
+        roof_cells = dict( kernel = "k_cells_walk + k_cells_finish", bound = "fp64-valu", achieved = cells_tf, peak = FP64_PEAK_TFLOPS, unit = "TFLOP/s",
+                           frac = cells_tf / FP64_PEAK_TFLOPS, traffic = None, avg_launch_ms = cells_avg_ms,
                            launches = cells_launches, flops_per_launch = flops / max( cells_launches, 1 ) )
     spmv_ms, spmv_launches = times[ "spmv" ]
     spmv_avg_ms = spmv_ms / max( spmv_launches, 1 )
     spmv_gbs = ( spmv_bytes / max( spmv_launches, 1 ) ) / ( spmv_avg_ms * 1e-3 ) / 1e9 if spmv_launches else 0.0
-    roof_spmv = dict( kernel = "k_cg_spmv_dot" if args.linear == "cg" else "k_fcg_spmv", bound = "hbm", achieved = spmv_gbs, peak = HBM_PEAK_GBS, unit = "GB/s", frac = spmv_gbs / HBM_PEAK_GBS,
-                      traffic = measured_traffic( "k_fcg_spmv" if args.linear != "cg" else "k_cg_spmv_dot", args ), avg_launch_ms = spmv_avg_ms,
+    roof_spmv = dict( kernel = "k_cg_spmv_dot" if args.linear == "cg" else "k_direction", bound = "hbm", achieved = spmv_gbs, peak = HBM_PEAK_GBS, unit = "GB/s", frac = spmv_gbs / HBM_PEAK_GBS,
+                      traffic = measured_traffic( "k_direction" if args.linear != "cg" else "k_cg_spmv_dot", args ), avg_launch_ms = spmv_avg_ms,
                       launches_timed = spmv_launches,
                       bytes_per_launch = spmv_bytes / max( spmv_launches, 1 ) )
     # the SpMV is timed one launch in sixteen: its share of the step is estimated from the CG iteration count

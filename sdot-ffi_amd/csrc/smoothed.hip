@@ -11,7 +11,7 @@
 //     coarse rows would grow past 100 entries ), the rest scaled to a unit sum ( `k_prolongator` ); the restriction is `P^T`,
 //     listed per coarse row in increasing order of the fine rows;
 //   * the Galerkin row `P^T A P` by one wave: its columns found by an LDS hash, each column's sum taken in whole numbers of
-//     a bound's 2^-57, so the result does not depend on the hash's races ( `k_galerkin` );
+//     a bound's 2^-60, so the result does not depend on the hash's races ( `k_galerkin` );
 //   * two damped Jacobi sweeps before ( from zero: one pass ) and after, Chebyshev dampings; the correction scaled by 1.2, which
 //     saves 10 % of the iterations ( 1.15 to 1.45 measured alike ), as truncated prolongations under-correct;
 //   * THE BOTTOM: the first level of at most 2048 rows is one product with a dense operator, the V-cycle over the levels below
@@ -260,9 +260,9 @@ __device__ __forceinline__ int sorted_list( I64 I, I64 nf, const int *pn, const 
 
 /// THE GALERKIN ROWS, one wave a coarse row ( see the file's header ): the terms `P_iI a_ij P_jK` of the fine rows `i` of its list, eight
 /// lanes a fine row, added in LDS at their column's place in a hash of the columns met ( at most `SA_SMAX + 1` ). The sums are 64-bit
-/// whole numbers of `2^-57` of a bound of the row's terms ( `P`'s rows sum to 1, a row of `A` to at most twice its diagonal: there are four
+/// whole numbers of `2^-60` of a bound of the row's terms ( `P`'s rows sum to 1, a row of `A` to at most twice its diagonal: there are three
 /// bits for what is off this ), so that the atomics' order does not matter: the row is the same in every run, and each sum is within
-/// `2^-58` of the bound a term, where a sum in double rounds by `2^-53` of itself. `state[ S_BAD ]` when a list or a row outgrows its room.
+/// `2^-61` of the bound a term, where a sum in double rounds by `2^-53` of itself. `state[ S_BAD ]` when a list or a row outgrows its room.
 /// ( Terms staged in LDS and added up by their column's lane, every lane looking at every term: 1M rows 2.05 ms a hierarchy, 0.90 so )
 template<class P>
 __global__ __launch_bounds__( 64 ) void k_galerkin( Rows<P> A, const int *pn, const int *pcol, const P *pval, int *tn, int *tcol, P *tval, int room,
@@ -280,7 +280,7 @@ __global__ __launch_bounds__( 64 ) void k_galerkin( Rows<P> A, const int *pn, co
     for ( int k = lane; k < cnt; k += 64 ) bound += 2 * fabs( sw[ k ] * double( A.dia[ si[ k ] ] ) );
     for ( int o = 32; o; o >>= 1 ) bound += __shfl_xor( bound, o, 64 );
     const int ex = bound > 0 && bound < 1e300 ? ilogb( bound ) + 1 : 0;
-    const double scale = ldexp( 1.0, 57 - ex ), unit = ldexp( 1.0, ex - 57 );
+    const double scale = ldexp( 1.0, 60 - ex ), unit = ldexp( 1.0, ex - 60 );
     const int g = lane >> 3, sub = lane & 7;
     for ( int base = 0; base < cnt && nkeys <= SA_SMAX + 1; base += 8 ) {   // ( past any room the hash would fill up )
         if ( base + g < cnt ) {
