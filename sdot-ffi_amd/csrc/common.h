@@ -263,6 +263,15 @@ inline unsigned long long ordered_key_host( double x ) {
     return ( u >> 63 ) ? ~u : ( u | 0x8000000000000000ull );
 }
 
+/// a stop flag read once for the whole block, for the kernels that may set it themselves: read by each thread, one wave of a block could
+/// see it clear and a later one set by another block of the same launch, and leave before the block's barriers
+__device__ __forceinline__ bool block_stopped( const double *flag ) {
+    __shared__ int stop;
+    if ( threadIdx.x == 0 ) stop = *flag != 0;
+    __syncthreads();
+    return stop != 0;
+}
+
 /// block-wide sum of a double, deterministic ( fixed tree over the block )
 template<int THREADS>
 __device__ __forceinline__ double block_sum( double v, double *sh ) {

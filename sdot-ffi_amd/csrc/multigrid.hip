@@ -611,7 +611,7 @@ __global__ __launch_bounds__( RED_THREADS ) void k_fcg_spmv( MatT<R> A, const R 
 template<class R>
 __global__ __launch_bounds__( RED_THREADS ) void k_pcg_update( I64 n, const R *p, const R *q, R *d, R *r, double *part, double *state ) {
     __shared__ double sh[ RED_THREADS ];
-    if ( state[ S_DONE ] != 0 ) return;
+    if ( block_stopped( &state[ S_DONE ] ) ) return;
     const double pq = sum_parts( part, RED_BLOCKS, sh ), pr = sum_parts( part + RED_BLOCKS, RED_BLOCKS, sh );
     if ( ! ( pq > 0 ) ) {
         if ( blockIdx.x == 0 && threadIdx.x == 0 ) { state[ S_PQ ] = pq; state[ S_DONE ] = 1; state[ S_FAILED ] = 1; }
@@ -632,7 +632,7 @@ __global__ __launch_bounds__( RED_THREADS ) void k_pcg_update( I64 n, const R *p
 
 __global__ __launch_bounds__( RED_THREADS ) void k_pcg_check( const double *part, double *state ) {
     __shared__ double sh[ RED_THREADS ];
-    if ( state[ S_DONE ] != 0 ) return;
+    if ( block_stopped( &state[ S_DONE ] ) ) return;
     const double rr = sum_parts( part + 2 * RED_BLOCKS, RED_BLOCKS, sh );
     if ( threadIdx.x == 0 ) {
         state[ S_RR ] = rr;

@@ -618,7 +618,7 @@ template<class P, bool TEST>
 __global__ __launch_bounds__( TH ) void k_fine_two( Rows<P> A, const P *dinv, const P *r, const P *y, P *x, double w1, const double *part, int nblk,
                                                    double *state ) {
     __shared__ double sh[ 4 ];
-    if ( state[ S_DONE ] != 0 ) return;
+    if ( TEST ? block_stopped( &state[ S_DONE ] ) : state[ S_DONE ] != 0 ) return;
     if ( TEST ) {
         const double err = sqrt( sum_partials( part + P_RR * SA_BLOCKS, nblk, sh ) ) / state[ S_NB ];
         const bool done = err <= state[ S_TOL ];
@@ -771,7 +771,7 @@ template<class P>
 __global__ __launch_bounds__( TH ) void k_update( I64 n, const double *p, const double *q, const P *dinv, double w0, double *d, double *r, P *rp, P *y,
                                                  double *part, int nblk, double *state ) {
     __shared__ double sh[ 4 ];
-    if ( state[ S_DONE ] != 0 ) return;
+    if ( block_stopped( &state[ S_DONE ] ) ) return;
     const double pq = sum_partials( part + P_PQ * SA_BLOCKS, nblk, sh ), pr = sum_partials( part + P_PR * SA_BLOCKS, nblk, sh );
     if ( ! ( pq > 0 ) ) {
         if ( blockIdx.x == 0 && threadIdx.x == 0 ) { state[ S_PQ ] = pq; state[ S_DONE ] = 1; state[ S_FAILED ] = 1; }

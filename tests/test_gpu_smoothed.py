@@ -81,3 +81,11 @@ def test_rows_without_room_go_to_the_other_solvers( native ):
     assert its[ 0 ] > 0
     r = b.numpy()[ p ] - ( dia[ p ] * x - np.bincount( i2, weights = val * x[ j2 ], minlength = n ) )
     assert np.linalg.norm( r ) <= 1e-8 * np.linalg.norm( b.numpy() )
+
+
+@pytest.mark.parametrize( "fp32", [ False, True ] )
+def test_a_breakdown_leaves_the_solution_untouched( native, fp32 ):
+    # a negative definite system breaks down at its first step: every block of the update has to take that decision, none a step
+    row, col, val, dia, b = _system( native, 150_001, 2, 3 )
+    x, its = native.linear_solves_2d( row, col, -val, -dia, b, tol = 1e-8, method = "mg", smoothed = True, fp32 = fp32 )
+    assert its[ 0 ] == -1 and not x.any().item()
