@@ -69,8 +69,10 @@ void build_tree_device( DevTree &t, I64 n, const double *pos_dev, int leaf, hipS
 /// `|a| |y|` passes 100 times the weights' spread on the node, and raises the constant by 1e-6 of the weights' size, both against
 /// cancellation in `a . y + b`. On small cells under large weights that leaves nothing to prune with: weights of 0.02 that vary
 /// over the unit square, 1M seeds: every node under a hundredth of the square has its largest weight as its majorant, and a cell meets 127
-/// seeds and 101 nodes where 30 and 84 would do ( the FP32 walk 9.5 -> 7.2 ms ). In double the cancellation costs 1e-16 of `|a| |y|`: the walks take the slope up to 1e7
-/// times the spread and a slack of 1e-12. Pruning changes no cell
+/// seeds and 101 nodes where 30 and 84 would do ( the FP32 walk 9.5 -> 7.2 ms ). In double the cancellation costs 1e-16 of `|a_x x| + |a_y y|`: the
+/// walks take the slope up to 1e7 times the spread, and of the reference's slack what covers the rounding of the majorant and of the
+/// walk's test: 1e-12 of the weights' size, 2e-15 of the slope's terms, 1e-15 of the coordinates' size times the cloud's extent. So a node
+/// is pruned where the reference's rule keeps it only for lack of a slope
 void refresh_majorants( DevTree &t, hipStream_t st, bool reference = false );
 
 /// writes `w_user[ order[ k ] ]` into `seeds[ k ].z`

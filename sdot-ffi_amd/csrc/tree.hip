@@ -379,7 +379,7 @@ __global__ void k_major_spread( const double4 *seeds, int n, const int *node_end
 
 /// the decision of every node ( `bsp_build_level.h:176-208` ) and its walk record
 __global__ void k_major_final( const double *S, int N, const double *fit, const unsigned long long *rk, const double *box, const int *beg,
-                               const int *end, double slack, double reach, NodeRec *nodes, NodeF *nodes32 ) {
+                               const int *end, bool reference, NodeRec *nodes, NodeF *nodes32 ) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if ( m >= N ) return;
     NodeRec r;
@@ -392,12 +392,13 @@ __global__ void k_major_final( const double *S, int N, const double *fit, const 
         const double wmin = S[ S_WMIN * N + m ], wmax = S[ S_WMAX * N + m ], spread = wmax - wmin;
         const double fx = fit[ m ], fy = fit[ N + m ];
         bool accept = false;
-        double bb = wmax, amax = 0;
+        double bb = wmax, amax = 0, terms = 0;
         if ( fx == fx ) {
             const double rmin = ordered_value( rk[ m ] ), rmax = ordered_value( rk[ N + m ] );
             const double u = 1.0 - 2.0 / ( cnt - 1 );
             const double by_chance = sqrt( u > 0 ? u : 0.0 );
             bool well = true;
+            const double reach = reference ? 100.0 : 1e7;
             const double reach_x = fmax( fabs( r.lo_x ), fabs( r.hi_x ) ), reach_y = fmax( fabs( r.lo_y ), fabs( r.hi_y ) );
             if ( fabs( fx ) * ( r.hi_x - r.lo_x ) > 8 * spread || fabs( fx ) * reach_x > reach * spread ) well = false;
             if ( fabs( fy ) * ( r.hi_y - r.lo_y ) > 8 * spread || fabs( fy ) * reach_y > reach * spread ) well = false;
@@ -405,10 +406,19 @@ __global__ void k_major_final( const double *S, int N, const double *fit, const 
                 accept = true;
                 bb = rmax;
                 amax = ordered_value( rk[ 2 * N + m ] );
+                terms = fabs( fx ) * reach_x + fabs( fy ) * reach_y;
             }
         }
         if ( accept ) { r.wa_x = fx; r.wa_y = fy; }
-        r.wb = bb + slack * ( fabs( bb ) + spread + amax );
+        double slack = 1e-6 * ( fabs( bb ) + spread + amax );
+        if ( ! reference ) {
+            // `amax` is of the sum `a . y`, whose two terms may cancel while each rounds by itself, here and in the walk's test; that
+            // test also rounds a vertex's position to an ulp of its coordinates, times its distance to the node
+            const double R = fmax( fmax( fabs( box[ 0 ] ), fabs( box[ 2 ] ) ), fmax( fabs( box[ 1 ] ), fabs( box[ 3 ] ) ) );
+            const double rounding = 2e-15 * terms + 1e-15 * R * ( ( box[ 2 ] - box[ 0 ] ) + ( box[ 3 ] - box[ 1 ] ) );
+            slack = fmin( slack, 1e-12 * ( fabs( bb ) + spread + amax ) + rounding );
+        }
+        r.wb = bb + slack;
     }
     nodes[ m ] = r;
     if ( nodes32 ) {
@@ -451,8 +461,8 @@ void refresh_majorants( DevTree &t, hipStream_t st, bool reference ) {
     check_launch( "k_major_fit" );
     k_major_spread<<<blocks_for( t.n, 256 ), 256, 0, st>>>( t.seeds, int( t.n ), t.node_end, depth, t.fit, N, t.rkeys );
     check_launch( "k_major_spread" );
-    k_major_final<<<blocks_for( N, 256 ), 256, 0, st>>>( t.stat, N, t.fit, t.rkeys, t.node_box, t.node_beg, t.node_end, reference ? 1e-6 : 1e-12,
-                                                            reference ? 100.0 : 1e7, t.nodes, t.nodes32 );
+    k_major_final<<<blocks_for( N, 256 ), 256, 0, st>>>( t.stat, N, t.fit, t.rkeys, t.node_box, t.node_beg, t.node_end, reference,
+                                                            t.nodes, t.nodes32 );
     check_launch( "k_major_final" );
     if ( timed ) timing().end( tp, st );
 }

@@ -41,7 +41,7 @@ def test_many_sided_cells_by_whole_waves_and_by_lanes( native, oracle ):
 @pytest.mark.parametrize( "n, scale, shift", [ ( 60_000, 0.02, 0.0 ), ( 60_000, 0.02, 1e3 ), ( 60_000, 0.02, -1e6 ), ( 3_000, 30.0, 5.0 ) ] )
 def test_kept_slopes_change_no_cell( native, oracle, n, scale, shift ):
     # weights that vary slowly over the square: most nodes under a hundredth of it have their slope dropped by the reference's rule
-    # ( the oracle's ); a large common weight and large coordinates cancel in the majorants
+    # ( the oracle's ); a large common weight cancels in the majorants
     rng = np.random.default_rng( 3 )
     L = np.sqrt( scale / 0.02 )
     pos = rng.uniform( 0, L, ( n, 2 ) )
@@ -56,3 +56,21 @@ def test_kept_slopes_change_no_cell( native, oracle, n, scale, shift ):
     assert np.abs( m - mo ).max() <= tol
     m32 = native.measures_2d( pos, w, [ 0, 0, L, L ], dens, precision = 1 ).cpu().numpy()
     assert np.abs( m32 - mo ).max() <= 1e-9 * L * L / n + tol
+
+
+# `along`: weights `slope ( x - y )` plus a constant. On the diagonal the majorants' two terms cancel, and on a lattice every vertex is met by a
+# plane that passes it within rounding: a majorant or a test below its own rounding loses slivers
+@pytest.mark.parametrize( "at", [ ( 0.0, 0.0 ), ( 1e4, 1e4 ), ( 1e5, 0.0 ), ( 1e5, 1e5 ), ( -1e5, 1e5 ), ( 3.3e4, 7.7e5 ), ( 1e6, 1e6 ) ] )
+@pytest.mark.parametrize( "slope, constant", [ ( 0.1, 0.0 ), ( 1e-3, 1e-3 ), ( 0.0, 1e-3 ) ] )
+def test_a_lattice_far_from_the_origin_loses_no_sliver( native, at, slope, constant ):
+    import torch
+    from sdot import UniformBox
+    at = np.array( at )
+    for k in ( 50, 141 ):
+        pos = np.stack( np.meshgrid( *[ ( np.arange( k ) + 0.5 ) / k ] * 2, indexing = "ij" ), -1 ).reshape( -1, 2 ) + at
+        w = slope * ( ( pos - at ) @ [ 1.0, -1.0 ] ) + constant
+        # ( counting the walk's steps takes the reference's majorants )
+        got = native.measures_2d( pos, w, [ *at, *( at + 1 ) ], UniformBox( at, at + 1 ), facets = True )
+        ref = native.measures_2d( pos, w, [ *at, *( at + 1 ) ], UniformBox( at, at + 1 ), facets = True, events = True )
+        pairs = [ torch.sort( r[ 1 ][ 0 ] * len( pos ) + r[ 1 ][ 1 ] )[ 0 ] for r in ( got, ref ) ]
+        assert torch.equal( *pairs ) and torch.equal( got[ 0 ], ref[ 0 ] )
