@@ -71,6 +71,11 @@ int sdot_amd_fp32_counts( long long *diagrams, long long *redone, long long *dro
  * HOST [ 1 ] each, may be null. */
 int sdot_amd_mg32_counts( long long *solves, long long *iterations, long long *fallbacks );
 
+/* WHICH CYCLE TOOK THE SYSTEMS ( no counterpart in the reference ): since the last `sdot_amd_kernel_times( ..., reset = 1 )`, the systems
+ * the smoothed-aggregation cycle was tried on, and those the K-cycle was ( asked for, or handed over by the smoothed cycle: a row
+ * past its room, or a tolerance it missed ). HOST [ 1 ] each, may be null. */
+int sdot_amd_cycle_counts( long long *smoothed, long long *kcycle );
+
 /* ONE DIAGRAM: the masses of the power cells of `( positions, weights )` in the box
  * `box = { lo_x, lo_y, hi_x, hi_y }` ( HOST ) against a density, and optionally the facets
  * `c_ij = int_facet rho / ( 2 |p_i - p_j| )` as triplets ( rows in user order, each row in its cell's

@@ -284,6 +284,13 @@ int sdot_amd_mg32_counts( long long *solves, long long *iterations, long long *f
     } );
 }
 
+int sdot_amd_cycle_counts( long long *smoothed, long long *kcycle ) {
+    return guarded( [&] {
+        if ( smoothed ) *smoothed = timing().smoothed_systems.load();
+        if ( kcycle ) *kcycle = timing().kcycle_systems.load();
+    } );
+}
+
 int sdot_amd_graph_counts( long long *captures, long long *replays ) {
     return guarded( [&] {
         if ( captures ) *captures = timing().graph_captures.load();

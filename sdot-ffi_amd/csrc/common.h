@@ -190,6 +190,8 @@ struct Timing {
     // the multigrid's FP32 preconditioner ( counted whether timing is on or not ): the solves, their flexible-CG iterations, and
     // the solves redone with the FP64 preconditioner because they did not converge
     std::atomic<long long> mg32_solves{ 0 }, mg32_iterations{ 0 }, mg32_fallbacks{ 0 };
+    // the systems the smoothed cycle was tried on, and those the K-cycle was ( counted whether timing is on or not )
+    std::atomic<long long> smoothed_systems{ 0 }, kcycle_systems{ 0 };
     std::mutex mtx;
 
     hipEvent_t take() {
@@ -232,6 +234,7 @@ struct Timing {
         graph_captures = 0;
         fp32_diagrams = 0; fp32_redone = 0; fp32_dropped = 0;
         mg32_solves = 0; mg32_iterations = 0; mg32_fallbacks = 0;
+        smoothed_systems = 0; kcycle_systems = 0;
         graph_replays = 0;
     }
 };

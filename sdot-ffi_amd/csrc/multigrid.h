@@ -22,7 +22,8 @@ struct MgOptions {
     /// the FP64 cycle when that solve does not converge
     bool   fp32 = false;
     /// the smoothed-aggregation V-cycle ( smoothed.hip ) before the K-cycle over plain aggregates, which then takes the systems it has
-    /// no room for ( a coarse row past its entries ) and the callers that set `pack`, `nu`, `kcycle` or `bottom` themselves
+    /// no room for ( a coarse row past its entries ) or does not bring to the tolerance, and the callers that set `pack`, `nu`, `kcycle`
+    /// or `bottom` themselves
     bool   smoothed = true;
 };
 

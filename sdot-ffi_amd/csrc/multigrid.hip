@@ -984,26 +984,8 @@ int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, i
     bool done = false;
     double err = 1, true_err = 1;
     bool breakdown = false;
-    bool smoothed = o.smoothed && n > SA_MIN_ROWS;
-    float *valf = nullptr, *diaf = nullptr;
-    // one solve of the system ( `f32`: the cycle in FP32 ); false when its hierarchy could not be built
-    auto attempt = [&]( bool f32 ) {
-        const int left = f32 ? maxit : std::max( maxit - total, 4 );
-        FcgResult f;
-        if ( smoothed ) {
-            f = smoothed_solve( L, f32 ? valf : nullptr, f32 ? diaf : nullptr, b, d, tol, left, o, st, nb_levels, cs.last_its );
-            if ( ! f.bad ) cs.last_its = f.its;
-            smoothed = ! f.bad;                          // ( a coarse row past its room: the K-cycle from here on )
-        }
-        if ( ! smoothed ) {
-            if ( f32 ) {
-                MatT<float> Af;
-                Af.n = n; Af.step = L.step; Af.row_off = L.row_off; Af.row_cnt = L.row_cnt; Af.col = L.col; Af.val = valf; Af.dia = diaf;
-                f = fcg_mg<double, float>( A0, Af, L.nnz, b, d, tol, left, o, st, nb_levels, "mgm" );
-            } else
-                f = fcg_mg<double, double>( A0, A0, L.nnz, b, d, tol, left, o, st, nb_levels, "mg" );
-            if ( f.bad ) return false;
-        }
+    // what one flexible CG came to ( `f32`: its cycle in FP32 )
+    auto take = [&]( const FcgResult &f, bool f32 ) {
         total += f.its;
         err = f.err;
         true_err = f.true_err;
@@ -1014,8 +996,8 @@ int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, i
             timing().mg32_iterations += f.its;
             if ( ! done ) { cs.nb_fp64_fallbacks += 1; ++timing().mg32_fallbacks; }
         }
-        return true;
     };
+    float *valf = nullptr, *diaf = nullptr;
     if ( o.fp32 ) {
         // THE FP32 PRECONDITIONER: the hierarchy, its smoothing and its coarse solves in FP32 ( from an FP32 copy of the rows ),
         // the flexible CG, its SpMV and its vectors in FP64; the FP64 preconditioner when that solve does not converge
@@ -1023,9 +1005,36 @@ int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, i
         diaf = A.get<float>( "mgm.diaf", size_t( n ) );
         k_to_float_rows<<<blocks_for( n, 256 ), 256, 0, st>>>( n, L.row_off, L.row_cnt, L.step, L.val, L.dia, valf, diaf );
         check_launch( "k_to_float_rows" );
-        if ( ! attempt( true ) ) return -2;
     }
-    if ( ! done && ! attempt( false ) ) return -2;
+    bool missed = false;                                 // ( the smoothed cycle had its hierarchy and did not reach the tolerance )
+    if ( o.smoothed && n > SA_MIN_ROWS ) {
+        const FcgResult f = smoothed_solve( L, valf, diaf, b, d, tol, maxit, o, st, nb_levels, cs.last_its );
+        ++timing().smoothed_systems;
+        if ( ! f.bad ) {
+            cs.last_its = f.its;
+            take( f, o.fp32 );
+            missed = ! done;
+        }
+    }
+    if ( ! done ) {
+        // THE K-CYCLE: asked for, or a system the smoothed one has no room for or misses; it has iterations of its own. In FP32 first,
+        // unless the smoothed cycle has missed the system in FP32 already
+        int left = maxit;
+        ++timing().kcycle_systems;
+        if ( o.fp32 && ! missed ) {
+            MatT<float> Af;
+            Af.n = n; Af.step = L.step; Af.row_off = L.row_off; Af.row_cnt = L.row_cnt; Af.col = L.col; Af.val = valf; Af.dia = diaf;
+            const FcgResult f = fcg_mg<double, float>( A0, Af, L.nnz, b, d, tol, left, o, st, nb_levels, "mgm" );
+            if ( f.bad ) return -2;
+            take( f, true );
+            left = std::max( left - f.its, 4 );
+        }
+        if ( ! done ) {
+            const FcgResult f = fcg_mg<double, double>( A0, A0, L.nnz, b, d, tol, left, o, st, nb_levels, "mg" );
+            if ( f.bad ) return -2;
+            take( f, false );
+        }
+    }
     double *g = A.get<double>( "mg.g", 1 );
     k_read_gauge<<<1, 64, 0, st>>>( d, gauge, g );
     k_shift_gauge<<<blocks_for( n, 256 ), 256, 0, st>>>( n, d, g, gauge );

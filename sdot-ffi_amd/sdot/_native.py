@@ -32,7 +32,7 @@ EXPORTS = [ "sdot_amd_abi_version", "sdot_amd_last_error", "sdot_amd_device_byte
             "sdot_amd_linear_solves_2d", "sdot_amd_solve_2d_batch", "sdot_amd_server_start", "sdot_amd_server_submit",
             "sdot_amd_server_wait", "sdot_amd_server_stop", "sdot_amd_measures_3d", "sdot_amd_solve_3d",
             "sdot_amd_solve_2d_precision", "sdot_amd_graph_counts", "sdot_amd_solve_bytes", "sdot_amd_server_submit_nd", "sdot_amd_server_info",
-            "sdot_amd_measures_2d_noalloc", "sdot_amd_measures_2d_noalloc_max_seeds", "sdot_amd_fp32_counts", "sdot_amd_mg32_counts",
+            "sdot_amd_measures_2d_noalloc", "sdot_amd_measures_2d_noalloc_max_seeds", "sdot_amd_fp32_counts", "sdot_amd_mg32_counts", "sdot_amd_cycle_counts",
             "sdot_amd_measures_2d_precision", "sdot_amd_moments_2d", "sdot_amd_moments_3d", "sdot_amd_cells_2d",
             "sdot_amd_measures_vjp_2d", "sdot_amd_solve_2d_batch_precision", "sdot_amd_measures_2d_domain", "sdot_amd_solve_2d_domain",
             "sdot_amd_measures_3d_image", "sdot_amd_solve_3d_image", "sdot_amd_moments_3d_image", "sdot_amd_server_submit_3d_image" ]
@@ -123,6 +123,8 @@ def lib():
         L.sdot_amd_fp32_counts.restype = _I
         L.sdot_amd_mg32_counts.argtypes = [ _P, _P, _P ]
         L.sdot_amd_mg32_counts.restype = _I
+        L.sdot_amd_cycle_counts.argtypes = [ _P, _P ]
+        L.sdot_amd_cycle_counts.restype = _I
         L.sdot_amd_graph_counts.argtypes = [ _P, _P ]
         L.sdot_amd_graph_counts.restype = _I
         L.sdot_amd_solve_bytes.argtypes = [ _LL, _I, _I, _P, _I, _P ]
@@ -591,6 +593,14 @@ def mg32_counts():
     s, r, f = _LL(), _LL(), _LL()
     _check( lib().sdot_amd_mg32_counts( ctypes.byref( s ), ctypes.byref( r ), ctypes.byref( f ) ) )
     return dict( solves = int( s.value ), iterations = int( r.value ), fallbacks = int( f.value ) )
+
+
+def cycle_counts():
+    """the linear systems since the last reset of the kernel times, by the cycle they were tried with: `{ smoothed, kcycle }` ( both, for one
+    that the smoothed cycle handed over )"""
+    s, k = _LL(), _LL()
+    _check( lib().sdot_amd_cycle_counts( ctypes.byref( s ), ctypes.byref( k ) ) )
+    return dict( smoothed = int( s.value ), kcycle = int( k.value ) )
 
 
 def graph_counts():

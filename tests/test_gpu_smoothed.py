@@ -34,6 +34,12 @@ def _system( native, n, d, seed ):
     return row, j, c, dia, torch.as_tensor( b - b.mean() )
 
 
+def _cycles_since( native, before ):
+    """the systems tried with the smoothed cycle and with the K-cycle since `before`"""
+    now = native.cycle_counts()
+    return now[ "smoothed" ] - before[ "smoothed" ], now[ "kcycle" ] - before[ "kcycle" ]
+
+
 # the sizes: one level over the coarsest ( 65: the smallest the cycle takes ), a bottom of one level and of two, the first
 # aggregates of 4 and of 8 ( 8192 / 8193 ), a level between the finest and the bottom, 3D rows
 @pytest.mark.parametrize( "n, d", [ ( 65, 2 ), ( 256, 2 ), ( 261, 2 ), ( 2049, 2 ), ( 8192, 2 ), ( 8193, 2 ), ( 40_003, 2 ), ( 150_001, 2 ), ( 700, 3 ), ( 9_001, 3 ) ] )
@@ -76,9 +82,10 @@ def test_rows_without_room_go_to_the_other_solvers( native ):
     i2, j2 = inv[ i ], inv[ col ]
     at = np.lexsort( ( j2, i2 ) )
     row2 = np.concatenate( [ [ 0 ], np.cumsum( np.bincount( i2, minlength = n ) ) ] )
+    before = native.cycle_counts()
     x, its = native.linear_solves_2d( row2, j2[ at ], val[ at ], dia[ p ], b.numpy()[ p ], tol = 1e-9, method = "mg", smoothed = True, fp32 = True )
     x = x[ 0 ].cpu().numpy()
-    assert its[ 0 ] > 0
+    assert its[ 0 ] > 0 and _cycles_since( native, before ) == ( 1, 1 )
     r = b.numpy()[ p ] - ( dia[ p ] * x - np.bincount( i2, weights = val * x[ j2 ], minlength = n ) )
     assert np.linalg.norm( r ) <= 1e-8 * np.linalg.norm( b.numpy() )
 
@@ -87,5 +94,18 @@ def test_rows_without_room_go_to_the_other_solvers( native ):
 def test_a_breakdown_leaves_the_solution_untouched( native, fp32 ):
     # a negative definite system breaks down at its first step: every block of the update has to take that decision, none a step
     row, col, val, dia, b = _system( native, 150_001, 2, 3 )
+    before = native.cycle_counts()
     x, its = native.linear_solves_2d( row, col, -val, -dia, b, tol = 1e-8, method = "mg", smoothed = True, fp32 = fp32 )
-    assert its[ 0 ] == -1 and not x.any().item()
+    assert its[ 0 ] == -1 and not x.any().item() and _cycles_since( native, before ) == ( 1, 1 )
+
+
+@pytest.mark.parametrize( "fp32", [ False, True ] )
+def test_a_missed_tolerance_goes_to_the_k_cycle( native, fp32 ):
+    # coefficients over twenty orders of magnitude: no cycle brings them to the tolerance, each is tried
+    row, col, val, dia, b = _system( native, 9_000, 2, 7 )
+    i = np.repeat( np.arange( 9_000 ), np.diff( row ) )
+    far = np.exp( 4 * np.random.default_rng( 1 ).normal( size = 9_000 ) )
+    val = val * far[ i ] * far[ col ]
+    before = native.cycle_counts()
+    _, its = native.linear_solves_2d( row, col, val, np.bincount( i, weights = val ), b, tol = 1e-8, method = "mg", smoothed = True, fp32 = fp32 )
+    assert its[ 0 ] == -1 and _cycles_since( native, before ) == ( 1, 1 )
