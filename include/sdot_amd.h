@@ -72,8 +72,8 @@ int sdot_amd_fp32_counts( long long *diagrams, long long *redone, long long *dro
 int sdot_amd_mg32_counts( long long *solves, long long *iterations, long long *fallbacks );
 
 /* WHICH CYCLE TOOK THE SYSTEMS ( no counterpart in the reference ): since the last `sdot_amd_kernel_times( ..., reset = 1 )`, the systems
- * the smoothed-aggregation cycle was tried on, and those the K-cycle was ( asked for, or handed over by the smoothed cycle: a row
- * past its room, or a tolerance it missed ). HOST [ 1 ] each, may be null. */
+ * the smoothed-aggregation cycle ran on, and those the K-cycle was tried on ( asked for; or handed over, by a smoothed hierarchy that could
+ * not be built or a cycle that missed the tolerance: the second kind counts in both ). HOST [ 1 ] each, may be null. */
 int sdot_amd_cycle_counts( long long *smoothed, long long *kcycle );
 
 /* ONE DIAGRAM: the masses of the power cells of `( positions, weights )` in the box

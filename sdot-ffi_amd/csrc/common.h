@@ -190,7 +190,7 @@ struct Timing {
     // the multigrid's FP32 preconditioner ( counted whether timing is on or not ): the solves, their flexible-CG iterations, and
     // the solves redone with the FP64 preconditioner because they did not converge
     std::atomic<long long> mg32_solves{ 0 }, mg32_iterations{ 0 }, mg32_fallbacks{ 0 };
-    // the systems the smoothed cycle was tried on, and those the K-cycle was ( counted whether timing is on or not )
+    // the systems the smoothed cycle ran on, and those the K-cycle was tried on ( counted whether timing is on or not )
     std::atomic<long long> smoothed_systems{ 0 }, kcycle_systems{ 0 };
     std::mutex mtx;
 

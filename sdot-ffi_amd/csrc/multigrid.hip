@@ -1009,8 +1009,8 @@ int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, i
     bool missed = false;                                 // ( the smoothed cycle had its hierarchy and did not reach the tolerance )
     if ( o.smoothed && n > SA_MIN_ROWS ) {
         const FcgResult f = smoothed_solve( L, valf, diaf, b, d, tol, maxit, o, st, nb_levels, cs.last_its );
-        ++timing().smoothed_systems;
         if ( ! f.bad ) {
+            ++timing().smoothed_systems;
             cs.last_its = f.its;
             take( f, o.fp32 );
             missed = ! done;

@@ -260,9 +260,10 @@ __device__ __forceinline__ int sorted_list( I64 I, I64 nf, const int *pn, const 
 
 /// THE GALERKIN ROWS, one wave a coarse row ( see the file's header ): the terms `P_iI a_ij P_jK` of the fine rows `i` of its list, eight
 /// lanes a fine row, added in LDS at their column's place in a hash of the columns met ( at most `SA_SMAX + 1` ). The sums are 64-bit
-/// whole numbers of `2^-60` of a bound of the row's terms ( `P`'s rows sum to 1, a row of `A` to at most twice its diagonal: there are three
-/// bits for what is off this ), so that the atomics' order does not matter: the row is the same in every run, and each sum is within
-/// `2^-61` of the bound a term, where a sum in double rounds by `2^-53` of itself. `state[ S_BAD ]` when a list or a row outgrows its room.
+/// whole numbers of `2^-60` of a guess of the row's terms' size ( `P`'s rows sum to 1, a Laplacian's row to twice its diagonal ), so that the
+/// atomics' order does not matter: the row is the same in every run, and each sum is within `2^-61` of the guess a term, where a sum in
+/// double rounds by `2^-53` of itself. Entries of both signs can pass the guess, so the terms' sizes are summed too, in double: below `2^62`
+/// units no column's sum wraps. `state[ S_BAD ]` beyond it, and when a list or a row outgrows its room.
 /// ( Terms staged in LDS and added up by their column's lane, every lane looking at every term: 1M rows 2.05 ms a hierarchy, 0.90 so )
 template<class P>
 __global__ __launch_bounds__( 64 ) void k_galerkin( Rows<P> A, const int *pn, const int *pcol, const P *pval, int *tn, int *tcol, P *tval, int room,
@@ -279,7 +280,8 @@ __global__ __launch_bounds__( 64 ) void k_galerkin( Rows<P> A, const int *pn, co
     double bound = 0;
     for ( int k = lane; k < cnt; k += 64 ) bound += 2 * fabs( sw[ k ] * double( A.dia[ si[ k ] ] ) );
     for ( int o = 32; o; o >>= 1 ) bound += __shfl_xor( bound, o, 64 );
-    const int ex = bound > 0 && bound < 1e300 ? ilogb( bound ) + 1 : 0;
+    const int ex = bound > 0 && bound < 1e300 ? max( ilogb( bound ) + 1, -900 ) : 0;
+    double size = 0;
     const double scale = ldexp( 1.0, 60 - ex ), unit = ldexp( 1.0, ex - 60 );
     const int g = lane >> 3, sub = lane & 7;
     for ( int base = 0; base < cnt && nkeys <= SA_SMAX + 1; base += 8 ) {   // ( past any room the hash would fill up )
@@ -296,7 +298,9 @@ __global__ __launch_bounds__( 64 ) void k_galerkin( Rows<P> A, const int *pn, co
                 const int np = pn[ j ];
                 for ( int e = 0; e < np; ++e ) {
                     const int K = pcol[ I64( e ) * A.n + j ];
-                    const long long term = __double2ll_rn( wi * a * double( pval[ I64( e ) * A.n + j ] ) );
+                    const double t = wi * a * double( pval[ I64( e ) * A.n + j ] );
+                    const long long term = __double2ll_rn( t );
+                    size += fabs( t );
                     unsigned h = ( unsigned( K ) * 2654435761u ) >> 23;
                     for ( int probe = 0; probe < SA_HASH; ++probe, h = ( h + 1 ) & ( SA_HASH - 1 ) ) {
                         int prev = hk[ h ];
@@ -315,6 +319,7 @@ __global__ __launch_bounds__( 64 ) void k_galerkin( Rows<P> A, const int *pn, co
         }
         __syncthreads();
     }
+    size = wave_sum( size );
     const int m = min( nkeys, SA_SMAX + 1 );
     bool diag = false;
     for ( int id = lane; id < m; id += 64 ) {
@@ -336,7 +341,7 @@ __global__ __launch_bounds__( 64 ) void k_galerkin( Rows<P> A, const int *pn, co
         if ( ! has_diag ) { cdia[ I ] = 1; cdinv[ I ] = 1; }
         ccnt[ I ] = min( max( m - ( has_diag ? 1 : 0 ), 0 ), room );
         if ( over ) tn[ I ] = SA_TMAX;
-        if ( over || nkeys > room + 1 ) state[ S_BAD ] = 1;
+        if ( over || nkeys > room + 1 || ! ( size < 0x1p62 ) ) state[ S_BAD ] = 1;
     }
 }
 

@@ -596,8 +596,8 @@ def mg32_counts():
 
 
 def cycle_counts():
-    """the linear systems since the last reset of the kernel times, by the cycle they were tried with: `{ smoothed, kcycle }` ( both, for one
-    that the smoothed cycle handed over )"""
+    """the linear systems since the last reset of the kernel times, by the cycle: `{ smoothed, kcycle }` ( one that the smoothed cycle
+    missed counts in both, one whose smoothed hierarchy could not be built in the second )"""
     s, k = _LL(), _LL()
     _check( lib().sdot_amd_cycle_counts( ctypes.byref( s ), ctypes.byref( k ) ) )
     return dict( smoothed = int( s.value ), kcycle = int( k.value ) )
