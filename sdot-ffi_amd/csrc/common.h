@@ -138,6 +138,14 @@ struct Arena {
         return reinterpret_cast<T *>( b.ptr );
     }
 
+    /// gives back the device buffers whose names begin with `prefix` ( waits for the device: nothing may be queued that uses them later )
+    void drop( const std::string &prefix ) {
+        std::lock_guard<std::mutex> lk( mtx );
+        if ( fix_dev ) return;                           // ( a fixed region is carved anew by each call )
+        for ( auto it = bufs.lower_bound( prefix ); it != bufs.end() && it->first.compare( 0, prefix.size(), prefix ) == 0; it = bufs.erase( it ) )
+            if ( it->second.ptr ) (void) hipFree( it->second.ptr );
+    }
+
     size_t bytes_held() {
         std::lock_guard<std::mutex> lk( mtx );
         size_t s = 0;

@@ -1,7 +1,7 @@
 // WHAT A SOLVE TAKES FROM THE DEVICE, buffer by buffer, before it starts: the model the server admits requests by and the
 // Python side checks against the free memory ( the role of the reference's `src/sdot/CardMemory.py:47-190`,
 // `card_solve_bytes`, for this library's own buffers ). It follows the arena's takes of `solve_2d` ( solver.hip ), the cells
-// ( cells.hip, cells3.hip ), the trees ( tree_gpu.hip, tree3.hip ), the multigrid ( multigrid.hip ) and the step by the limits
+// ( cells.hip, cells3.hip ), the trees ( tree_gpu.hip, tree3.hip ), the multigrids ( smoothed.hip, multigrid.hip ) and the step by the limits
 // ( limits.hip ), with the sizes they ask for on a generic cloud; a diagram whose rows overflow their first room takes more.
 
 #include "../../include/sdot_amd.h"
@@ -52,24 +52,26 @@ void solve_parts( I64 n, int dim, int density_kind, const double *o, int precisi
     parts[ 6 ] = ( d3 ? 24 : 16 ) * m + 16 * m;
     // the linear solver: the multigrid's levels, their vectors, the outer iteration's; Jacobi-PCG's when asked for
     if ( o && int( o[ O_LIN ] ) == 1 ) {
-        // the FP32 preconditioner's copies of the rows and their diagonal ( `mg_float` ), then the smoothed hierarchy in the cycle's
-        // float; or, where the options set the K-cycle's own, its coarse levels in `s`-byte values and vectors. ( A system redone with
-        // the FP64 cycle, or one the smoothed hierarchy has no room for, takes that cycle's buffers beside these. )
-        const bool f32 = o[ O_MG_FLOAT ] != 0;
-        const double s = f32 ? 4 : 8;
-        double lin = f32 ? 4 * cap + 4 * m : 0;
-        if ( smoothed_asked( o ) && n > SA_MIN_ROWS )
-            lin += smoothed_bytes( n, d3, s );
-        else {
-            const int pack = o[ O_MG_SHIFT ] > 0 ? 1 << int( o[ O_MG_SHIFT ] ) : 8;
-            const int kc = o[ O_MG_KCYCLE ] >= 0 ? int( o[ O_MG_KCYCLE ] ) : 2;
+        // the K-cycle: its coarse levels in `s`-byte values and vectors, the outer iteration's four, the finest level's work vector ( and the
+        // cycle's copies of `r` and `z` ), the partial sums and the dense inverse
+        const int pack = o[ O_MG_SHIFT ] > 0 ? 1 << int( o[ O_MG_SHIFT ] ) : 8;
+        const int kc = o[ O_MG_KCYCLE ] >= 0 ? int( o[ O_MG_KCYCLE ] ) : 2;
+        auto kcycle = [&]( double s ) {
+            double b = 4 * 8 * m + s * m + ( s < 8 ? 2 * s * m : 0 ) + 24 * 5 * 512 * 8 + 64 * 64 * 8 + 4 * 512 * 8;
             double nl = m;
-            lin += 4 * 8 * m + s * m + ( f32 ? 8 * m : 0 ) + 24 * 5 * 512 * 8 + 64 * 64 * 8 + 4 * 512 * 8;
             for ( int l = 1; nl > 64 && l < 24; ++l ) {
                 nl = std::ceil( nl / pack );
-                lin += nl * ( 4 + MG_STRIDE_B * ( 4 + s ) + s ) + 3 * s * nl + ( l <= kc ? 5 * s * nl : 0 );
+                b += nl * ( 4 + MG_STRIDE_B * ( 4 + s ) + s ) + 3 * s * nl + ( l <= kc ? 5 * s * nl : 0 );
             }
-        }
+            return b;
+        };
+        // the FP32 preconditioner's copies of the rows and their diagonal ( `mg_float` ), then the FP32 K-cycle beside the FP64 one it falls
+        // back to; or the smoothed hierarchy, or those it hands a system over to ( its own buffers are given back first )
+        const bool f32 = o[ O_MG_FLOAT ] != 0;
+        double lin = kcycle( 8 ) + ( f32 ? kcycle( 4 ) : 0 );
+        if ( smoothed_asked( o ) && n > SA_MIN_ROWS ) lin = std::max( lin, smoothed_bytes( n, d3, f32 ? 4 : 8 ) );
+        else lin += 3 * 8 * m;                           // ( Jacobi-PCG's vectors beside it, for a system it misses )
+        if ( f32 ) lin += 4 * cap + 4 * m;
         parts[ 7 ] = lin;
     } else
         parts[ 7 ] = 3 * 8 * m;

@@ -1001,13 +1001,14 @@ int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, i
     if ( o.fp32 ) {
         // THE FP32 PRECONDITIONER: the hierarchy, its smoothing and its coarse solves in FP32 ( from an FP32 copy of the rows ),
         // the flexible CG, its SpMV and its vectors in FP64; the FP64 preconditioner when that solve does not converge
-        valf = A.get<float>( "mgm.valf", size_t( L.cap ) );
-        diaf = A.get<float>( "mgm.diaf", size_t( n ) );
+        valf = A.get<float>( "mgf.val", size_t( L.cap ) );
+        diaf = A.get<float>( "mgf.dia", size_t( n ) );
         k_to_float_rows<<<blocks_for( n, 256 ), 256, 0, st>>>( n, L.row_off, L.row_cnt, L.step, L.val, L.dia, valf, diaf );
         check_launch( "k_to_float_rows" );
     }
+    const bool smoothed = o.smoothed && n > SA_MIN_ROWS;
     bool missed = false;                                 // ( the smoothed cycle had its hierarchy and did not reach the tolerance )
-    if ( o.smoothed && n > SA_MIN_ROWS ) {
+    if ( smoothed ) {
         const FcgResult f = smoothed_solve( L, valf, diaf, b, d, tol, maxit, o, st, nb_levels, cs.last_its );
         if ( ! f.bad ) {
             ++timing().smoothed_systems;
@@ -1018,7 +1019,14 @@ int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, i
     }
     if ( ! done ) {
         // THE K-CYCLE: asked for, or a system the smoothed one has no room for or misses; it has iterations of its own. In FP32 first,
-        // unless the smoothed cycle has missed the system in FP32 already
+        // unless the smoothed cycle has missed the system in FP32 already. Two cycles' buffers are never held at once, so that a handed over
+        // system takes no more than the solve was admitted with ( memory.hip ); it costs their allocation, and is rare
+        struct Dropped {
+            Arena &A;
+            bool also;
+            ~Dropped() { if ( also ) { A.drop( "mg." ); A.drop( "mgm." ); } }
+        } dropped{ A, smoothed };
+        if ( smoothed ) { A.drop( "saf." ); A.drop( "sad." ); }
         int left = maxit;
         ++timing().kcycle_systems;
         if ( o.fp32 && ! missed ) {
@@ -1035,7 +1043,7 @@ int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, i
             take( f, false );
         }
     }
-    double *g = A.get<double>( "mg.g", 1 );
+    double *g = A.get<double>( "mgf.g", 1 );
     k_read_gauge<<<1, 64, 0, st>>>( d, gauge, g );
     k_shift_gauge<<<blocks_for( n, 256 ), 256, 0, st>>>( n, d, g, gauge );
     k_zero_gauge<<<1, 64, 0, st>>>( d, gauge );

@@ -119,3 +119,21 @@ def test_rows_past_the_whole_numbers_room_build_no_hierarchy( native, fp32 ):
     before = native.cycle_counts()
     native.linear_solves_2d( row, col, val, 1e-3 * dia, b, tol = 1e-8, method = "mg", smoothed = True, fp32 = fp32 )
     assert _cycles_since( native, before ) == ( 0, 1 )
+
+
+@pytest.mark.parametrize( "tuning", [ dict(), dict( mg_precision = "double" ), dict( mg_kcycle = 2 ) ] )
+def test_handed_over_systems_stay_within_the_byte_model( native, tuning ):
+    # a linear tolerance below rounding: every system goes through the smoothed cycle ( or the K-cycle that the options ask for, in FP32 ), the
+    # FP64 K-cycle and Jacobi-PCG
+    import sdot
+    from sdot import memory
+    rng = np.random.default_rng( 5 )
+    dens = sdot.UniformBox( [ 0, 0 ], [ 1, 1 ] )
+    it = sdot.Iterative( tol = 1e-9, on_failure = "ignore", tuning = sdot.Tuning( linear_tol = 1e-18, **tuning ) )
+    print( f"case handed over { tuning }", flush = True )
+    native.release()
+    before = native.cycle_counts()
+    sol = sdot.OtProblem( sdot.SumOfDiracs( rng.uniform( 0, 1, ( 9_000, 2 ) ) ), dens ).solve( it )
+    smoothed, kcycle = _cycles_since( native, before )
+    assert kcycle >= sol.stats[ "nb_iter" ] >= 3 and smoothed == ( 0 if "mg_kcycle" in tuning else kcycle )
+    assert native.device_bytes() <= sum( memory.solve_bytes( 9_000, 2, dens, it ).values() )
