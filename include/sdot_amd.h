@@ -395,7 +395,8 @@ int sdot_amd_build_tree_2d( void *stream, long long n, const double *positions, 
 /* WHETHER TWO ROWS OF A CLOUD MAY BE EQUAL: `*found` = 1 when two 64-bit prints of the rows' bits ( `-0.0` as `0.0` ) are equal, 0 when the
  * cloud surely has no exact duplicate ( the first step of the search of `src/sdot/SdotPlanNd.py:124-155` ). Returns at once; the
  * answer is there when the stream has run.
- *   positions DEVICE [ n ][ dim ], table DEVICE [ slots ] ( scratch; a power of two, at least 2 n ), found DEVICE [ 1 ] */
+ *   positions DEVICE [ n ][ dim ], table DEVICE [ slots ] ( scratch; a power of two, at least 2 n; null: the library's own, in buffers that a
+ *   solve takes anyway ), found DEVICE [ 1 ] */
 int sdot_amd_equal_prints( void *stream, long long n, int dim, const double *positions, unsigned long long *table, long long slots,
                            int *found );
 

@@ -830,7 +830,13 @@ int sdot_amd_build_tree_2d( void *stream, long long n, const double *positions, 
 
 int sdot_amd_equal_prints( void *stream, long long n, int dim, const double *positions, unsigned long long *table, long long slots, int *found ) {
     return guarded( [&] {
-        SDOT_CHECK( n >= 1 && dim >= 1 && positions && table && found, "equal_prints: n >= 1, dim >= 1 and the arrays are required" );
+        SDOT_CHECK( n >= 1 && dim >= 1 && positions && found, "equal_prints: n >= 1, dim >= 1 and the arrays are required" );
+        if ( ! table ) {
+            // the rows' room of the solve that follows: nothing of its own is held ( `solve_2d`, `solve_3d`: slot 0's values )
+            for ( slots = 2; slots < 2 * n; ) slots *= 2;
+            const I64 rows = dim == 3 ? ( n + 63 ) / 64 * 64 * 44 : 12 * n + 4096;
+            table = arena().get<unsigned long long>( "slot0.val", size_t( std::max<I64>( slots, rows ) ) );
+        }
         SDOT_CHECK( slots >= 2 * n && ( slots & ( slots - 1 ) ) == 0, "equal_prints: the table's slots are a power of two, at least 2 n" );
         hipStream_t st = hipStream_t( stream );
         k_clear_prints<<<blocks_for( slots, 256 ), 256, 0, st>>>( slots, table, found );

@@ -502,12 +502,8 @@ def equal_prints( positions ):
     T = torch()
     pos = on_device( positions )
     pos = pos.reshape( pos.shape[ 0 ], -1 )
-    n, slots = pos.shape[ 0 ], 2
-    while slots < 2 * n:
-        slots *= 2
-    table = T.empty( slots, dtype = T.int64, device = device() )
     found = T.empty( 1, dtype = T.int32, device = device() )
-    _check( lib().sdot_amd_equal_prints( _stream(), n, pos.shape[ 1 ], _ptr( pos ), _ptr( table ), slots, _ptr( found ) ) )
+    _check( lib().sdot_amd_equal_prints( _stream(), pos.shape[ 0 ], pos.shape[ 1 ], _ptr( pos ), None, 0, _ptr( found ) ) )
     return bool( found.item() )
 
 

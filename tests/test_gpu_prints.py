@@ -21,3 +21,22 @@ def test_duplicates_are_the_hosts( native, n, d ):
         dup_h, rep_h = exact_duplicates( P )
         assert np.array_equal( dup, dup_h ) and np.array_equal( rep, rep_h )
     assert native.equal_prints( torch.as_tensor( np.ones( ( 2, d ) ) ).cuda() ) and not native.equal_prints( torch.as_tensor( pos ).cuda() )
+
+
+@pytest.mark.parametrize( "d", [ 2, 3 ] )
+def test_the_search_holds_no_memory_of_its_own( native, d ):
+    import sdot
+    import torch
+    from sdot import memory
+    from sdot.SdotPlanNd import exact_duplicates
+    pos = torch.as_tensor( np.random.default_rng( d ).uniform( 0, 1, ( 300_001, d ) ) ).cuda()
+    native.equal_prints( pos[ :2 ] )
+    native.release()
+    torch.cuda.empty_cache()
+    before = torch.cuda.memory_reserved()
+    exact_duplicates( pos )
+    assert torch.cuda.memory_reserved() <= before + ( 2 << 20 )   # ( the answer's four bytes: torch's smallest segment )
+    # what it took of the library's is the solve's: the whole stays within the solve's model
+    dens, it = sdot.UniformBox( [ 0 ] * d, [ 1 ] * d ), sdot.Iterative( tol = 1e-9 )
+    sdot.OtProblem( sdot.SumOfDiracs( pos ), dens ).solve( it )
+    assert native.device_bytes() <= sum( memory.solve_bytes( 300_001, d, dens, it ).values() )
