@@ -880,7 +880,7 @@ __device__ void finish_cell( const Params &P, int k, const S &c, int nb, bool ac
 __device__ __forceinline__ void flush_events( const Params &P, const Ev &ev ) {
     const unsigned long long a = wave_sum64( ev.side ), b = wave_sum64( ev.prune ), c = wave_sum64( ev.newv );
     const unsigned long long d = wave_sum64( ev.visits ), e = wave_sum64( ev.cuts );
-    if ( ( threadIdx.x & 63 ) == 0 && d ) {
+    if ( ( threadIdx.x & 63 ) == 0 && ( a | d ) ) {      // ( a walk that starts in the only leaf visits no node )
         unsigned long long *to = P.shards + 8 * ( blockIdx.x & ( EV_SHARDS - 1 ) );
         atomicAdd( &to[ 0 ], a );
         atomicAdd( &to[ 1 ], b );

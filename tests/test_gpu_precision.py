@@ -137,3 +137,18 @@ def test_fp32_topology_repairs_at_1m_on_the_bench_image( native ):
     say( f"  fp32 repairs: { counts }" )
     assert counts[ "dropped" ] == 0
     assert float( ( m32 - m64 ).abs().max() ) <= 1e-6 / n
+
+
+@pytest.mark.parametrize( "n", [ 3, 10, 11 ] )
+def test_the_float_walks_steps_are_counted_whatever_the_tree( native, n ):
+    # a tree of one leaf ( 10 seeds ) and of two: the float walk tests as many seeds as the FP64 one over the same diagrams
+    import sdot
+    pos = np.random.default_rng( n ).uniform( 0, 1, ( n, 2 ) )
+    counts = []
+    native.set_timing( True )
+    for precision in ( "fp64", "fp32" ):
+        native.kernel_times( reset = True )
+        sol = sdot.OtProblem( sdot.SumOfDiracs( pos ), sdot.UniformBox( [ 0, 0 ], [ 1, 1 ] ) ).solve( sdot.Iterative( tol = 1e-8, precision = precision ) )
+        counts.append( ( sol.stats[ "nb_diag" ], native.kernel_times( reset = True )[ 2 ][ "cuts" ] ) )
+    native.set_timing( False )
+    assert counts[ 0 ] == counts[ 1 ]
