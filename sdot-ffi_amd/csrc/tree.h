@@ -31,7 +31,7 @@ struct alignas( 32 ) NodeF {
 };
 static_assert( sizeof( NodeF ) == 32, "one float node, one 32-byte record" );
 
-/// the tree on the device, plus what its host build keeps
+/// the tree on the device
 struct DevTree {
     I64  n = 0, nb_nodes = 0;
     int  depth = 0, leaf = 10;
@@ -50,18 +50,13 @@ struct DevTree {
     double  *stat = nullptr;      ///< [ 11 ][ N ] centred moments per node
     double  *fit = nullptr;       ///< [ 2 ][ N ]
     unsigned long long *rkeys = nullptr;  ///< [ 3 ][ N ] ordered keys: min r, max r, max |a.y|
-    // host copies of the level structure
-    std::vector<int> h_lvl_nodes;
 };
 
 /// `AaBsp.py:264`
 int max_depth_for( I64 n, I64 leaf );
 
-/// builds the tree of `pos_host[ n ][ 2 ]` ( user order ) on the host and uploads it; the arena
-/// buffers are named with `tag` so two trees can live side by side
-void build_tree( DevTree &t, I64 n, const double *pos_host, int leaf, hipStream_t st, const std::string &tag );
-
-/// builds the same tree on the device from `pos_dev[ n ][ 2 ]` ( device, user order ): no host round trip
+/// builds the tree on the device from `pos_dev[ n ][ 2 ]` ( device, user order ): no host round trip; the arena buffers are named
+/// with `tag` so that two trees can live side by side
 void build_tree_device( DevTree &t, I64 n, const double *pos_dev, int leaf, hipStream_t st, const std::string &tag );
 
 /// rank-ordered weights are in `t.seeds[ k ].z`: the majorants of every node and the walk records. `reference`: the reference's rule

@@ -1,10 +1,10 @@
-// The BSP tree: host build ( median cut on the longest axis, level by level ) and the device-side
-// refresh of the affine weight majorants.
+// The BSP tree's depth, its weights, and the device-side refresh of the affine weight majorants ( the tree itself: tree_gpu.hip ).
 //
 // Majorant rule ( reference `bsp_build_level.h:84-209` ): least-squares slope `a` of `w` over the
 // node's seeds, kept when the residual spread `max r - min r` ( `r = w - a . y` ) is below
 // `0.85 sqrt( 1 - 2 / ( m - 1 ) )` times the weight spread and the slope is well behaved over the
-// node's extent; then `b = max( w - a . y )` plus `1e-6 ( |b| + spread + max |a . y| )`. A majorant
+// node's extent; then `b = max( w - a . y )` plus `1e-6 ( |b| + spread + max |a . y| )` ( the walks nobody
+// counts keep more slopes under a smaller slack: `refresh_majorants` ). A majorant
 // only prunes: any `( a, b )` that majorizes gives the same cells, so the device computes it its own
 // way -- centred moments merged up the tree ( Chan's parallel formula ), then one pass over the seeds
 // that walks root -> leaf and takes the residual extremes of every node on the path with a
@@ -14,8 +14,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <numeric>
-#include <thread>
 
 namespace sdot_amd {
 
@@ -23,168 +21,6 @@ int max_depth_for( I64 n, I64 leaf ) {
     if ( leaf < 1 ) leaf = 1;
     if ( n <= leaf ) return 1;
     return int( std::ceil( std::log2( double( n ) / double( leaf ) ) ) ) + 1;
-}
-
-// ---- host build -----------------------------------------------------------------------------------
-
-namespace {
-
-struct HostBuild {
-    I64 n;
-    int depth;
-    std::vector<double> x, y;     ///< permuted positions
-    std::vector<int> ord;         ///< permuted user indices
-};
-
-void run_parallel( int nt, const std::function<void( int )> &f ) {
-    if ( nt <= 1 ) { f( 0 ); return; }
-    std::vector<std::thread> ts;
-    for ( int i = 0; i < nt; ++i ) ts.emplace_back( f, i );
-    for ( auto &t : ts ) t.join();
-}
-
-} // namespace
-
-void build_tree( DevTree &t, I64 n, const double *pos, int leaf, hipStream_t st, const std::string &tag ) {
-    SDOT_CHECK( n >= 1, "a tree needs at least one seed" );
-    SDOT_CHECK( n < ( I64( 1 ) << 31 ) - 8, "more seeds than 32-bit ranks can index" );
-    const int depth = max_depth_for( n, leaf );
-    const I64 N = ( I64( 1 ) << depth ) - 1;
-    t.n = n;
-    t.depth = depth;
-    t.leaf = leaf;
-    t.nb_nodes = N;
-
-    std::vector<double> X( ( size_t( n ) ) ), Y( ( size_t( n ) ) );
-    std::vector<int> ord( ( size_t( n ) ) );
-    for ( I64 i = 0; i < n; ++i ) { X[ size_t( i ) ] = pos[ 2 * i ]; Y[ size_t( i ) ] = pos[ 2 * i + 1 ]; ord[ size_t( i ) ] = int( i ); }
-
-    // heap numbering while building, preorder at the end
-    std::vector<int> hbeg( ( size_t( N ) ) ), hend( ( size_t( N ) ) );
-    std::vector<double> hbox( size_t( N ) * 4, 0.0 );
-    std::vector<int> beg{ 0 }, end{ int( n ) };
-    const int hw = int( std::max( 1u, std::min( 16u, std::thread::hardware_concurrency() ) ) );
-    std::vector<int> idx( ( size_t( n ) ) );
-    for ( int level = 0; level < depth; ++level ) {
-        const I64 first = ( I64( 1 ) << level ) - 1;
-        const int nb = int( beg.size() );
-        std::vector<int> mid( end );
-        // one node: its box, the longest axis, the median of its slice
-        auto do_node = [&]( int j ) {
-            const int b = beg[ size_t( j ) ], e = end[ size_t( j ) ];
-            const I64 node = first + j;
-            hbeg[ size_t( node ) ] = b;
-            hend[ size_t( node ) ] = e;
-            if ( e <= b ) return;
-            double lo[ 2 ] = { X[ size_t( b ) ], Y[ size_t( b ) ] }, hi[ 2 ] = { lo[ 0 ], lo[ 1 ] };
-            for ( int k = b + 1; k < e; ++k ) {
-                lo[ 0 ] = std::min( lo[ 0 ], X[ size_t( k ) ] ); hi[ 0 ] = std::max( hi[ 0 ], X[ size_t( k ) ] );
-                lo[ 1 ] = std::min( lo[ 1 ], Y[ size_t( k ) ] ); hi[ 1 ] = std::max( hi[ 1 ], Y[ size_t( k ) ] );
-            }
-            double *bx = &hbox[ size_t( node ) * 4 ];
-            bx[ 0 ] = lo[ 0 ]; bx[ 1 ] = lo[ 1 ]; bx[ 2 ] = hi[ 0 ]; bx[ 3 ] = hi[ 1 ];
-            const int ax = ( hi[ 1 ] - lo[ 1 ] > hi[ 0 ] - lo[ 0 ] ) ? 1 : 0;
-            if ( e - b > leaf && hi[ ax ] > lo[ ax ] ) {
-                const int m = b + ( e - b ) / 2;
-                const std::vector<double> &K = ax ? Y : X;
-                for ( int k = b; k < e; ++k ) idx[ size_t( k ) ] = k;
-                std::nth_element( idx.begin() + b, idx.begin() + m, idx.begin() + e, [&]( int u, int v ) {
-                    return K[ size_t( u ) ] < K[ size_t( v ) ] || ( K[ size_t( u ) ] == K[ size_t( v ) ] && u < v );
-                } );
-                std::vector<double> tx( size_t( e - b ) ), ty( size_t( e - b ) );
-                std::vector<int> to( size_t( e - b ) );
-                for ( int k = b; k < e; ++k ) {
-                    const int s = idx[ size_t( k ) ];
-                    tx[ size_t( k - b ) ] = X[ size_t( s ) ]; ty[ size_t( k - b ) ] = Y[ size_t( s ) ]; to[ size_t( k - b ) ] = ord[ size_t( s ) ];
-                }
-                std::copy( tx.begin(), tx.end(), X.begin() + b );
-                std::copy( ty.begin(), ty.end(), Y.begin() + b );
-                std::copy( to.begin(), to.end(), ord.begin() + b );
-                mid[ size_t( j ) ] = m;
-            }
-        };
-        if ( nb >= 4 * hw ) {
-            run_parallel( hw, [&]( int th ) { for ( int j = th; j < nb; j += hw ) do_node( j ); } );
-        } else {
-            for ( int j = 0; j < nb; ++j ) do_node( j );
-        }
-        if ( level + 1 < depth ) {
-            std::vector<int> nb_( size_t( 2 * nb ) ), ne_( size_t( 2 * nb ) );
-            for ( int j = 0; j < nb; ++j ) {
-                nb_[ size_t( 2 * j ) ] = beg[ size_t( j ) ]; ne_[ size_t( 2 * j ) ] = mid[ size_t( j ) ];
-                nb_[ size_t( 2 * j + 1 ) ] = mid[ size_t( j ) ]; ne_[ size_t( 2 * j + 1 ) ] = end[ size_t( j ) ];
-            }
-            beg.swap( nb_ );
-            end.swap( ne_ );
-        }
-    }
-
-    // the seeds of each leaf in ascending user index ( a canonical order: the cut order inside a leaf
-    // is then the same whatever selection built the tree )
-    {
-        const I64 first = ( I64( 1 ) << ( depth - 1 ) ) - 1;
-        run_parallel( hw, [&]( int th ) {
-            std::vector<std::pair<int, int>> tmp;
-            std::vector<double> tx, ty;
-            for ( I64 h = first + th; h < N; h += hw ) {
-                const int b = hbeg[ size_t( h ) ], e = hend[ size_t( h ) ];
-                if ( e - b < 2 ) continue;
-                tmp.clear();
-                for ( int k = b; k < e; ++k ) tmp.emplace_back( ord[ size_t( k ) ], k );
-                std::sort( tmp.begin(), tmp.end() );
-                tx.resize( tmp.size() ); ty.resize( tmp.size() );
-                for ( size_t q = 0; q < tmp.size(); ++q ) { tx[ q ] = X[ size_t( tmp[ q ].second ) ]; ty[ q ] = Y[ size_t( tmp[ q ].second ) ]; }
-                for ( size_t q = 0; q < tmp.size(); ++q ) { X[ size_t( b ) + q ] = tx[ q ]; Y[ size_t( b ) + q ] = ty[ q ]; ord[ size_t( b ) + q ] = tmp[ q ].first; }
-            }
-        } );
-    }
-
-    // heap -> preorder ( reference `AaBsp.py:514-532` )
-    std::vector<int> pre( ( size_t( N ) ), 0 );
-    for ( int level = 0; level + 1 < depth; ++level ) {
-        const int h = depth - level;
-        for ( I64 i = ( I64( 1 ) << level ) - 1; i < ( I64( 1 ) << ( level + 1 ) ) - 1; ++i ) {
-            pre[ size_t( 2 * i + 1 ) ] = pre[ size_t( i ) ] + 1;
-            pre[ size_t( 2 * i + 2 ) ] = pre[ size_t( i ) ] + int( I64( 1 ) << ( h - 1 ) );
-        }
-    }
-    std::vector<int> pbeg( ( size_t( N ) ) ), pend( ( size_t( N ) ) );
-    std::vector<double> pbox( size_t( N ) * 4 );
-    for ( I64 h = 0; h < N; ++h ) {
-        const int p = pre[ size_t( h ) ];
-        pbeg[ size_t( p ) ] = hbeg[ size_t( h ) ];
-        pend[ size_t( p ) ] = hend[ size_t( h ) ];
-        for ( int c = 0; c < 4; ++c ) pbox[ size_t( p ) * 4 + c ] = hbox[ size_t( h ) * 4 + c ];
-    }
-    t.h_lvl_nodes = pre;                                  // heap rank `h` ( level by level ) -> preorder node
-
-    std::vector<int> rank_of( ( size_t( n ) ) );
-    for ( I64 k = 0; k < n; ++k ) rank_of[ size_t( ord[ size_t( k ) ] ) ] = int( k );
-    std::vector<double4> seeds( ( size_t( n ) ) );
-    for ( I64 k = 0; k < n; ++k ) seeds[ size_t( k ) ] = make_double4( X[ size_t( k ) ], Y[ size_t( k ) ], 0.0, 0.0 );
-
-    Arena &A = arena();
-    t.nodes = A.get<NodeRec>( tag + ".nodes", size_t( N ) );
-    t.nodes32 = A.get<NodeF>( tag + ".nodes32", size_t( N ) );
-    t.node_box = A.get<double>( tag + ".node_box", size_t( N ) * 4 );
-    t.node_beg = A.get<int>( tag + ".node_beg", size_t( N ) );
-    t.node_end = A.get<int>( tag + ".node_end", size_t( N ) );
-    t.lvl_nodes = A.get<int>( tag + ".lvl_nodes", size_t( N ) );
-    t.order = A.get<int>( tag + ".order", size_t( n ) );
-    t.rank_of = A.get<int>( tag + ".rank_of", size_t( n ) );
-    t.seeds = A.get<double4>( tag + ".seeds", size_t( n ) );
-    t.stat = A.get<double>( tag + ".stat", size_t( N ) * 11 );
-    t.fit = A.get<double>( tag + ".fit", size_t( N ) * 2 );
-    t.rkeys = A.get<unsigned long long>( tag + ".rkeys", size_t( N ) * 3 );
-    SDOT_HIP( hipMemcpyAsync( t.node_box, pbox.data(), sizeof( double ) * size_t( N ) * 4, hipMemcpyHostToDevice, st ) );
-    SDOT_HIP( hipMemcpyAsync( t.node_beg, pbeg.data(), sizeof( int ) * size_t( N ), hipMemcpyHostToDevice, st ) );
-    SDOT_HIP( hipMemcpyAsync( t.node_end, pend.data(), sizeof( int ) * size_t( N ), hipMemcpyHostToDevice, st ) );
-    SDOT_HIP( hipMemcpyAsync( t.lvl_nodes, pre.data(), sizeof( int ) * size_t( N ), hipMemcpyHostToDevice, st ) );
-    SDOT_HIP( hipMemcpyAsync( t.order, ord.data(), sizeof( int ) * size_t( n ), hipMemcpyHostToDevice, st ) );
-    SDOT_HIP( hipMemcpyAsync( t.rank_of, rank_of.data(), sizeof( int ) * size_t( n ), hipMemcpyHostToDevice, st ) );
-    SDOT_HIP( hipMemcpyAsync( t.seeds, seeds.data(), sizeof( double4 ) * size_t( n ), hipMemcpyHostToDevice, st ) );
-    // the host vectors die with this scope: the copies must be done before returning
-    SDOT_HIP( hipStreamSynchronize( st ) );
 }
 
 // ---- weights -------------------------------------------------------------------------------------

@@ -1,6 +1,5 @@
-// The BSP tree built on the device, no host round trip: the same tree as the host build ( median cut on
-// the longest axis, leaf <= `leaf`, perfect binary tree in preorder, each leaf's seeds in ascending
-// user index ).
+// The BSP tree built on the device, no host round trip: median cut on the longest axis, leaf <= `leaf`, perfect binary tree
+// in preorder, each leaf's seeds in ascending user index.
 //
 // How ( this build's own scheme; the reference's card builder is `gpu/Bsp2D.cuh:367` ):
 //   1. a stable LSD radix sort of the seeds along each axis, the axes in the same launches ( 64-bit order-preserving keys of the
@@ -509,7 +508,6 @@ void build_tree_device( DevTree &t, I64 n, const double *pos, int leaf, hipStrea
     t.fit = A.get<double>( tag + ".fit", size_t( N ) * 2 );
     t.rkeys = A.get<unsigned long long>( tag + ".rkeys", size_t( N ) * 3 );
     build_into<2>( SmallOut{ t.node_beg, t.node_end, t.lvl_nodes, t.order, t.rank_of, t.leaf_of, t.node_box, t.seeds }, n, pos, leaf, depth, st );
-    t.h_lvl_nodes.clear();
 }
 
 } // namespace sdot_amd
