@@ -29,7 +29,7 @@ void solve_parts( I64 n, int dim, int density_kind, const double *o, int precisi
     // build's sort keys, sorted lists, segments and flags
     // ( one workgroup builds a small cloud's tree in LDS: no build buffers )
     const double d = dim, lists = d3 ? 3 : 1;
-    const double build = n <= 8192 ? 0 : d * ( 16 + 8 ) * m + ( 8 + 1 + 4 * lists ) * m + 1024 * d * std::ceil( m / RS_TILE_B ) + 16 * N + 16 * d * N +
+    const double build = n <= SMALL_TREE ? 0 : d * ( 16 + 8 ) * m + ( 8 + 1 + 4 * lists ) * m + 1024 * d * std::ceil( m / RS_TILE_B ) + 16 * N + 16 * d * N +
                                          4 * lists * std::ceil( m / 1024 );
     if ( d3 ) parts[ 0 ] = 96 * N + 48 * N + 12 * N + 8 * m + 32 * m + ( 16 + 3 + 3 ) * 8 * N + build;
     else      parts[ 0 ] = 64 * N + 32 * N + 32 * N + 12 * N + 12 * m + 32 * m + ( 11 + 2 + 3 ) * 8 * N + build;

@@ -52,6 +52,9 @@ struct DevTree {
     unsigned long long *rkeys = nullptr;  ///< [ 3 ][ N ] ordered keys: min r, max r, max |a.y|
 };
 
+/// the seeds that one workgroup builds the tree of, at most ( `k_small_tree` )
+constexpr int SMALL_TREE = 4096;
+
 /// `AaBsp.py:264`
 int max_depth_for( I64 n, I64 leaf );
 

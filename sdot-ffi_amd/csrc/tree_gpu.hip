@@ -11,8 +11,10 @@
 //      level: the nodes, the flags, the scan in two, the partition, which also hands each position its child;
 //   3. the leaves' seeds sorted by user index, the preorder numbering and the rank tables.
 // Everything stays on the device; the host only issues launches ( their count is a function of `n` ) and waits for none of them.
-// A cloud of at most `SMALL_TREE` seeds is built by ONE workgroup with its lists in LDS ( `k_small_tree` ): its ~100 launches
-// took ~0.4 ms, whatever they did ( the line is what LDS holds: 64 KiB of keys, the lists and their partitions ).
+// A cloud of at most `SMALL_TREE` seeds is built by ONE workgroup with its lists in LDS ( `k_small_tree` ): the ~100 launches take ~0.25 ms
+// whatever they do. The line is where the two cross: the workgroup's sorting networks double at every power of two. Masses of a Voronoi
+// diagram, us a call by one workgroup / by launches: 2D 500 seeds 266 / 398, 2000 333 / 475, 4096 418 / 520; 3D 500 356 / 470, 2000 490 / 597,
+// 4096 663 / 704; with room for 8192 in it, 2D 5000 555 / 560, 8192 600 / 562; 3D 5000 895 / 761, 8192 1110 / 923.
 
 #include "tree.h"
 #include "tree3.h"
@@ -303,7 +305,8 @@ __global__ void k_to_preorder( I64 N, int depth, int box, const int *hbeg, const
 
 // ---- a small cloud's tree by one workgroup ----------------------------------------------------------------------------
 
-constexpr int SMALL_TREE = 8192, SMALL_T = 1024, SMALL_NODES = 1024;
+constexpr int SMALL_T = 1024, SMALL_NODES = 1024;
+constexpr int SMALL_PER = SMALL_TREE / SMALL_T;        ///< a thread's consecutive positions in a scan
 
 struct SmallOut {
     int *beg, *end, *lvl_nodes, *order, *rank_of, *leaf_of;
@@ -312,7 +315,7 @@ struct SmallOut {
 };
 
 /// THE SAME TREE in one launch: each axis sorted by a bitonic network over ( key, user index ), the lists and their partitions in LDS,
-/// the levels separated by barriers, each thread eight consecutive positions of a scan. It is bound by its barriers and LDS: 2k seeds 114
+/// the levels separated by barriers, each thread four consecutive positions of a scan. It is bound by its barriers and LDS: 2k seeds 114
 /// us, which made a call that measures 2k cells 0.79 -> 0.44 ms
 template<int D>
 __global__ __launch_bounds__( SMALL_T ) void k_small_tree( int n, const double *pos, int leaf, int depth, SmallOut out ) {
@@ -346,9 +349,9 @@ __global__ __launch_bounds__( SMALL_T ) void k_small_tree( int n, const double *
     u16 *alt = reinterpret_cast<u16 *>( keys );                       // [ D ][ SMALL_TREE ]
     unsigned char *flag = reinterpret_cast<unsigned char *>( alt + 3 * SMALL_TREE );
     u16 *cur = &lists[ 0 ][ 0 ];
-    const int p0 = 8 * tid;
-    int seg[ 8 ];
-    for ( int u = 0; u < 8; ++u ) seg[ u ] = 0;
+    const int p0 = SMALL_PER * tid;
+    int seg[ SMALL_PER ];
+    for ( int u = 0; u < SMALL_PER; ++u ) seg[ u ] = 0;
     for ( int L = 0; L < depth; ++L ) {
         const int count = 1 << L;
         if ( tid < count ) {
@@ -372,28 +375,28 @@ __global__ __launch_bounds__( SMALL_T ) void k_small_tree( int n, const double *
         }
         __syncthreads();
         if ( L + 1 == depth ) break;
-        for ( int u = 0; u < 8; ++u )
+        for ( int u = 0; u < SMALL_PER; ++u )
             if ( p0 + u < n ) flag[ cur[ naxis[ seg[ u ] ] * SMALL_TREE + p0 + u ] ] = p0 + u < nmid[ seg[ u ] ];
         __syncthreads();
         for ( int d = 0; d < D; ++d ) {
             const u16 *in = cur + d * SMALL_TREE;
             u16 *to = alt + d * SMALL_TREE;
             unsigned f = 0, c = 0, all;
-            for ( int u = 0; u < 8; ++u )
+            for ( int u = 0; u < SMALL_PER; ++u )
                 if ( p0 + u < n && flag[ in[ p0 + u ] ] ) { f |= 1u << u; ++c; }
             const unsigned before = block_exclusive<SMALL_T>( c, sh, all );
             // the prefix at each segment's start, from the thread that holds it
-            for ( int u = 0; u < 8; ++u )
+            for ( int u = 0; u < SMALL_PER; ++u )
                 if ( p0 + u < n && p0 + u == nbeg[ seg[ u ] ] ) npre[ seg[ u ] ] = u16( before + __popc( f & ( ( 1u << u ) - 1 ) ) );
             __syncthreads();
-            for ( int u = 0; u < 8; ++u ) {
+            for ( int u = 0; u < SMALL_PER; ++u ) {
                 if ( p0 + u >= n ) continue;
                 const int j = seg[ u ], lb = int( before ) + __popc( f & ( ( 1u << u ) - 1 ) ) - npre[ j ];
                 to[ f >> u & 1 ? nbeg[ j ] + lb : nmid[ j ] + ( p0 + u - nbeg[ j ] ) - lb ] = in[ p0 + u ];
             }
             __syncthreads();
         }
-        for ( int u = 0; u < 8; ++u )
+        for ( int u = 0; u < SMALL_PER; ++u )
             if ( p0 + u < n ) seg[ u ] = 2 * seg[ u ] + ( p0 + u >= nmid[ seg[ u ] ] );
         __syncthreads();
         if ( tid < count ) { pbeg[ tid ] = nbeg[ tid ]; pend[ tid ] = nend[ tid ]; pmid[ tid ] = nmid[ tid ]; }

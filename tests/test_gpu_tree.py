@@ -1,4 +1,4 @@
-"""The device's tree builds ( one workgroup's, for at most 8192 seeds; the launches' beyond ) against the oracle's tree."""
+"""The device's tree builds ( one workgroup's, for at most 4096 seeds; the launches' beyond ) against the oracle's tree."""
 import numpy as np
 import pytest
 
@@ -31,10 +31,10 @@ def _by_median( pos, leaf = 10 ):
     return order, np.array( beg ), np.array( end )
 
 
-# one seed, a leaf, two leaves, one seed past a power of two and past a scan's block, and both sides of the one workgroup's 8192;
+# one seed, a leaf, two leaves, one seed past a power of two and past a scan's block, and both sides of the one workgroup's 4096;
 # `grid`: coordinates with many ties ( where the oracle cuts by its own order among the tied ), `line`: an axis without any extent,
 # `same`: all seeds in one place ( no node is cut )
-@pytest.mark.parametrize( "n", [ 1, 2, 10, 11, 129, 1025, 8191, 8192, 8193, 70_000 ] )
+@pytest.mark.parametrize( "n", [ 1, 2, 10, 11, 129, 1025, 4095, 4096, 4097, 8191, 8192, 8193, 70_000 ] )
 @pytest.mark.parametrize( "kind", [ "uniform", "grid", "line", "same" ] )
 def test_the_tree_is_the_one_defined( native, oracle, n, kind ):
     rng = np.random.default_rng( n )
@@ -63,7 +63,7 @@ def test_other_leaves( native, oracle, leaf ):
 
 
 # the 3D tree through the counts of the walk over it ( the nodes tried and pruned, the cuts: another tree has others )
-@pytest.mark.parametrize( "n", [ 1, 10, 11, 1025, 8192, 8193 ] )
+@pytest.mark.parametrize( "n", [ 1, 10, 11, 1025, 4096, 4097, 8192, 8193 ] )
 def test_the_3d_walk_counts_the_oracles( native, oracle, n ):
     from sdot import UniformBox
     pos = np.random.default_rng( n ).uniform( 0, 1, ( n, 3 ) )
