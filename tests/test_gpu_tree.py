@@ -73,3 +73,18 @@ def test_the_3d_walk_counts_the_oracles( native, oracle, n ):
     assert np.allclose( m.cpu().numpy(), mo, rtol = 1e-10, atol = 1e-16 )
     for k in ( "side_tests", "node_visits", "cuts" ):     # ( the few cells of a second pass are walked, and counted, twice )
         assert abs( ev[ k ] - evo[ k ] ) <= 0.01 * evo[ k ], k
+
+
+# the 3D tree, seed for seed: each cell's facets come in the order of the cuts that made them, which is the order its walk met the leaves and
+# their seeds in ( another tree has another )
+@pytest.mark.parametrize( "n", [ 1, 10, 11, 1025, 4096, 4097, 8192, 8193, 30_000 ] )
+def test_the_3d_cells_are_cut_in_the_oracles_order( native, oracle, n ):
+    from sdot import UniformBox
+    rng = np.random.default_rng( n )
+    pos = rng.uniform( 0, 1, ( n, 3 ) ) * [ 1.0, 0.5, 1.0 ]
+    w = 0.1 * n ** ( -2 / 3 ) * rng.uniform( -1, 1, n )
+    print( f"case 3D tree n={ n }", flush = True )
+    m, ( fi, fj, _ ) = native.measures_3d( pos, w, [ 0, 0, 0, 1, 1, 1 ], UniformBox( [ 0 ] * 3, [ 1 ] * 3 ), facets = True )
+    mo, ( oi, oj, _ ) = oracle.measures_3d( pos, w, facets = True )
+    assert np.allclose( m.cpu().numpy(), mo, rtol = 1e-10, atol = 1e-16 )
+    assert np.array_equal( fi.cpu().numpy(), oi ) and np.array_equal( fj.cpu().numpy(), oj )
