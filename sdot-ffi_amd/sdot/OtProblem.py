@@ -16,7 +16,8 @@ _PRECISIONS = { "auto": "FP64", "fp64": "FP64", "fp32": "FP32", "mixed": "FP32" 
 class Tuning:
     """the bench settings ( reference `OtProblem.py:62-131` ): unstable, measured defaults. Taken for the reference's signature and read by
     nothing on this path: `amg_variant`, `mg_recycle`, `mg_rebuild`, `linear_host`, `mg_smoothed` ( the smoothed cycle always runs first,
-    unless `mg_pack`, `mg_nu`, `mg_kcycle` or `mg_stop` ask for the K-cycle ), `keep_start`, `accelerator`, `scratch_capacity`"""
+    unless `mg_pack`, `mg_nu`, `mg_kcycle` or `mg_stop` ask for the K-cycle ), `keep_start`, `accelerator`, `memory`,
+    `scratch_capacity`"""
 
     def __init__( self, step = "auto", linear_solver = "auto", amg_variant = "auto", linear_tol = None,
                   mg_pack = None, mg_recycle = None, mg_rebuild = None, mg_stop = None, mg_nu = None,
