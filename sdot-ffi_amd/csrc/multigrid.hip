@@ -1009,7 +1009,14 @@ int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, i
     const bool smoothed = o.smoothed && n > SA_MIN_ROWS;
     bool missed = false;                                 // ( the smoothed cycle had its hierarchy and did not reach the tolerance )
     if ( smoothed ) {
-        const FcgResult f = smoothed_solve( L, valf, diaf, b, d, tol, maxit, o, st, nb_levels, cs.last_its );
+        // coarse rows past their room, or with terms of both signs past their unit: the prolongations' rows are cut shorter, almost to the plain
+        // aggregates; the solve's next systems start from what fitted ( 300k 2D seeds in clusters, six systems: 38 ms at twice the
+        // threshold, 239 by the K-cycle )
+        FcgResult f;
+        for ( ;; cs.drop *= 2 ) {
+            f = smoothed_solve( L, valf, diaf, b, d, tol, maxit, o, st, nb_levels, cs.last_its, cs.drop );
+            if ( ! f.bad || cs.drop >= 4 ) break;
+        }
         if ( ! f.bad ) {
             ++timing().smoothed_systems;
             cs.last_its = f.its;

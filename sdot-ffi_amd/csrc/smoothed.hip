@@ -7,8 +7,8 @@
 // 63 iterations of ~70 launches with the K-cycle; 38 of ~21 with aggregates of 8; 27 with a first level of 4.
 //
 // What a level does:
-//   * `P = ( I - 2/3 D^-1 A ) P0`, a row's entries below 0.1 of its largest dropped ( 0.2 where rows are long, in 3D: there the
-//     coarse rows would grow past 100 entries ), the rest scaled to a unit sum ( `k_prolongator` ); the restriction is `P^T`,
+//   * `P = ( I - 2/3 D^-1 A ) P0`, a row's entries below 0.1 of its largest dropped ( 0.2 to 0.25 where rows are long, in 3D: there the
+//     coarse rows would outgrow their room ), the rest scaled to a unit sum ( `k_prolongator` ); the restriction is `P^T`,
 //     listed per coarse row in increasing order of the fine rows;
 //   * the Galerkin row `P^T A P` by one wave: its columns found by an LDS hash, each column's sum taken in whole numbers of
 //     a bound's 2^-60, so the result does not depend on the hash's races ( `k_galerkin` );
@@ -262,8 +262,8 @@ __device__ __forceinline__ int sorted_list( I64 I, I64 nf, const int *pn, const 
 /// lanes a fine row, added in LDS at their column's place in a hash of the columns met ( at most `SA_SMAX + 1` ). The sums are 64-bit
 /// whole numbers of `2^-60` of a guess of the row's terms' size ( `P`'s rows sum to 1, a Laplacian's row to twice its diagonal ), so that the
 /// atomics' order does not matter: the row is the same in every run, and each sum is within `2^-61` of the guess a term, where a sum in
-/// double rounds by `2^-53` of itself. Entries of both signs can pass the guess, so the terms' sizes are summed too, in double: below `2^62`
-/// units no column's sum wraps. `state[ S_BAD ]` beyond it, and when a list or a row outgrows its room.
+/// double rounds by `2^-53` of itself. Entries of both signs can pass the guess ( 1M 3D seeds in a thin slab ), so the terms' sizes are summed
+/// too, in double: below `2^62` units no column's sum wraps. `state[ S_BAD ]` beyond it, and when a list or a row outgrows its room.
 /// ( Terms staged in LDS and added up by their column's lane, every lane looking at every term: 1M rows 2.05 ms a hierarchy, 0.90 so )
 template<class P>
 __global__ __launch_bounds__( 64 ) void k_galerkin( Rows<P> A, const int *pn, const int *pcol, const P *pval, int *tn, int *tcol, P *tval, int room,
@@ -735,13 +735,14 @@ __global__ __launch_bounds__( TH ) void k_outer_init( I64 n, const double *b, co
     if ( threadIdx.x == 0 ) part[ blockIdx.x ] = s;
 }
 
+/// ( a system whose hierarchy could not be built stops here: the iterations queued behind are no-ops )
 __global__ __launch_bounds__( TH ) void k_outer_start( const double *part, int nblk, double *state, double tol ) {
     __shared__ double sh[ 4 ];
     const double bb = sum_partials( part, nblk, sh );
     if ( threadIdx.x == 0 ) {
         state[ S_NB ] = sqrt( bb );
         state[ S_ERR ] = 1;
-        state[ S_DONE ] = bb > 0 ? 0.0 : 1.0;
+        state[ S_DONE ] = bb > 0 && state[ S_BAD ] == 0 ? 0.0 : 1.0;
         state[ S_TOL ] = tol;
     }
 }
@@ -818,13 +819,15 @@ __global__ __launch_bounds__( TH ) void k_true_end( const double *part, int nblk
 
 /// the levels' sizes: `n[ 0 ]` the system's, `lb` the dense bottom, the last one at most `SA_DENSE`. The first aggregates hold 4
 /// ranks where that takes no more levels above the bottom than 8 ( 27 iterations against 38 on the 200k image Laplacian, the same
-/// launches ), 8 elsewhere and below ( a level more costs six launches an iteration )
+/// launches ), 8 elsewhere and below ( a level more costs six launches an iteration ). In 3D only where the level they make is the bottom itself:
+/// its rows have up to 120 entries, and the next level's then 280 and more, past any room ( from 12k seeds on every system was handed over
+/// to the K-cycle; three systems of 20k / 60k / 250k / 1M uniform seeds: 28.9 / 44.7 / 80 / 140 ms so, 4.0 / 5.4 / 11.6 / 37 ms with 8 )
 struct Sizes { int nl = 0, lb = 0; I64 n[ SA_LEVELS ]; int pack[ SA_LEVELS ]; };
-Sizes sizes_of( I64 n ) {
+Sizes sizes_of( I64 n, bool wide ) {
     auto above = [&]( I64 p ) { int k = 1; for ( I64 m = ( n + p - 1 ) / p; m > SA_BOTTOM; m = ( m + 7 ) / 8 ) ++k; return k; };
     Sizes s;
     s.n[ 0 ] = n;
-    s.pack[ 0 ] = above( 4 ) == above( 8 ) ? 4 : 8;
+    s.pack[ 0 ] = above( 4 ) == above( 8 ) && ! ( wide && above( 4 ) > 1 ) ? 4 : 8;
     s.lb = above( s.pack[ 0 ] );
     int l = 0;
     while ( l < s.lb || s.n[ l ] > SA_DENSE ) {
@@ -837,19 +840,23 @@ Sizes sizes_of( I64 n ) {
     return s;
 }
 
-/// the entries a row of level `l + 1` has room for. 2D: 17 to 22 a row on the first coarse level, 30 to 60 on the next; 3D: 50 to 80;
-/// below the bottom's level rows may be full
-int room_of( const Sizes &sz, int l, bool wide ) { return l >= sz.lb ? SA_DENSE_COLS : wide || l ? 192 : 96; }
+/// the entries a row of level `l + 1` has room for. 2D: 17 to 22 a row on the first coarse level, 30 to 60 on the next; 3D, at most: 100 ( 120
+/// with packs of 4 ), 150, 180 ( 1M seeds ); below the bottom's level rows may be full
+int room_of( const Sizes &sz, int l, bool wide ) { return l >= sz.lb ? SA_DENSE_COLS : wide && l ? SA_SMAX : wide || l ? 192 : 96; }
+
+/// the prolongation's rows drop what is below this part of their largest entry: more where rows are long, in 3D, and more still between the
+/// levels above the bottom there ( the 1M seeds' third level has rows of 180 entries so, of 260 at 0.2 )
+double theta_of( const Sizes &sz, int l, bool wide ) { return ! wide ? 0.1 : l && l < sz.lb ? 0.25 : 0.2; }
 
 template<class P>
 FcgResult solve_with( const Csr &L, const P *val, const P *dia, const double *b, double *d, double tol, int maxit, const MgOptions &o, hipStream_t st,
-                      int &nb_levels, int prev_its, const std::string &pfx ) {
+                      int &nb_levels, int prev_its, double drop, const std::string &pfx ) {
     constexpr bool same = std::is_same<P, double>::value;
     Arena &A = arena();
     const I64 n = L.n;
-    const Sizes sz = sizes_of( n );
     const bool wide = L.nnz > 10 * n;                    // ( 3D: 15.5 entries a row, 2D: 6 )
-    const double theta = wide ? 0.2 : 0.1, omega = 2.0 / 3, over = 1.2;
+    const Sizes sz = sizes_of( n, wide );
+    const double omega = 2.0 / 3, over = 1.2;
     // the sweeps' dampings: the Chebyshev nodes of [ 0.2, 2 ] ( 2 bounds the spectrum of `D^-1 A` )
     const double th = 1.1, de = 0.9, pi = 3.14159265358979323846;
     const double w0 = 1 / ( th + de * std::cos( pi / 4 ) ), w1 = 1 / ( th + de * std::cos( 3 * pi / 4 ) );
@@ -871,6 +878,7 @@ FcgResult solve_with( const Csr &L, const P *val, const P *dia, const double *b,
         const size_t nf = size_t( sz.n[ l ] ), nc = size_t( sz.n[ l + 1 ] );
         const std::string tag = pfx + "." + std::to_string( l );
         const int room = room_of( sz, l, wide );
+        const double theta = std::min( drop * theta_of( sz, l, wide ), 0.9 );
         F.pn = A.get<int>( tag + ".pn", nf );
         F.pcol = A.get<int>( tag + ".pcol", nf * SA_PMAX );
         F.pval = A.get<P>( tag + ".pval", nf * SA_PMAX );
@@ -1044,7 +1052,7 @@ FcgResult solve_with( const Csr &L, const P *val, const P *dia, const double *b,
 } // namespace
 
 double smoothed_bytes( I64 n, bool wide, double s ) {
-    const Sizes sz = sizes_of( n );
+    const Sizes sz = sizes_of( n, wide );
     const double m = double( n ), nb = double( sz.n[ sz.lb ] );
     double b = 8 * S_NB_STATE + 8.0 * P_NB * SA_BLOCKS + s * m + 8.0 * SA_DENSE * SA_DENSE + s * nb * nb + 4 * 8 * m;
     if ( sz.nl - 1 > sz.lb ) b += double( SA_BOTTOM ) * SA_DENSE_COLS * ( s + 8 );
@@ -1057,9 +1065,9 @@ double smoothed_bytes( I64 n, bool wide, double s ) {
 }
 
 FcgResult smoothed_solve( const Csr &L, const float *valf, const float *diaf, const double *b, double *d, double tol, int maxit, const MgOptions &o,
-                          hipStream_t st, int &nb_levels, int prev_its ) {
-    if ( valf ) return solve_with<float>( L, valf, diaf, b, d, tol, maxit, o, st, nb_levels, prev_its, "saf" );
-    return solve_with<double>( L, L.val, L.dia, b, d, tol, maxit, o, st, nb_levels, prev_its, "sad" );
+                          hipStream_t st, int &nb_levels, int prev_its, double drop ) {
+    if ( valf ) return solve_with<float>( L, valf, diaf, b, d, tol, maxit, o, st, nb_levels, prev_its, drop, "saf" );
+    return solve_with<double>( L, L.val, L.dia, b, d, tol, maxit, o, st, nb_levels, prev_its, drop, "sad" );
 }
 
 } // namespace sdot_amd

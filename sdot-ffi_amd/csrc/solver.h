@@ -39,6 +39,7 @@ struct Csr {
 struct CgStats {
     int nb_iter = 0;
     int last_its = 0;                   ///< the smoothed hierarchy's last system ( so many are queued before the next one's first look )
+    double drop = 1;                    ///< the smoothed hierarchy's prolongations: how much more is dropped, as the last systems' rows needed
     double worst = 0;
     // the last solve's end: its residual by the recurrence and the true one ( relative ), a breakdown ( `p . q <= 0` )
     double last_err = 0, last_true = 0;

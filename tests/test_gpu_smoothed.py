@@ -137,3 +137,41 @@ def test_handed_over_systems_stay_within_the_byte_model( native, tuning ):
     smoothed, kcycle = _cycles_since( native, before )
     assert kcycle >= sol.stats[ "nb_iter" ] >= 3 and smoothed == ( 0 if "mg_kcycle" in tuning else kcycle )
     assert native.device_bytes() <= sum( memory.solve_bytes( 9_000, 2, dens, it ).values() )
+
+
+@pytest.mark.parametrize( "d, n, kind", [ ( 3, 20_000, "uniform" ), ( 3, 60_000, "uniform" ), ( 3, 60_000, "clusters" ), ( 2, 300_000, "clusters" ) ] )
+def test_3d_and_clustered_clouds_keep_the_smoothed_cycle( native, d, n, kind ):
+    # their coarse rows grow past the room where the prolongations are those of a 2D uniform cloud
+    import sdot
+    rng = np.random.default_rng( n )
+    pos = rng.uniform( 0, 1, ( n, d ) )
+    if kind == "clusters":
+        centre, size, at = rng.uniform( 0.1, 0.9, ( 20, d ) ), 10 ** rng.uniform( -3, -1, 20 ), rng.integers( 0, 20, n )
+        pos = np.clip( centre[ at ] + size[ at, None ] * rng.normal( size = ( n, d ) ), 1e-9, 1 - 1e-9 )
+    print( f"case { kind } n={ n } d={ d }", flush = True )
+    before = native.cycle_counts()
+    sol = sdot.OtProblem( sdot.SumOfDiracs( pos ), sdot.UniformBox( [ 0 ] * d, [ 1 ] * d ) ).solve( sdot.Iterative( tol = 1e-3 / n, max_iter = 2, on_failure = "ignore" ) )
+    smoothed, kcycle = _cycles_since( native, before )
+    assert smoothed >= 2 and kcycle == 0 and sol.stats[ "lin_nb_iter" ] < 60 * smoothed
+
+
+def test_rows_that_no_prolongation_fits_go_to_the_other_solvers( native ):
+    # a random graph of ~40 neighbours a row: its coarse rows are full whatever is dropped
+    import torch
+    n = 9_000
+    rng = np.random.default_rng( 4 )
+    i, j = rng.integers( 0, n, ( 2, 20 * n ) )
+    keep = i != j
+    pair = np.unique( np.minimum( i, j )[ keep ] * n + np.maximum( i, j )[ keep ] )
+    i, j = np.concatenate( [ pair // n, pair % n ] ), np.concatenate( [ pair % n, pair // n ] )
+    at = np.lexsort( ( j, i ) )
+    i, j = i[ at ], j[ at ]
+    row = np.concatenate( [ [ 0 ], np.cumsum( np.bincount( i, minlength = n ) ) ] )
+    val, dia = np.ones( len( i ) ), np.bincount( i, minlength = n ).astype( float )
+    b = rng.normal( size = n )
+    b -= b.mean()
+    before = native.cycle_counts()
+    x, its = native.linear_solves_2d( row, j, val, dia, torch.as_tensor( b ), tol = 1e-9, method = "mg", smoothed = True, fp32 = True )
+    x = x[ 0 ].cpu().numpy()
+    assert its[ 0 ] > 0 and _cycles_since( native, before ) == ( 0, 1 )
+    assert np.linalg.norm( b - ( dia * x - np.bincount( i, weights = val * x[ j ], minlength = n ) ) ) <= 1e-8 * np.linalg.norm( b )
