@@ -1025,8 +1025,9 @@ int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, i
         }
     }
     if ( ! done ) {
-        // THE K-CYCLE: asked for, or a system the smoothed one has no room for or misses; it has iterations of its own. In FP32 first,
-        // unless the smoothed cycle has missed the system in FP32 already. Two cycles' buffers are never held at once, so that a handed over
+        // THE K-CYCLE: asked for, or a system the smoothed one has no room for or misses. In FP32 first, unless the smoothed cycle has missed
+        // the system in FP32 already; with what that left of the iterations ( it takes about twice as many: a system the smoothed cycle
+        // did not solve in all of them goes on to Jacobi-PCG, a breakdown or a drifted residual is worth the try ). Two cycles' buffers are never held at once, so that a handed over
         // system takes no more than the solve was admitted with ( memory.hip ); it costs their allocation, and is rare
         struct Dropped {
             Arena &A;
@@ -1034,7 +1035,7 @@ int mg_solve( const Csr &L, int gauge, const double *b, double *d, double tol, i
             ~Dropped() { if ( also ) { A.drop( "mg." ); A.drop( "mgm." ); } }
         } dropped{ A, smoothed };
         if ( smoothed ) { A.drop( "saf." ); A.drop( "sad." ); }
-        int left = maxit;
+        int left = std::max( maxit - total, 4 );
         ++timing().kcycle_systems;
         if ( o.fp32 && ! missed ) {
             MatT<float> Af;
