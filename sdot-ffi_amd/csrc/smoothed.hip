@@ -1052,7 +1052,8 @@ FcgResult solve_with( const Csr &L, const P *val, const P *dia, const double *b,
 } // namespace
 
 double smoothed_bytes( I64 n, bool wide, double s ) {
-    const Sizes sz = sizes_of( n, wide );
+    // ( a flat 3D cloud's rows are a 2D cloud's, and may grow within a solve: the smaller aggregates, the longer rows )
+    const Sizes sz = sizes_of( n, false );
     const double m = double( n ), nb = double( sz.n[ sz.lb ] );
     double b = 8 * S_NB_STATE + 8.0 * P_NB * SA_BLOCKS + s * m + 8.0 * SA_DENSE * SA_DENSE + s * nb * nb + 4 * 8 * m;
     if ( sz.nl - 1 > sz.lb ) b += double( SA_BOTTOM ) * SA_DENSE_COLS * ( s + 8 );

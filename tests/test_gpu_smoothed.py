@@ -175,3 +175,17 @@ def test_rows_that_no_prolongation_fits_go_to_the_other_solvers( native ):
     x = x[ 0 ].cpu().numpy()
     assert its[ 0 ] > 0 and _cycles_since( native, before ) == ( 0, 1 )
     assert np.linalg.norm( b - ( dia * x - np.bincount( i, weights = val * x[ j ], minlength = n ) ) ) <= 1e-8 * np.linalg.norm( b )
+
+
+def test_a_flat_3d_cloud_stays_within_the_byte_model( native ):
+    # seeds in one layer: rows of 2D length, whose hierarchy is a 2D cloud's
+    import sdot
+    from sdot import memory
+    rng = np.random.default_rng( 6 )
+    n = 20_000
+    pos = np.column_stack( [ rng.uniform( 0, 1, ( n, 2 ) ), 0.5 + 1e-7 * rng.uniform( -1, 1, n ) ] )
+    dens, it = sdot.UniformBox( [ 0 ] * 3, [ 1 ] * 3 ), sdot.Iterative( tol = 1e-7, max_iter = 3, on_failure = "ignore" )
+    native.release()
+    sol = sdot.OtProblem( sdot.SumOfDiracs( pos ), dens ).solve( it )
+    assert sol.stats[ "lin_nb_iter" ] > 0
+    assert native.device_bytes() <= sum( memory.solve_bytes( n, 3, dens, it ).values() )
